@@ -496,6 +496,81 @@ CRP_MATH_FN double crp_sin_cr(double x) {
 	return crp_cos_accurate_shift(x, 3);
 }
 
+/*
+ * cos(x) (shift 0) or sin(x) (shift 256), quick phase over a table of the whole turn: with
+ * x = k 2pi/1024 + r, |r| <= 2^-8.34, and j = k mod 512,
+ *   +-cos x = C cos r - S sin r,   S = sin(2pi j/1024) = tab[j], C = cos(2pi j/1024) = tab[j + 256],
+ * the sign from bit 9 of k.  No octant folding, no choice between sine and cosine: about a quarter of
+ * the instructions of crp_cos_quick_shift.  The one large product S r is formed and added exactly; the
+ * rest is summed in double from the small terms up.
+ *   reduction: x - k P1 is exact by FMA (both are multiples of 2^-61 and the difference is below 2^-8);
+ *     P2 and P3 leave |r_h + r_l - r| < 2^-83, and < 2^-105 |r| where |r| > 2^-29;
+ *   errors relative to C: C r (r/2 + r_l), at most 2^-17.7, takes a rounding in each of its factors and
+ *     one in the last addition, the rounding test one more: 4 x 2^-70.7; C_l (cos r - 1) is left out:
+ *     2^-70.7; the rest (C z^2/24 and z^3/720, S r z/6 and its series, the low parts) below 2^-72.  In all
+ *     below 2^-68.3, and |y| >= |C|/2 (equality at C = sin(2pi/1024)), so below 2^-67.3 of the result.
+ * Returned when every value within 1.25 x 2^-67 of it rounds the same way; |y| <= 2^-28 (only there can
+ * r be so small that its absolute error matters), |x| >= 2^30, infinities and NaN do not decide.  Returns
+ * 0 when it does not decide: 2e-4 of arguments.  `tab` is crp_turn_tab or a copy of it.
+ */
+#define CRP_TURN_ENTRIES 768
+CRP_MATH_FN int crp_cos_turn(double x, int shift, const double *tab, double *out) {
+	const double big = 6755399441055744.0; /* 1.5 * 2^52: the sum's low bits are the nearest integer */
+	const double kb = __builtin_fma(x, CRP_TURN_INV, big);
+	const uint32_t ki = (uint32_t)crp_as_u64(kb) - (uint32_t)shift;
+	const double k = kb - big;
+	const double r0 = __builtin_fma(-k, CRP_TURN_P1, x); /* exact */
+	const double t = k * CRP_TURN_P2, te = __builtin_fma(k, CRP_TURN_P2, -t);
+	const double rh = r0 - t;
+	const double rl = __builtin_fma(-k, CRP_TURN_P3, ((r0 - rh) - t) - te);
+	const double *const e = tab + 2 * (ki & 511u);
+	const double Sh = e[0], Sl = e[1], Ch = e[512], Cl = e[513];
+	const double z = rh * rh;
+	const double c4 = (z * z) * __builtin_fma(z, -1.0 / 720, 1.0 / 24); /* cos r - 1 + z/2 */
+	/* sin r - rh */
+	const double s3 = __builtin_fma(rh * z, __builtin_fma(z, __builtin_fma(z, -1.0 / 5040, 1.0 / 120), -1.0 / 6), rl);
+	const double hr = __builtin_fma(0.5, rh, rl); /* cos r - 1 = -rh hr + c4 */
+	const double q = Ch * rh;
+	const double p = -Sh * rh, pe = __builtin_fma(-Sh, rh, -p);
+	const crp_dd s = crp_two_sum(Ch, p);
+	double lo = __builtin_fma(-Sl, rh, pe + Cl);
+	lo = __builtin_fma(Ch, c4, lo);
+	lo = __builtin_fma(-Sh, s3, lo);
+	lo = s.lo + lo;
+	lo = __builtin_fma(-q, hr, lo);
+	const double as = __builtin_fabs(s.hi);
+	const double y = s.hi + __builtin_fma(as, 1.25 * 0x1p-67, lo);
+	const double y2 = s.hi + __builtin_fma(as, -1.25 * 0x1p-67, lo);
+	if (!(y == y2 && as > 0x1p-28 && __builtin_fabs(x) < 0x1p30))
+		return 0;
+	*out = crp_from_u64(crp_as_u64(y) ^ ((uint64_t)((ki << 22) & 0x80000000u) << 32));
+	return 1;
+}
+
+/* cos(x) for shift 0, sin(x) for shift 3, correctly rounded, out of line: the rest of crp_cos_turn's arguments */
+CRP_MATH_COLD double crp_cos_cr_cold(double x, int shift) {
+	double v;
+	if (crp_cos_quick_shift(x, shift, &v))
+		return v;
+	return crp_cos_accurate_shift(x, shift);
+}
+
+/* cos(x), correctly rounded, through the whole-turn table */
+CRP_MATH_FN double crp_cos_cr_turn(double x, const double *tab) {
+	double v;
+	if (crp_cos_turn(x, 0, tab, &v))
+		return v;
+	return crp_cos_cr_cold(x, 0);
+}
+
+/* sin(x) likewise: sin x = cos(x - pi/2), a quarter turn is 256 entries */
+CRP_MATH_FN double crp_sin_cr_turn(double x, const double *tab) {
+	double v;
+	if (crp_cos_turn(x, 256, tab, &v))
+		return v;
+	return crp_cos_cr_cold(x, 3);
+}
+
 /* log(x) for finite x > 0: the double-double logarithm (absolute error about 2^-104)
  * rounded once; the same bits on the host and the device */
 CRP_MATH_FN double crp_log_dd_rn(double x) {

@@ -118,7 +118,8 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 	constexpr bool kAdaptive = (KIND == PK_BP_ADAPTIVE || KIND == PK_CK_ADAPTIVE);
 	constexpr unsigned long long kEvalsPerTrial = kCK ? 6 : (kAdaptive ? 3 : 1);
 	const int lane = __lane_id();
-	F field = field0; // the lane's copy: a field that reads the candidate's redshift binds it at refill
+	// the lane's copy: a field that reads the candidate's redshift binds it at refill
+	typename KernelField<F, MIX>::type field = KernelField<F, MIX>::make(field0);
 
 	bool have = false, exhausted = false, inProc = false;
 	CkB0Store<FloatValuedField<F>::value> b0; // the field at the trial sequence's start (adaptive CK), for retries

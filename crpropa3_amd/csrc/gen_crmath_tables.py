@@ -104,6 +104,31 @@ for j in range(33):
 out.append("};")
 out.append("")
 
+# sin(2 pi j/1024), j = 0..767: one and a half half-turns, so that entry j + 256 is cos(2 pi j/1024) for
+# j = 0..511.  The quarter-turn points are exact.
+out.append("/* sin(2 pi j/1024), j = 0..767, as {hi, lo} */")
+out.append("CRP_TABLE double crp_turn_tab[1536] = {")
+for j in range(768):
+    m = j % 512  # sin(pi + a) = -sin a
+    m = min(m, 512 - m)  # sin(pi - a) = sin a
+    if m <= 128:
+        v = dsin_cos(2 * PI * m / 1024)[0]
+    else:
+        v = dsin_cos(2 * PI * (256 - m) / 1024)[1]
+    if j >= 512:
+        v = -v
+    hi, lo = split_dd(v)
+    out.append("  %s, %s," % (fmt(hi), fmt(lo)))
+out.append("};")
+p1 = float(2 * PI / 1024)
+p2 = float(2 * PI / 1024 - Decimal(p1))
+p3 = float(2 * PI / 1024 - Decimal(p1) - Decimal(p2))
+out.append("/* 2 pi/1024 = P1 + P2 + P3, 53 bits each; 1024/(2 pi) */")
+for i, v in enumerate((p1, p2, p3)):
+    out.append("#define CRP_TURN_P%d %s" % (i + 1, fmt(v)))
+out.append("#define CRP_TURN_INV %s" % fmt(float(1024 / (2 * PI))))
+out.append("")
+
 # 1/n! as dd, n = 0..20
 out.append("/* 1/n!, n = 0..20, as {hi, lo} */")
 out.append("CRP_TABLE double crp_invfact_tab[42] = {")

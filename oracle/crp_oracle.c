@@ -1399,6 +1399,13 @@ void orc_cos_phases(const double *x, size_t n, double *quick, int32_t *decided, 
 	}
 }
 
+void orc_cos_turn_phases(const double *x, size_t n, int sine, double *quick, int32_t *decided, double *accurate) {
+	for (size_t i = 0; i < n; i++) {
+		decided[i] = crp_cos_turn(x[i], sine ? 256 : 0, crp_turn_tab, &quick[i]);
+		accurate[i] = crp_cos_accurate_shift(x[i], sine ? 3 : 0);
+	}
+}
+
 void orc_philox4x32_10(const uint32_t ctr[4], const uint32_t key[2], uint32_t out[4]) {
 	crp_philox_ctr c;
 	for (int i = 0; i < 4; i++)

@@ -4,6 +4,7 @@ differs from correct rounding."""
 from decimal import Decimal, getcontext
 
 import numpy as np
+import pytest
 
 import oracle_ctypes as O
 
@@ -79,6 +80,27 @@ def test_cos_quick_phase_agrees_with_accurate_phase():
     q, dec, a = O.cos_phases(x)
     assert dec.mean() > 0.9
     assert np.array_equal(q[dec].view(np.uint64), a[dec].view(np.uint64))
+
+
+@pytest.mark.parametrize("sine", [False, True])
+def test_cos_turn_phase_agrees_with_accurate_phase(sine):
+    """The quick phase over the whole-turn table: every value it decides equals the accurate phase's, near
+    table points, halfway between them and near the zeros and extrema too, and it leaves few arguments
+    undecided; tiny, huge, infinite and NaN arguments are left to the other phases or are right."""
+    rng = np.random.default_rng(17)
+    n = 200000
+    step = np.pi / 512
+    x = np.concatenate([rng.uniform(-10, 10, n), rng.uniform(-1e6, 1e6, n), rng.uniform(-1.3e7, 1.3e7, n),
+                        np.floor(rng.uniform(-1e6, 1e6, n)) * step + rng.uniform(-1e-9, 1e-9, n),
+                        (np.floor(rng.uniform(-1e4, 1e4, n)) + 0.5) * step + rng.uniform(-1e-12, 1e-12, n),
+                        np.floor(rng.uniform(0, 1e5, n)) * (np.pi / 2) + rng.uniform(-5e-7, 5e-7, n)])
+    q, dec, a = O.cos_turn_phases(x, sine)
+    assert dec[:3 * n].mean() > 0.999
+    assert np.array_equal(q[dec].view(np.uint64), a[dec].view(np.uint64))
+    x = np.array([0.0, -0.0, 1e-300, -1e-12, 2.0 ** 30, -1e300, np.inf, -np.inf, np.nan])
+    q, dec, a = O.cos_turn_phases(x, sine)
+    assert np.array_equal(q[dec].view(np.uint64), a[dec].view(np.uint64))
+    assert not dec[4:].any()
 
 
 def test_philox_known_answers():

@@ -560,26 +560,37 @@ struct FieldGridCells {
 	GridDesc g;
 	const float *cells; // [nx*ny*nz][32]
 
-	__device__ __forceinline__ V3 eval(const V3 &p) const {
-		if (g.clip) {
-			bool in = (p.x >= g.origin[0]) && (p.x <= g.edge[0]);
-			in &= (p.y >= g.origin[1]) && (p.y <= g.edge[1]);
-			in &= (p.z >= g.origin[2]) && (p.z <= g.edge[2]);
-			if (!in)
-				return v3(0.0, 0.0, 0.0);
-		}
+	__device__ __forceinline__ bool outside(const V3 &p) const {
+		if (!g.clip)
+			return false;
+		bool in = (p.x >= g.origin[0]) && (p.x <= g.edge[0]);
+		in &= (p.y >= g.origin[1]) && (p.y <= g.edge[1]);
+		in &= (p.z >= g.origin[2]) && (p.z <= g.edge[2]);
+		return !in;
+	}
+	// the cell of a position and the position within it
+	__device__ __forceinline__ size_t cell(const V3 &p, double &fx, double &fy, double &fz) const {
 		double rx = div_cr(p.x - g.gridOrigin[0], g.spacing[0], g.invSpacing[0], g.fastDiv);
 		double ry = div_cr(p.y - g.gridOrigin[1], g.spacing[1], g.invSpacing[1], g.fastDiv);
 		double rz = div_cr(p.z - g.gridOrigin[2], g.spacing[2], g.invSpacing[2], g.fastDiv);
 		int x0, x1, y0, y1, z0, z1;
-		double fx, fy, fz;
 		periodic_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
 		periodic_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
 		periodic_clamp(rz, g.nz, g.invN[2], z0, z1, fz);
+		return ((size_t)x0 * g.ny + y0) * g.nz + z0;
+	}
+	// mixed precision: reciprocal spacing, division-free periodic wrap
+	__device__ __forceinline__ size_t cellf(const V3 &p, float &fx, float &fy, float &fz) const {
+		int x0, y0, z0;
+		periodic_cell_fast((p.x - g.gridOrigin[0]) * g.invSpacing[0], g.nx, 1.0 / g.nx, x0, fx);
+		periodic_cell_fast((p.y - g.gridOrigin[1]) * g.invSpacing[1], g.ny, 1.0 / g.ny, y0, fy);
+		periodic_cell_fast((p.z - g.gridOrigin[2]) * g.invSpacing[2], g.nz, 1.0 / g.nz, z0, fz);
+		return ((size_t)x0 * g.ny + y0) * g.nz + z0;
+	}
+	// the sum over the corners of Grid.h:572-579
+	static __device__ __forceinline__ V3 sum(const float4 *c, double fx, double fy, double fz) {
 		const float wx0 = (float)fx, wy0 = (float)fy, wz0 = (float)fz;
 		const float wx1 = (float)(1 - fx), wy1 = (float)(1 - fy), wz1 = (float)(1 - fz);
-		const size_t cidx = ((size_t)x0 * g.ny + y0) * g.nz + z0;
-		const float4 *c = reinterpret_cast<const float4 *>(cells + kCellFloats * cidx);
 		const float4 q0 = c[0], q1 = c[1], q2 = c[2], q3 = c[3], q4 = c[4], q5 = c[5];
 		const float v[24] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w,
 		                     q3.x, q3.y, q3.z, q3.w, q4.x, q4.y, q4.z, q4.w, q5.x, q5.y, q5.z, q5.w};
@@ -599,27 +610,26 @@ struct FieldGridCells {
 		}
 		return v3((double)b[0], (double)b[1], (double)b[2]);
 	}
-
-	// mixed precision: reciprocal spacing, division-free periodic wrap, fused FP32 sum
-	__device__ __forceinline__ float3 evalf(const V3 &p) const {
-		if (g.clip) {
-			bool in = (p.x >= g.origin[0]) && (p.x <= g.edge[0]);
-			in &= (p.y >= g.origin[1]) && (p.y <= g.edge[1]);
-			in &= (p.z >= g.origin[2]) && (p.z <= g.edge[2]);
-			if (!in)
-				return make_float3(0.f, 0.f, 0.f);
-		}
-		int x0, y0, z0;
-		float fx, fy, fz;
-		periodic_cell_fast((p.x - g.gridOrigin[0]) * g.invSpacing[0], g.nx, 1.0 / g.nx, x0, fx);
-		periodic_cell_fast((p.y - g.gridOrigin[1]) * g.invSpacing[1], g.ny, 1.0 / g.ny, y0, fy);
-		periodic_cell_fast((p.z - g.gridOrigin[2]) * g.invSpacing[2], g.nz, 1.0 / g.nz, z0, fz);
-		const size_t cidx = ((size_t)x0 * g.ny + y0) * g.nz + z0;
-		const float4 *c = reinterpret_cast<const float4 *>(cells + kCellFloats * cidx);
+	static __device__ __forceinline__ float3 sumf(const float4 *c, float fx, float fy, float fz) {
 		const float4 q0 = c[0], q1 = c[1], q2 = c[2], q3 = c[3], q4 = c[4], q5 = c[5];
 		const float v[24] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w,
 		                     q3.x, q3.y, q3.z, q3.w, q4.x, q4.y, q4.z, q4.w, q5.x, q5.y, q5.z, q5.w};
 		return trilinear_f32(v, fx, fy, fz);
+	}
+
+	__device__ __forceinline__ V3 eval(const V3 &p) const {
+		if (outside(p))
+			return v3(0.0, 0.0, 0.0);
+		double fx, fy, fz;
+		const size_t c = cell(p, fx, fy, fz);
+		return sum(reinterpret_cast<const float4 *>(cells + kCellFloats * c), fx, fy, fz);
+	}
+	__device__ __forceinline__ float3 evalf(const V3 &p) const {
+		if (outside(p))
+			return make_float3(0.f, 0.f, 0.f);
+		float fx, fy, fz;
+		const size_t c = cellf(p, fx, fy, fz);
+		return sumf(reinterpret_cast<const float4 *>(cells + kCellFloats * c), fx, fy, fz);
 	}
 };
 
@@ -784,6 +794,11 @@ struct FieldPlaneWave {
 	}
 };
 
+// Fields whose evaluation is one computation of all 64 lanes: callers reach it with the whole wave converged
+template <class F> struct WaveField {
+	static constexpr bool value = false;
+};
+
 // FieldPlaneWave with the cosine's table in LDS
 struct FieldPlaneWaveLds : FieldPlaneWave {
 	const double *tab;
@@ -791,17 +806,20 @@ struct FieldPlaneWaveLds : FieldPlaneWave {
 };
 
 // The field a propagation kernel evaluates for its argument: `make` is called once by every thread of
-// the workgroup.  The FP64 plane waves copy the cosine's 12 KB table to LDS: 64 lanes read 64 entries of
-// it per mode, which as global loads would be up to 128 line requests per mode and wave.  The mode loop is
-// bound by FP64 issue: 65 vector instructions a mode with this table against about 230 with the octant
-// table and its selection; 2^18 particles x 300 steps x 256 modes in 52.7 ms against 147.5.
+// the workgroup; `lds` are kLdsPerWave bytes of dynamic LDS for each of its waves.  The FP64 plane waves
+// copy the cosine's 12 KB table to LDS: 64 lanes read 64 entries of it per mode, which as global loads
+// would be up to 128 line requests per mode and wave.  The mode loop is bound by FP64 issue: 65 vector
+// instructions a mode with this table against about 230 with the octant table and its selection; 2^18
+// particles x 300 steps x 256 modes in 52.7 ms against 147.5.
 template <class F, bool MIX> struct KernelField {
 	typedef F type;
-	static __device__ __forceinline__ type make(const F &f) { return f; }
+	static constexpr int kLdsPerWave = 0;
+	static __device__ __forceinline__ type make(const F &f, char *) { return f; }
 };
 template <> struct KernelField<FieldPlaneWave, false> {
 	typedef FieldPlaneWaveLds type;
-	static __device__ __forceinline__ type make(const FieldPlaneWave &f) {
+	static constexpr int kLdsPerWave = 0;
+	static __device__ __forceinline__ type make(const FieldPlaneWave &f, char *) {
 		__shared__ double tab[2 * CRP_TURN_ENTRIES];
 		for (int i = threadIdx.x; i < 2 * CRP_TURN_ENTRIES; i += blockDim.x)
 			tab[i] = crp_turn_tab[i];
@@ -809,6 +827,71 @@ template <> struct KernelField<FieldPlaneWave, false> {
 		type r;
 		r.w = f.w;
 		r.tab = tab;
+		return r;
+	}
+};
+
+// FieldGridCells whose cell lines are gathered by the wave together.  A lane that reads its own line does
+// it in six 16-byte loads, and each of them translates an address for every lane: once the table outgrows
+// the reach of the first-level translation cache (about 3 GB) all six miss, and random lines come at
+// 1.3e10/s.  Here eight lanes read one line in one load, piece by piece, straight into LDS, and eight
+// loads serve the wave's 64 lines: one translation per line, 4.6e10 lines/s at 17 GB; below the cliff
+// both ways reach the same 5.3e10/s, and the lane's own loads need no LDS (measured, 96 bytes per line).
+// Lane 8g + j loads piece j ^ p of the line of lane 8g + p in load p, so that the eight lanes of a group
+// find their pieces in eight different 16-byte columns of LDS when they read them back.
+struct FieldGridCellsWave : FieldGridCells {
+	static constexpr int kLdsPerWave = 8 * 1024;
+	char *lds; // the wave's 8 KB
+
+	template <int P> __device__ __forceinline__ void load(unsigned c, int lane) const {
+		const unsigned line = (unsigned)__builtin_amdgcn_ds_swizzle((int)c, 0x18 | (P << 5)); // lane 8g + P's
+		const int piece = (lane & 7) ^ P;
+		if (piece < 6) // 96 of a line's 128 bytes hold corners
+			__builtin_amdgcn_global_load_lds(
+			    (const __attribute__((address_space(1))) void *)(cells + (size_t)kCellFloats * line + 4 * piece),
+			    (__attribute__((address_space(3))) void *)(lds + P * 1024), 16, 0, 0);
+	}
+	// the six pieces of this lane's line; every lane of the wave calls it, with a cell of the table
+	__device__ __forceinline__ void gather(size_t cidx, float4 q[6]) const {
+		const int lane = __lane_id();
+		const unsigned c = (unsigned)cidx;
+		load<0>(c, lane); load<1>(c, lane); load<2>(c, lane); load<3>(c, lane);
+		load<4>(c, lane); load<5>(c, lane); load<6>(c, lane); load<7>(c, lane);
+		asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the lines are in LDS
+		const int p = lane & 7;
+		const char *r = lds + p * 1024 + (lane >> 3) * 128;
+#pragma unroll
+		for (int i = 0; i < 6; i++)
+			q[i] = *reinterpret_cast<const float4 *>(r + ((i ^ p) << 4));
+		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // and read before the next gather overwrites them
+	}
+	__device__ __forceinline__ V3 eval(const V3 &p) const {
+		double fx, fy, fz;
+		float4 q[6];
+		gather(cell(p, fx, fy, fz), q);
+		const V3 b = sum(q, fx, fy, fz);
+		return outside(p) ? v3(0.0, 0.0, 0.0) : b;
+	}
+	__device__ __forceinline__ float3 evalf(const V3 &p) const {
+		float fx, fy, fz;
+		float4 q[6];
+		gather(cellf(p, fx, fy, fz), q);
+		const float3 b = sumf(q, fx, fy, fz);
+		return outside(p) ? make_float3(0.f, 0.f, 0.f) : b;
+	}
+};
+template <> struct WaveField<FieldGridCellsWave> {
+	static constexpr bool value = true;
+};
+// the argument a kernel is launched with for FieldGridCellsWave
+struct FieldGridCellsBig : FieldGridCells {};
+template <bool MIX> struct KernelField<FieldGridCellsBig, MIX> {
+	typedef FieldGridCellsWave type;
+	static constexpr int kLdsPerWave = FieldGridCellsWave::kLdsPerWave;
+	static __device__ __forceinline__ type make(const FieldGridCellsBig &f, char *lds) {
+		type r;
+		static_cast<FieldGridCells &>(r) = f;
+		r.lds = lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kLdsPerWave;
 		return r;
 	}
 };
@@ -862,6 +945,9 @@ template <> struct FloatValuedField<FieldGridCells> {
 template <> struct FloatValuedField<FieldGrid> {
 	static constexpr bool value = true;
 };
+template <> struct FloatValuedField<FieldGridCellsWave> {
+	static constexpr bool value = true;
+};
 template <bool F32> struct CkB0Store;
 template <> struct CkB0Store<false> {
 	V3 B;
@@ -888,7 +974,15 @@ __device__ __forceinline__ void ck_dydt_mixed(const F &field, const YM &y, float
                                               CkB0f *b0 = nullptr) {
 	n = unit3(y.u);                 // velocity / c
 	float3 B;
-	if (b0 && b0->have) {
+	if (WaveField<F>::value && b0) { // the whole wave evaluates while any lane needs it
+		if (__ballot(!b0->have)) {
+			const float3 e = field.evalf(y.x);
+			if (!b0->have)
+				b0->B = e;
+			b0->have = true;
+		}
+		B = b0->B;
+	} else if (b0 && b0->have) {
 		B = b0->B;
 	} else {
 		B = field.evalf(y.x);
@@ -984,7 +1078,15 @@ __device__ __forceinline__ Y ck_dydt(const F &field, const Y &y, double qcE,
 	const double invn = 1 / n;
 	d.x = v3(div_rn(y.u.x, n, invn) * kCLight, div_rn(y.u.y, n, invn) * kCLight, div_rn(y.u.z, n, invn) * kCLight);
 	V3 B;
-	if (b0 && b0->have) {
+	if (WaveField<F>::value && b0) { // the whole wave evaluates while any lane needs it
+		if (__ballot(!b0->have)) {
+			const V3 e = field.eval(y.x);
+			if (!b0->have)
+				b0->put(e);
+			b0->have = true;
+		}
+		B = b0->get();
+	} else if (b0 && b0->have) {
 		B = b0->get();
 	} else {
 		B = field.eval(y.x);

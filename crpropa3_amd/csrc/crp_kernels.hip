@@ -411,7 +411,9 @@ static int launch_propagate(const F &f, const crp_propagator *p, const Params &P
 		return CRP_E_HIP;
 	const int block = (p->block == 64 || p->block == 128) ? p->block : 256;
 	int bpcMax = 0;
-	const size_t lds = (size_t)kColdDoubles * block * sizeof(double);
+	size_t lds = (size_t)kColdDoubles * block * sizeof(double);
+	if (KIND != PK_SDE)
+		lds += (size_t)KernelField<F, MIX>::kLdsPerWave * (block / 64);
 	CRP_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpcMax, kern, block, lds));
 	if (bpcMax < 1)
 		bpcMax = 1;
@@ -538,6 +540,22 @@ static int dispatch_kind(const F &f, const crp_propagator *p, const Params &P, c
 	if (p->precision == CRP_PRECISION_MIXED)
 		return dispatch_kind_p<F, true>(f, p, P, b, launches);
 	return dispatch_kind_p<F, false>(f, p, P, b, launches);
+}
+
+// A cell table beyond the reach of the first-level address translation is gathered by waves
+// (FieldGridCellsWave).  The rate of a lane's own loads falls from 5.3e10 lines/s at 2 GiB and 4.9e10 at
+// 3.0 GB to 1.7e10 at 3.2 GB and 1.3e10 at 17 GB; the waves' loads reach 4.9e10 at 3.2 GB and 4.6e10 at
+// 17 GB.  Line numbers are 32 bits.
+constexpr size_t kWaveGatherBytes = 3000000000ull;
+
+static int dispatch_cells(const FieldGridCells &f, const crp_propagator *p, const Params &P, crp_batch *b,
+                          int *launches) {
+	const size_t ncell = (size_t)f.g.nx * f.g.ny * f.g.nz;
+	if (p->type == 2 || ncell * kCellFloats * sizeof(float) <= kWaveGatherBytes || ncell > 0xffffffffull)
+		return dispatch_kind(f, p, P, b, launches);
+	const FieldGridCellsBig big{f};
+	return p->precision == CRP_PRECISION_MIXED ? dispatch_kind_p<FieldGridCellsBig, true>(big, p, P, b, launches)
+	                                           : dispatch_kind_p<FieldGridCellsBig, false>(big, p, P, b, launches);
 }
 
 // ------------------------------------------------------------------ C ABI
@@ -2243,7 +2261,7 @@ int crp_propagate(const crp_propagator_t *p, crp_batch_t *b, long long max_steps
 		if (p->precision == CRP_PRECISION_MIXED && f->cells16)
 			rc = dispatch_kind_p<FieldGridCells16, true>(FieldGridCells16{f->grid, f->cells16}, p, P, b, &st.launches);
 		else
-			rc = f->cells ? dispatch_kind(FieldGridCells{f->grid, f->cells}, p, P, b, &st.launches)
+			rc = f->cells ? dispatch_cells(FieldGridCells{f->grid, f->cells}, p, P, b, &st.launches)
 			              : dispatch_kind(FieldGrid{f->grid}, p, P, b, &st.launches);
 		break;
 	case FK_PLANEWAVE: rc = dispatch_kind(FieldPlaneWave{f->pw}, p, P, b, &st.launches); break;

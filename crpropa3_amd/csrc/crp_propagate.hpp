@@ -100,29 +100,34 @@ __device__ __forceinline__ double pow_m02(double r) {
 }
 
 // Register budget: the FP64 path through the cell table is asked for 3 waves per SIMD (<= 168
-// VGPRs; it needs 169 unconstrained and then runs at 2), everything else is left to the compiler.
+// VGPRs; it needs 169 unconstrained and then runs at 2), gathered by waves on the mixed path for 2 (it
+// needs 257); everything else is left to the compiler.
 template <class F>
 struct WavesHint {
-	static constexpr int fp64 = 1;
+	static constexpr int fp64 = 1, mixed = 1;
 };
 template <>
 struct WavesHint<FieldGridCells> {
-	static constexpr int fp64 = 3;
+	static constexpr int fp64 = 3, mixed = 1;
+};
+template <>
+struct WavesHint<FieldGridCellsBig> {
+	static constexpr int fp64 = 1, mixed = 2;
 };
 
 template <class F, int KIND, bool MIX>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MIX ? 1 : WavesHint<F>::fp64, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MIX ? WavesHint<F>::mixed : WavesHint<F>::fp64, 8)))
 k_propagate(F field0, Params P, Soa S, unsigned long long n,
                                                    unsigned long long *__restrict__ ctr) {
 	constexpr bool kCK = (KIND == PK_CK_FIXED || KIND == PK_CK_ADAPTIVE);
 	constexpr bool kAdaptive = (KIND == PK_BP_ADAPTIVE || KIND == PK_CK_ADAPTIVE);
 	constexpr unsigned long long kEvalsPerTrial = kCK ? 6 : (kAdaptive ? 3 : 1);
+	// fields whose evaluation is one computation of the whole wave: every lane takes part, busy or not
+	constexpr bool kWave = WaveField<typename KernelField<F, MIX>::type>::value;
 	const int lane = __lane_id();
-	// the lane's copy: a field that reads the candidate's redshift binds it at refill
-	typename KernelField<F, MIX>::type field = KernelField<F, MIX>::make(field0);
 
 	bool have = false, exhausted = false, inProc = false;
-	CkB0Store<FloatValuedField<F>::value> b0; // the field at the trial sequence's start (adaptive CK), for retries
+	CkB0Store<FloatValuedField<typename KernelField<F, MIX>::type>::value> b0; // the field at the trial sequence's start (adaptive CK), for retries
 	CkB0f b0f;
 	b0.have = false;
 	b0f.have = false;
@@ -144,6 +149,9 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 	double *const cPDx = cw + 192, *const cPDy = cw + 256, *const cPDz = cw + 320;
 	double *const cCur = cw + 384, *const cLen = cw + 448, *const cTim = cw + 512;
 	double *const cDet = cw + 576; // observer detection count (small integer held as a double)
+	// the lane's copy: a field that reads the candidate's redshift binds it at refill
+	typename KernelField<F, MIX>::type field =
+	    KernelField<F, MIX>::make(field0, (char *)(crp_cold + kColdDoubles * blockDim.x));
 
 	for (;;) {
 		if (nEval > 0x80000000u) { // flush this lane's counters long before they wrap
@@ -194,7 +202,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 				break;
 			continue;
 		}
-		if (!have)
+		if (!kWave && !have)
 			continue;
 
 		// ---- one trial of process() for this lane
@@ -203,59 +211,38 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 		Y yOut;          // FP64 path result
 		V3 oPos;         // mixed path result
 		float3 oDir;
-		if (!inProc) {
-			*cPPx = pos.x; *cPPy = pos.y; *cPPz = pos.z; // candidate->previous = current
+		// rectilinear propagation for neutral particles (PropagationBP.cpp:74-80)
+		auto neutral_trial = [&]() {
+			if (MIX)
+				oPos = v3(pos.x + (double)dirf.x * step, pos.y + (double)dirf.y * step, pos.z + (double)dirf.z * step);
+			else
+				yOut.x = v3(pos.x + dir.x * step, pos.y + dir.y * step, pos.z + dir.z * step);
+		};
+		// the trial of a fixed step, and of an adaptive one (returns the error over the tolerance)
+		auto fixed_trial = [&]() {
 			if (MIX) {
-				*cPDx = dirf.x; *cPDy = dirf.y; *cPDz = dirf.z;
-			} else {
-				*cPDx = dir.x; *cPDy = dir.y; *cPDz = dir.z;
-			}
-			if (q == 0) {
-				// rectilinear propagation for neutral particles (PropagationBP.cpp:74-80)
-				neutral = true;
-				step = dclip(next, P.minStep, P.maxStep);
-				if (MIX)
-					oPos = v3(pos.x + (double)dirf.x * step, pos.y + (double)dirf.y * step, pos.z + (double)dirf.z * step);
-				else
-					yOut.x = v3(pos.x + dir.x * step, pos.y + dir.y * step, pos.z + dir.z * step);
-				newStep = P.maxStep;
-				commit = true;
-			} else if (!kAdaptive) {
-				step = P.maxStep;
-				newStep = step;
-				if (MIX) {
-					if (kCK) {
-						double eU;
-						YM o;
-						ck_trystep_mixed(field, YM{pos, dirf}, step / kCLight, (float)((q * kCLight * kCLight) / E), o, eU);
-						oPos = o.x;
-						oDir = o.u;
-					} else {
-						oPos = pos;
-						oDir = dirf;
-						bp_dy_mixed(field, oPos, oDir, step, (float)((q * kCLight * kCLight) / (2 * E) * step / kCLight));
-					}
+				if (kCK) {
+					double eU;
+					YM o;
+					ck_trystep_mixed(field, YM{pos, dirf}, step / kCLight, (float)((q * kCLight * kCLight) / E), o, eU);
+					oPos = o.x;
+					oDir = o.u;
 				} else {
-					if (kCK) {
-						double eU;
-						ck_trystep(field, Y{pos, dir}, step / kCLight, (q * kCLight) / E, yOut, eU);
-					} else {
-						const double m_ = E / (kCLight * kCLight);
-						yOut = bp_dy(field, pos, dir, step, q, m_, 1 / m_);
-					}
+					oPos = pos;
+					oDir = dirf;
+					bp_dy_mixed(field, oPos, oDir, step, (float)((q * kCLight * kCLight) / (2 * E) * step / kCLight));
 				}
-				nEval += kEvalsPerTrial;
-				commit = true;
 			} else {
-				step = dclip(next, P.minStep, P.maxStep);
-				newStep = step;
-				inProc = true;
-				b0.have = false;
-				b0f.have = false;
+				if (kCK) {
+					double eU;
+					ck_trystep(field, Y{pos, dir}, step / kCLight, (q * kCLight) / E, yOut, eU);
+				} else {
+					const double m_ = E / (kCLight * kCLight);
+					yOut = bp_dy(field, pos, dir, step, q, m_, 1 / m_);
+				}
 			}
-		}
-		if (kAdaptive && inProc) {
-			double r;
+		};
+		auto adaptive_trial = [&]() -> double {
 			if (MIX) {
 				if (kCK) {
 					double eU;
@@ -264,36 +251,36 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 					                 &b0f);
 					oPos = o.x;
 					oDir = o.u;
-					r = eU / P.tol;
-				} else {
-					const double k0 = (q * kCLight * kCLight) / (2 * E) / kCLight;
-					oPos = pos;
-					oDir = dirf;
-					bp_dy_mixed(field, oPos, oDir, step, (float)(k0 * step));
-					V3 hPos = pos;
-					float3 hDir = dirf;
-					bp_dy_mixed(field, hPos, hDir, step / 2, (float)(k0 * (step / 2)));
-					bp_dy_mixed(field, hPos, hDir, step / 2, (float)(k0 * (step / 2)));
-					V3 d = v3(oPos.x - hPos.x, oPos.y - hPos.y, oPos.z - hPos.z);
-					double Sv = norm(d) / (step * 0.75);
-					r = __builtin_sqrt(3.0 * Sv * Sv) / P.tol;
+					return eU / P.tol;
 				}
-			} else {
-				if (kCK) {
-					double eU;
-					ck_trystep(field, Y{pos, dir}, step / kCLight, (q * kCLight) / E, yOut, eU, &b0);
-					r = eU / P.tol;
-				} else {
-					const double m_ = E / (kCLight * kCLight);
-					const double im_ = 1 / m_;
-					yOut = bp_dy(field, pos, dir, step, q, m_, im_);
-					Y half = bp_dy(field, pos, dir, step / 2, q, m_, im_);
-					Y cmp = bp_dy(field, half.x, half.u, step / 2, q, m_, im_);
-					V3 d = v3(yOut.x.x - cmp.x.x, yOut.x.y - cmp.x.y, yOut.x.z - cmp.x.z);
-					double Sv = norm(d) / (step * (1 - 1 / 4.));
-					r = __builtin_sqrt((Sv * Sv + Sv * Sv) + Sv * Sv) / P.tol;
-				}
+				const double k0 = (q * kCLight * kCLight) / (2 * E) / kCLight;
+				oPos = pos;
+				oDir = dirf;
+				bp_dy_mixed(field, oPos, oDir, step, (float)(k0 * step));
+				V3 hPos = pos;
+				float3 hDir = dirf;
+				bp_dy_mixed(field, hPos, hDir, step / 2, (float)(k0 * (step / 2)));
+				bp_dy_mixed(field, hPos, hDir, step / 2, (float)(k0 * (step / 2)));
+				V3 d = v3(oPos.x - hPos.x, oPos.y - hPos.y, oPos.z - hPos.z);
+				double Sv = norm(d) / (step * 0.75);
+				return __builtin_sqrt(3.0 * Sv * Sv) / P.tol;
 			}
+			if (kCK) {
+				double eU;
+				ck_trystep(field, Y{pos, dir}, step / kCLight, (q * kCLight) / E, yOut, eU, &b0);
+				return eU / P.tol;
+			}
+			const double m_ = E / (kCLight * kCLight);
+			const double im_ = 1 / m_;
+			yOut = bp_dy(field, pos, dir, step, q, m_, im_);
+			Y half = bp_dy(field, pos, dir, step / 2, q, m_, im_);
+			Y cmp = bp_dy(field, half.x, half.u, step / 2, q, m_, im_);
+			V3 d = v3(yOut.x.x - cmp.x.x, yOut.x.y - cmp.x.y, yOut.x.z - cmp.x.z);
+			double Sv = norm(d) / (step * (1 - 1 / 4.));
+			return __builtin_sqrt((Sv * Sv + Sv * Sv) + Sv * Sv) / P.tol;
+		};
+		// accept or repeat an adaptive trial, and the next step's size
+		auto step_control = [&](double r) {
 			nEval += kEvalsPerTrial; // the reference's getField calls, the reused first stage included
 			if (r > 1) {
 				if (step == P.minStep) {
@@ -313,7 +300,50 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 				}
 				commit = true;
 			}
+		};
+		// with kWave every lane goes through the trial, and those without a trial of their own (no particle,
+		// or a neutral one) drop its results
+		if (have && !inProc) {
+			*cPPx = pos.x; *cPPy = pos.y; *cPPz = pos.z; // candidate->previous = current
+			if (MIX) {
+				*cPDx = dirf.x; *cPDy = dirf.y; *cPDz = dirf.z;
+			} else {
+				*cPDx = dir.x; *cPDy = dir.y; *cPDz = dir.z;
+			}
+			if (q == 0) {
+				neutral = true;
+				step = dclip(next, P.minStep, P.maxStep);
+				if (!kWave)
+					neutral_trial();
+				newStep = P.maxStep;
+				commit = true;
+			} else if (!kAdaptive) {
+				step = P.maxStep;
+				newStep = step;
+				if (!kWave)
+					fixed_trial();
+				nEval += kEvalsPerTrial;
+				commit = true;
+			} else {
+				step = dclip(next, P.minStep, P.maxStep);
+				newStep = step;
+				inProc = true;
+				b0.have = false;
+				b0f.have = false;
+			}
 		}
+		const bool go = have && inProc;
+		if (kWave && !go)
+			b0.have = b0f.have = true; // asks for no evaluation of its own
+		if (kWave && !kAdaptive)
+			fixed_trial();
+		if (kAdaptive && (kWave || go)) {
+			const double r = adaptive_trial();
+			if (go)
+				step_control(r);
+		}
+		if (kWave && neutral)
+			neutral_trial();
 		if (!commit)
 			continue;
 

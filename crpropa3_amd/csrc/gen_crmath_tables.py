@@ -82,6 +82,16 @@ for j in range(256):
 out.append("};")
 out.append("")
 
+# 1/c_j rounded to a double, and -log of that double, for the logarithm's quick phase
+out.append("/* {R_j, -log R_j hi, lo}, R_j = 1/(1 + (j + 0.5)/256) rounded, j = 0..255 */")
+out.append("CRP_TABLE double crp_logr_tab[768] = {")
+for j in range(256):
+    r = float(1 / (Decimal(1) + (Decimal(j) + Decimal("0.5")) / 256))
+    hi, lo = split_dd(-dln(Decimal(r)))
+    out.append("  %s, %s, %s," % (fmt(r), fmt(hi), fmt(lo)))
+out.append("};")
+out.append("")
+
 # 2^(j/256), j = 0..255
 out.append("/* 2^(j/256), j = 0..255, as {hi, lo} */")
 out.append("CRP_TABLE double crp_exp2_tab[512] = {")

@@ -1,0 +1,173 @@
+"""The straight-line forms of the FP64 steps (range tests merged, repeated with the tested form where one
+fails), the folded mirror boundary, small batches spread over the GPU, quads of lanes on tricubic grids and the
+pinned transfers: bit for bit against the oracle, at the operands and sizes where each can go wrong."""
+import numpy as np
+import pytest
+
+import oracle_ctypes as O
+from crpropa3_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+KPC = 3.0856775814913674e19
+EPLUS = 1.602176487e-19
+EEV = 1e18 * EPLUS
+
+
+def same(a, b):
+    a = np.ascontiguousarray(a, dtype=np.float64)
+    b = np.ascontiguousarray(b, dtype=np.float64)
+    return np.array_equal(a.view(np.uint64), b.view(np.uint64))
+
+
+def noise(shape, seed=3):
+    return (np.random.default_rng(seed).normal(size=tuple(shape) + (3,)) * 1e-13).astype(np.float32)
+
+
+def compare(field, ofield, kind, pos, d, E, q, steps, lo, hi, tol):
+    ref = O.OracleState(pos, d, E, q)
+    O.propagate(ofield, O.PROP_BP if kind == "BP" else O.PROP_CK, ref, steps, tolerance=tol, min_step=lo, max_step=hi,
+                libm=O.LIBM_CR)
+    p = capi.Propagator(kind, field, tol, lo, hi)
+    b = capi.Batch(len(E))
+    b.upload(pos, O.normalise(d), E, q)
+    p.propagate(b, max_steps=steps)
+    out = b.download()
+    for k in ("pos", "dir", "prev_pos", "prev_dir", "current_step", "next_step", "trajectory_length", "time"):
+        assert same(out[k], getattr(ref, k)), k
+    return out
+
+
+def special_particles():
+    """Directions with zero, negative-zero and tiny components, energies and charges from far below to far above
+    the bounds of the straight line, positions at the origin and far away, between ordinary ones."""
+    dirs = [(1, 0, 0), (0, -1, 0), (-0.0, 0.0, 1), (1, 1e-170, 0), (1e-300, 1, 1), (1, 2, 3), (3, -2, 1e-160),
+            (1e-308, 1e-308, 1)]
+    es = [1e-60, 1e-30, 1e-10, 1 * EEV, 1e3 * EEV, 1e40, 1e90]
+    qs = [EPLUS, -EPLUS, 26 * EPLUS, 1e-40, 1e30, 0.0]
+    ps = [(0, 0, 0), (-0.0, 1e-200, 3e20), (1e21, -2e21, 5e20), (1e28, 1e21, 1e21), (3e19, 3e19, 3e19)]
+    rows = [(p, d, e, q) for p in ps for d in dirs for e in es for q in qs]
+    P, D, E, Q = (np.array(x, dtype=np.float64) for x in zip(*rows))
+    return P, D, E, Q
+
+
+@pytest.mark.parametrize("reflective", [False, True])
+@pytest.mark.parametrize("kind,fixed", [("BP", True), ("BP", False), ("CK", True), ("CK", False)])
+def test_extreme_operands(kind, fixed, reflective):
+    g = noise((7, 5, 6))
+    g[0, 0, 0] = 0.0  # cells with zero, tiny and huge values
+    g[1, 1, 1] = (1e-45, -1e-40, 0.0)
+    g[3, 2, 2] = (1e30, -1e20, 1e-20)
+    P, D, E, Q = special_particles()
+    if reflective:  # the reference's mirror loop takes a pass per box length
+        keep = np.abs(P).max(axis=1) < 1e25
+        P, D, E, Q = P[keep], D[keep], E[keep], Q[keep]
+    sp = [2e19, 3e19, 1e19]
+    f = capi.Field.grid3f(g, [-1e19, 0, 0], sp, reflective=reflective)
+    of = O.OracleField.grid(g, [-1e19, 0, 0], sp, reflective)
+    lo, hi = (1e19, 1e19) if fixed else (1e17, 1e20)
+    ref = O.OracleState(P, D, E, Q)
+    O.propagate(of, O.PROP_BP if kind == "BP" else O.PROP_CK, ref, 3, tolerance=1e-3, min_step=lo, max_step=hi,
+                libm=O.LIBM_CR)
+    b = capi.Batch(len(E))
+    b.upload(P, O.normalise(D), E, Q)
+    capi.Propagator(kind, f, 1e-3, lo, hi).propagate(b, max_steps=3)
+    out = b.download()
+    for k in ("pos", "dir", "current_step", "next_step"):
+        a, r = out[k], getattr(ref, k)
+        ok = (a.view(np.uint64) == r.view(np.uint64)) | (np.isnan(a) & np.isnan(r))
+        assert ok.all(), (k, np.argwhere(~ok)[:4], a[~ok][:4], r[~ok][:4])
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 3, 1), (5, 8, 7), (97, 4, 33)])
+def test_mirror_fold(shape):
+    """Reflective positions inside, on and around the mirrors, up to 3000 boxes away."""
+    rng = np.random.default_rng(7)
+    g = noise(shape)
+    sp, o = 1.5, [0.25, -3.0, 7.0]
+    n = np.array(shape)
+    half = rng.integers(-40, 40, (4000, 3)) * 0.5 * n + rng.choice([0, 0.5, -0.5, 1e-9, -1e-9, 1e-16], (4000, 3))
+    cells = np.concatenate([half, rng.uniform(-3, 4, (4000, 3)) * n, rng.uniform(-3000, 3000, (2000, 3)) * n])
+    pos = np.array(o) + 0.5 * sp + cells * sp
+    pos = np.concatenate([pos, np.nextafter(pos[:4000], 1e9), np.nextafter(pos[:4000], -1e9)])
+    want = O.OracleField.grid(g, o, sp, True).eval(pos)
+    assert same(capi.Field.grid3f(g, o, sp, reflective=True).eval(pos), want)
+
+
+@pytest.mark.parametrize("n", [1, 5, 63, 1023, 1025, 4097, 66000])
+@pytest.mark.parametrize("kind", ["BP", "CK"])
+def test_spread_batches(kind, n):
+    """A particle's steps do not depend on how many share its wave."""
+    rng = np.random.default_rng(11)
+    m = 4097
+    g = noise((16, 16, 16))
+    sp = [50 * KPC] * 3
+    d = rng.normal(size=(m, 3))
+    pos = rng.uniform(0, 800 * KPC, (m, 3))
+    E = 10 ** rng.uniform(0, 2, m) * EEV
+    q = np.where(np.arange(m) % 5 == 0, 0.0, EPLUS)
+    if n <= m:
+        pos, d, E, q = pos[:n], d[:n], E[:n], q[:n]
+    else:
+        pos, d, E, q = (np.concatenate([x] * (n // m + 1))[:n] for x in (pos, d, E, q))
+    ref = O.OracleState(pos[:m], d[:m], E[:m], q[:m])
+    O.propagate(O.OracleField.grid(g, [0, 0, 0], sp), O.PROP_BP if kind == "BP" else O.PROP_CK, ref, 20,
+                tolerance=1e-3, min_step=KPC, max_step=100 * KPC, libm=O.LIBM_CR)
+    b = capi.Batch(n)
+    b.upload(pos, O.normalise(d), E, q)
+    st = capi.Propagator(kind, capi.Field.grid3f(g, [0, 0, 0], sp), 1e-3, KPC, 100 * KPC).propagate(b, max_steps=20)
+    out = b.download()
+    assert st.accepted_steps == 20 * n
+    for i in range(0, n, m):
+        k = min(m, n - i)
+        assert same(out["pos"][i:i + k], ref.pos[:k]) and same(out["next_step"][i:i + k], ref.next_step[:k])
+
+
+@pytest.mark.parametrize("shape,reflective,clip", [((1, 1, 1), False, False), ((2, 3, 5), True, False),
+                                                   ((4, 4, 4), False, True), ((33, 6, 19), False, False),
+                                                   ((33, 6, 19), True, True)])
+@pytest.mark.parametrize("kind,fixed", [("BP", True), ("BP", False), ("CK", True), ("CK", False)])
+def test_tricubic_quads(kind, fixed, shape, reflective, clip):
+    """Four lanes to a particle: every wrap of a row, ragged quads and waves, neutral particles among them."""
+    rng = np.random.default_rng(13)
+    n = 1003
+    g = noise(shape)
+    sp = [20 * KPC] * 3
+    f = capi.Field.grid3f(g, [0, 0, 0], sp, reflective=reflective, clip_volume=clip)
+    f.set_interpolation("TRICUBIC")
+    of = O.OracleField.grid(g, [0, 0, 0], sp, reflective, clip, interp=O.GRID_TRICUBIC)
+    L = np.array(shape) * 20 * KPC
+    pos = rng.uniform(-0.6, 1.6, (n, 3)) * L
+    q = np.where(np.arange(n) % 6 == 1, 0.0, EPLUS)
+    lo, hi = (20 * KPC, 20 * KPC) if fixed else (KPC, 60 * KPC)
+    compare(f, of, kind, pos, rng.normal(size=(n, 3)), 10 ** rng.uniform(0, 2, n) * EEV, q, 12, lo, hi, 1e-3)
+
+
+@pytest.mark.parametrize("n", [1, 10279, 10281, 250001])
+def test_download_returns_what_was_uploaded(n):
+    """One chunk, a chunk's edges and several threads."""
+    rng = np.random.default_rng(n)
+    v = {k: rng.normal(size=(n, 3)) for k in ("pos", "dir", "source_pos", "created_pos")}
+    s = {k: rng.normal(size=n) for k in ("energy", "charge", "current_step", "next_step", "trajectory_length", "time")}
+    w = dict(active=rng.integers(0, 2, n).astype(np.int32), detection_index=rng.integers(0, 9, n).astype(np.int32),
+             sde_step=rng.integers(0, 2 ** 32, n).astype(np.uint32))
+    b = capi.Batch(n)
+    b.upload(v["pos"], v["dir"], s["energy"], s["charge"], **{k: s[k] for k in list(s)[2:]}, **w,
+             source_pos=v["source_pos"], created_pos=v["created_pos"])
+    out = b.download()
+    for k, a in {**v, **s, **w, "prev_pos": v["pos"], "prev_dir": v["dir"]}.items():
+        assert np.array_equal(out[k].view(np.uint8), a.view(np.uint8)), k
+
+
+@pytest.mark.parametrize("precision", [capi.PRECISION_FP64, capi.PRECISION_MIXED])
+@pytest.mark.parametrize("n", [1, 255, 257, 43690, 43691, 100003])
+def test_staged_eval(n, precision):
+    """Positions that fill a slot and one more, against calls of 1000."""
+    g = noise((9, 11, 10))
+    f = capi.Field.grid3f(g, [0, 0, 0], 1.0)
+    pos = np.random.default_rng(n).uniform(-20, 30, (n, 3))
+    got = f.eval(pos, precision)
+    want = np.concatenate([f.eval(pos[i:i + 1000], precision) for i in range(0, n, 1000)])
+    assert same(got, want)
+    if precision == capi.PRECISION_FP64:
+        assert same(got, O.OracleField.grid(g, [0, 0, 0], 1.0).eval(pos))

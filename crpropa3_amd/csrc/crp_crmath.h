@@ -235,6 +235,72 @@ CRP_MATH_FN double crp_pow_cr(double x, double y) {
 	return v * crp_pow2i(s1) * crp_pow2i(s2);
 }
 
+/*
+ * Quick phase of pow (Ziv), finite normal x > 0 and |y log x| < 700: both halves in double around
+ * their large terms, about a seventh of the double-double phase's instructions.
+ *   log x = e ln2 - log R_j + log1p t with t = m R_j - 1 = th + tl exactly (|t| <= 2^-8.9):
+ *     log1p t = th + [tl - th tl - th^2/2 + th^3 (1/3 - th/4 + ... + th^6/9)], the bracket (<= 2^-18.8) in
+ *     double to a few ulps (2^-70), the large terms added exactly, ln2 to 2^-120: absolute error < 2^-69.5;
+ *   z = y log x as a pair (its error below 2^-69.5 |y| and 2^-104 |z|), and exp z as in crp_exp_quick, with
+ *     z's low part in the reduced argument: below 2^-69 relative.
+ * With |y| <= 1 that is below 2^-68.2; the value is returned when everything within 2^-66 of it rounds the
+ * same way.  Returns 0 when it does not decide (2.5e-4 of arguments).  logr and ex are crp_logr_tab and
+ * crp_exp2_tab or copies of them.
+ */
+CRP_MATH_FN int crp_pow_quick(double x, double y, const double *logr, const double *ex, double *out) {
+	const uint64_t u = crp_as_u64(x);
+	const uint32_t be = (uint32_t)(u >> 52) - 1u; /* 0..2045 for positive normal numbers */
+	const double m = crp_from_u64((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL); /* [1,2) */
+	const double *const T = logr + 3 * (int)((uint32_t)(u >> 44) & 255u);
+	const double R = T[0];
+	const crp_dd pm = crp_two_prod(m, R);
+	const double th = pm.hi - 1.0, tl = pm.lo; /* exact */
+	const double t2 = th * th;
+	const double ser = 1.0 / 3 + th * (-0.25 + th * (0.2 + th * (-1.0 / 6 + th * (1.0 / 7 + th * (-0.125 + th * (1.0 / 9))))));
+	const double fe = (double)((int)be - 1022);
+	const crp_dd a = crp_two_sum(fe * CRP_LN2_1, T[1]);
+	const crp_dd s = crp_two_sum(a.hi, th);
+	const double br = (t2 * th * ser + (tl - th * tl)) - 0.5 * t2;
+	const double llo = (s.lo + a.lo) + ((fe * CRP_LN2_2 + (T[2] + fe * CRP_LN2_3)) + br);
+	/* z = y log x */
+	const crp_dd zp = crp_two_prod(s.hi, y);
+	const double zl = zp.lo + llo * y;
+	const double zh = zp.hi;
+	if (!(be < 2046u && __builtin_fabs(zh) < 700.0 && __builtin_fabs(y) <= 1.0))
+		return 0;
+	/* exp(zh + zl) */
+	const double k = crp_rint(zh * CRP_INV_LN2_256);
+	const double r0 = zh - k * CRP_LN2_256_1; /* exact */
+	const crp_dd r = crp_two_sum(r0, -k * CRP_LN2_256_2);
+	const crp_dd rr = crp_fast_two_sum(r.hi, r.lo - k * CRP_LN2_256_3 + zl);
+	const double rh = rr.hi, rl = rr.lo;
+	const double q = rh * rh * (0.5 + rh * (1.0 / 6 + rh * (1.0 / 24 + rh * (1.0 / 120 + rh * (1.0 / 720)))));
+	const double em = rl + rh * rl + q; /* expm1(r) - rh */
+	const int ki = (int)k, j = ki & 255, sc = (ki - j) / 256;
+	const crp_dd E = crp_tab_dd(ex, j);
+	const crp_dd p = crp_two_prod(E.hi, rh);
+	const double lo = p.lo + (E.hi * em + (E.lo + E.lo * (rh + em)));
+	const crp_dd sh = crp_fast_two_sum(E.hi, p.hi);
+	const double hi = sh.hi, l2 = sh.lo + lo, eps = hi * 0x1p-66;
+	const double v = hi + (l2 + eps);
+	if (v != hi + (l2 - eps))
+		return 0;
+	*out = v * crp_pow2i(sc); /* |z| < 700: normal */
+	return 1;
+}
+
+CRP_MATH_COLD double crp_pow_cr_cold(double x, double y) {
+	return crp_pow_cr(x, y);
+}
+
+/* pow(x, y), correctly rounded, |y| <= 1: the quick phase first */
+CRP_MATH_FN double crp_pow_cr_quick(double x, double y, const double *logr, const double *ex) {
+	double v;
+	if (crp_pow_quick(x, y, logr, ex, &v))
+		return v;
+	return crp_pow_cr_cold(x, y);
+}
+
 /* ---------------------------------------------------------- large arguments */
 /*
  * |x| = M 2^e reduced modulo pi/2 for any finite |x| >= 2^23 pi/2 (Payne and Hanek): only

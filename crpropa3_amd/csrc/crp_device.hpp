@@ -67,6 +67,73 @@ __device__ __forceinline__ double div_rn(double x, double s, double invs) {
 
 constexpr double kInvCLight = 1.0 / 299792458.0; // RN(1/c), folded by the compiler
 
+// The quotient of div_rn without its range test, for callers that test several operands at once and take
+// the tested form where one of them fails: the tests and their branches, one per quotient, are a third of a
+// Boris step's instructions and keep loads and independent steps from overlapping.  x = 0 is right too (the
+// sum would lose the sign of -0).
+__device__ __forceinline__ double div_fast(double x, double s, double invs) {
+	const double q = x * invs;
+	const double r = __builtin_fma(-q, s, x);
+	return __builtin_copysign(__builtin_fma(r, invs, q), q);
+}
+
+// RN(1/s) for s within [2^-500, 2^500] without the division's scaling and special cases: the hardware's
+// approximation (better than 2^-20) and a third-order step give 1/s to less than an ulp, and one more step
+// rounds it correctly unless the significand of s is all ones (Markstein; Handbook of Floating-Point
+// Arithmetic, the reciprocal with an FMA); 1/(2^k (2 - 2^-52)) rounds to 2^-(k+1) (1 + 2^-52).
+__device__ __forceinline__ double rcp_rn(double s) {
+	const double r = __builtin_amdgcn_rcp(s);
+	const double e = __builtin_fma(-s, r, 1.0);
+	const double y = __builtin_fma(r, __builtin_fma(e, e, e), r);
+	const int hi = __double2hiint(s);
+	const bool ones = (hi & 0xfffff) == 0xfffff && __double2loint(s) == -1;
+	const double z = __builtin_fma(__builtin_fma(-s, y, 1.0), y, y);
+	return ones ? __hiloint2double(0x7fd00000 - (hi & 0x7ff00000), 1) : z;
+}
+
+// RN(1/s) for s near 1; `bad` is set for |1 - s| > 2^-45.  With e = 1 - s (exact), 1/s = 1 + e + e^2 + ...: for
+// s > 1, 1 - |e| is a double and the rest too small to matter; for s < 1, e is a multiple of 2^-53 and where
+// 1 + e is a tie the rest decides it upwards, which e (1 + 2^-50) does as well.
+__device__ __forceinline__ double rcp_near_one(double s, bool &bad) {
+	const double e = 1.0 - s;
+	bad |= !(__builtin_fabs(e) <= 0x1p-45);
+	return __builtin_fma(e, 1.0 + 0x1p-50, 1.0);
+}
+
+// RN(sqrt(d)) for d near 1; `bad` is set for |d - 1| > 2^-44.  With e = d - 1 (exact), sqrt(d) = 1 + e/2 - e^2/8
+// + ...: 1 + e/2 is a double or halfway between two, and the rest, too small to matter otherwise, decides a tie
+// downwards, as |e| 2^-52 taken off does.
+__device__ __forceinline__ double sqrt_near_one(double d, bool &bad) {
+	const double e = d - 1.0, ae = __builtin_fabs(e);
+	bad |= !(ae <= 0x1p-44);
+	return 1.0 + __builtin_fma(ae, -0x1p-52, 0.5 * e);
+}
+
+// every component zero or of magnitude within [2^-500, 2^500) (infinities and NaN pass: their exponent reads 0)
+__device__ __forceinline__ bool in_div_range(const V3 &v) {
+	const int a = __builtin_amdgcn_frexp_exp(v.x), b = __builtin_amdgcn_frexp_exp(v.y),
+	          c = __builtin_amdgcn_frexp_exp(v.z);
+	const int lo = min(min(a, b), c), hi = max(max(a, b), c);
+	return lo > -500 && hi <= 500;
+}
+
+// v / s, component by component, with one range test
+__device__ __forceinline__ V3 div3_rn(const V3 &v, double s, double invs) {
+	V3 r = v3(div_fast(v.x, s, invs), div_fast(v.y, s, invs), div_fast(v.z, s, invs));
+	if (!(s > 0x1p-500 && s < 0x1p500 && in_div_range(v)))
+		r = v3(v.x / s, v.y / s, v.z / s);
+	return r;
+}
+
+// u / |u|, one range test
+__device__ __forceinline__ V3 unit_rn(const V3 &u) {
+	const double n = norm(u), invn = rcp_rn(n);
+	V3 r = v3(div_fast(u.x, n, invn), div_fast(u.y, n, invn), div_fast(u.z, n, invn));
+	if (!(n > 0x1p-500 && n < 0x1p500 && in_div_range(u)))
+		r = v3(u.x / n, u.y / n, u.z / n);
+	return r;
+}
+
 // ---------------------------------------------------------------- fields
 // Parameters as the host computes them from the reference's field objects.
 struct GridDesc {
@@ -78,7 +145,7 @@ struct GridDesc {
 	double origin[3], edge[3]; // clipVolume box: origin, origin + N*spacing (Grid.h:320-327)
 	double invSpacing[3];      // RN(1/spacing), computed on the host
 	double invN[3];            // 1/N per axis, for the division-free periodic wrap
-	int fastDiv;               // spacing within [2^-500, 2^500]: div_cr may use its reciprocal path
+	int fastDiv;               // spacing within [2^-300, 2^300]: its reciprocal may stand for the division
 	int interp;                // GridInterp: Grid::setInterpolationType (Grid.h:24-28, 255-264)
 };
 
@@ -167,13 +234,14 @@ __device__ __forceinline__ double div_cr(double x, double s, double invs, int fa
 }
 
 // ((i % n) + n) % n (Grid.h:31-34) without an integer division: floor(i * (1/n)) is within one
-// of floor(i/n) for |i| < 2^31, the remainder is corrected into [0, n).
+// of floor(i/n) for |i| <= 2^31, the remainder is corrected into [0, n).  The remainder lies within
+// (-n, 2n), so 32-bit arithmetic modulo 2^32 forms it (n < 2^30).
 __device__ __forceinline__ int wrap_index(int i, int n, double invn) {
-	const long long q = (long long)__builtin_floor((double)i * invn);
-	long long r = (long long)i - q * (long long)n;
+	const int q = (int)__builtin_floor((double)i * invn);
+	int r = (int)((unsigned)i - (unsigned)q * (unsigned)n);
 	r += (r < 0) ? n : 0;
 	r -= (r >= n) ? n : 0;
-	return (int)r;
+	return r;
 }
 
 __device__ __forceinline__ void periodic_clamp(double x, int n, double invn, int &lo, int &hi, double &frac) {
@@ -183,7 +251,22 @@ __device__ __forceinline__ void periodic_clamp(double x, int n, double invn, int
 	frac = x - fl;
 }
 
-__device__ __forceinline__ void reflective_clamp(double x, int n, int &lo, int &hi, double &frac) {
+// reflectiveClamp's loop (Grid.h:49-59) without its passes: mirrored at -1/2 once, moved by a multiple of the
+// period 2n and mirrored at n - 1/2 once, x lies in [-1/2, n - 1/2] where the loop ends.  Below 2^50 every
+// one of these operations is exact (a result is a multiple of the operand's last bit and no larger), as the
+// loop's are, and two points of [-1/2, n - 1/2] are never images of each other, so the bits agree.  The
+// multiple can come out one too large where x + 1/2 rounds up to it: x then lies just outside, which the
+// caller tests.
+__device__ __forceinline__ double mirror_fold(double x, int n, double invn) {
+	const double dn = (double)n, p = 2 * dn;
+	x = (x < -0.5) ? -x - 1 : x;
+	x = __builtin_fma(-__builtin_floor((x + 0.5) * (0.5 * invn)), p, x);
+	return (x > dn - 0.5) ? p - x - 1 : x;
+}
+
+__device__ __forceinline__ void reflective_clamp(double x, int n, double invn, int &lo, int &hi, double &frac) {
+	if (__builtin_fabs(x) < 0x1p50)
+		x = mirror_fold(x, n, invn);
 	while ((x < -0.5) || (x > (n - 0.5)))
 		x = 2 * n * (x > (n - 0.5)) - x - 1;
 	double fl = __builtin_floor(x);
@@ -193,6 +276,22 @@ __device__ __forceinline__ void reflective_clamp(double x, int n, int &lo, int &
 		lo = 0;
 		hi = 0;
 	}
+	frac = x - fl;
+}
+
+// one axis of a trilinear cell in a straight line, periodic or reflective; `bad` where reflective_clamp has
+// to be asked
+__device__ __forceinline__ void clamp_fast(double x, int n, double invn, bool refl, int &lo, int &hi, double &frac,
+                                           bool &bad) {
+	if (refl) { // the same for every lane
+		bad |= !(__builtin_fabs(x) < 0x1p50);
+		x = mirror_fold(x, n, invn);
+		bad |= !(x >= -0.5 && x <= n - 0.5);
+	}
+	const double fl = __builtin_floor(x);
+	const int i = (int)fl, w = wrap_index(i, n, invn);
+	lo = refl ? min(max(i, 0), n - 1) : w;
+	hi = refl ? min(max(i + 1, 0), n - 1) : (w + 1 == n ? 0 : w + 1);
 	frac = x - fl;
 }
 
@@ -373,31 +472,35 @@ __device__ __attribute__((noinline)) float scalar_grid_other(const GridDesc &g, 
 	return scalar_grid_other_inline(g, p);
 }
 
+// p in units of the spacing from the first point: the reference's (pos - gridOrigin) / spacing, with one
+// range test for the three.  Fast: without the division, `bad` set where it is needed.  A quotient of magnitude
+// below 2^-500 need not be rounded right (fastDiv: the spacing is within [2^-300, 2^300]): only its sign
+// reaches the cell, and the position within the cell rounds to 0 or 1 all the same.
+template <bool Fast>
+__device__ __forceinline__ void grid_position(const GridDesc &g, const V3 &p, double &rx, double &ry, double &rz,
+                                              bool *bad) {
+	const double dx = p.x - g.gridOrigin[0], dy = p.y - g.gridOrigin[1], dz = p.z - g.gridOrigin[2];
+	const double qx = dx * g.invSpacing[0], qy = dy * g.invSpacing[1], qz = dz * g.invSpacing[2];
+	rx = __builtin_fma(__builtin_fma(-qx, g.spacing[0], dx), g.invSpacing[0], qx);
+	ry = __builtin_fma(__builtin_fma(-qy, g.spacing[1], dy), g.invSpacing[1], qy);
+	rz = __builtin_fma(__builtin_fma(-qz, g.spacing[2], dz), g.invSpacing[2], qz);
+	const double far = __builtin_fmax(__builtin_fmax(__builtin_fabs(dx), __builtin_fabs(dy)), __builtin_fabs(dz));
+	const bool slow = !(far < 0x1p500 && g.fastDiv);
+	if (Fast) {
+		*bad |= slow;
+	} else if (slow) {
+		rx = dx / g.spacing[0];
+		ry = dy / g.spacing[1];
+		rz = dz / g.spacing[2];
+	}
+}
+
 struct FieldGrid {
 	GridDesc g;
 
-	__device__ __forceinline__ V3 eval(const V3 &p) const {
-		if (g.clip) {
-			bool in = (p.x >= g.origin[0]) && (p.x <= g.edge[0]);
-			in &= (p.y >= g.origin[1]) && (p.y <= g.edge[1]);
-			in &= (p.z >= g.origin[2]) && (p.z <= g.edge[2]);
-			if (!in)
-				return v3(0.0, 0.0, 0.0);
-		}
-		double rx = div_cr(p.x - g.gridOrigin[0], g.spacing[0], g.invSpacing[0], g.fastDiv);
-		double ry = div_cr(p.y - g.gridOrigin[1], g.spacing[1], g.invSpacing[1], g.fastDiv);
-		double rz = div_cr(p.z - g.gridOrigin[2], g.spacing[2], g.invSpacing[2], g.fastDiv);
-		int x0, x1, y0, y1, z0, z1;
-		double fx, fy, fz;
-		if (g.reflective) {
-			reflective_clamp(rx, g.nx, x0, x1, fx);
-			reflective_clamp(ry, g.ny, y0, y1, fy);
-			reflective_clamp(rz, g.nz, z0, z1, fz);
-		} else {
-			periodic_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
-			periodic_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
-			periodic_clamp(rz, g.nz, g.invN[2], z0, z1, fz);
-		}
+	// the corners' values in the order of Grid.h:572-579
+	__device__ __forceinline__ V3 sum(int x0, int x1, int y0, int y1, int z0, int z1, double fx, double fy,
+	                                  double fz) const {
 		// weights narrowed to float (Vector3<float>::operator*(float))
 		const float wx0 = (float)fx, wy0 = (float)fy, wz0 = (float)fz;
 		const float wx1 = (float)(1 - fx), wy1 = (float)(1 - fy), wz1 = (float)(1 - fz);
@@ -405,7 +508,6 @@ struct FieldGrid {
 		const size_t bx0 = (size_t)x0 * sx, bx1 = (size_t)x1 * sx;
 		const size_t by0 = (size_t)y0 * sy, by1 = (size_t)y1 * sy;
 		const float *v = g.values;
-		// corner order of Grid.h:572-579
 		const float *c0 = v + 3 * (bx0 + by0 + z0);
 		const float *c1 = v + 3 * (bx1 + by0 + z0);
 		const float *c2 = v + 3 * (bx0 + by1 + z0);
@@ -430,6 +532,45 @@ struct FieldGrid {
 		}
 		return v3((double)b[0], (double)b[1], (double)b[2]);
 	}
+	__device__ __forceinline__ bool outside(const V3 &p) const {
+		if (!g.clip)
+			return false;
+		bool in = (p.x >= g.origin[0]) && (p.x <= g.edge[0]);
+		in &= (p.y >= g.origin[1]) && (p.y <= g.edge[1]);
+		in &= (p.z >= g.origin[2]) && (p.z <= g.edge[2]);
+		return !in;
+	}
+	__device__ __forceinline__ V3 eval(const V3 &p) const {
+		if (outside(p))
+			return v3(0.0, 0.0, 0.0);
+		double rx, ry, rz;
+		grid_position<false>(g, p, rx, ry, rz, nullptr);
+		int x0, x1, y0, y1, z0, z1;
+		double fx, fy, fz;
+		if (g.reflective) {
+			reflective_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
+			reflective_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
+			reflective_clamp(rz, g.nz, g.invN[2], z0, z1, fz);
+		} else {
+			periodic_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
+			periodic_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
+			periodic_clamp(rz, g.nz, g.invN[2], z0, z1, fz);
+		}
+		return sum(x0, x1, y0, y1, z0, z1, fx, fy, fz);
+	}
+	// eval's straight line: the same value wherever it leaves `bad` alone
+	__device__ __forceinline__ V3 eval_fast(const V3 &p, bool &bad) const {
+		double rx, ry, rz, fx, fy, fz;
+		grid_position<true>(g, p, rx, ry, rz, &bad);
+		int x0, x1, y0, y1, z0, z1;
+		const bool refl = g.reflective != 0;
+		clamp_fast(rx, g.nx, g.invN[0], refl, x0, x1, fx, bad);
+		clamp_fast(ry, g.ny, g.invN[1], refl, y0, y1, fy, bad);
+		clamp_fast(rz, g.nz, g.invN[2], refl, z0, z1, fz, bad);
+		const V3 b = sum(x0, x1, y0, y1, z0, z1, fx, fy, fz);
+		return outside(p) ? v3(0.0, 0.0, 0.0) : b;
+	}
+	__device__ __forceinline__ const FieldGrid &lane_field() const { return *this; }
 
 	// mixed precision: reference index arithmetic, FP32 weights and fused sum
 	__device__ __forceinline__ float3 evalf(const V3 &p) const {
@@ -446,9 +587,9 @@ struct FieldGrid {
 		int x0, x1, y0, y1, z0, z1;
 		double fx, fy, fz;
 		if (g.reflective) {
-			reflective_clamp(rx, g.nx, x0, x1, fx);
-			reflective_clamp(ry, g.ny, y0, y1, fy);
-			reflective_clamp(rz, g.nz, z0, z1, fz);
+			reflective_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
+			reflective_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
+			reflective_clamp(rz, g.nz, g.invN[2], z0, z1, fz);
 		} else {
 			periodic_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
 			periodic_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
@@ -487,9 +628,9 @@ __device__ __forceinline__ float scalar_grid_eval(const GridDesc &g, const V3 &p
 	int x0, x1, y0, y1, z0, z1;
 	double fx, fy, fz;
 	if (g.reflective) {
-		reflective_clamp(rx, g.nx, x0, x1, fx);
-		reflective_clamp(ry, g.ny, y0, y1, fy);
-		reflective_clamp(rz, g.nz, z0, z1, fz);
+		reflective_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
+		reflective_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
+		reflective_clamp(rz, g.nz, g.invN[2], z0, z1, fz);
 	} else {
 		periodic_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
 		periodic_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
@@ -526,9 +667,9 @@ __device__ __forceinline__ float scalar_grid_evalf(const GridDesc &g, const V3 &
 	int x0, x1, y0, y1, z0, z1;
 	double fx, fy, fz;
 	if (g.reflective) {
-		reflective_clamp(rx, g.nx, x0, x1, fx);
-		reflective_clamp(ry, g.ny, y0, y1, fy);
-		reflective_clamp(rz, g.nz, z0, z1, fz);
+		reflective_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
+		reflective_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
+		reflective_clamp(rz, g.nz, g.invN[2], z0, z1, fz);
 	} else {
 		periodic_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
 		periodic_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
@@ -568,11 +709,12 @@ struct FieldGridCells {
 		in &= (p.z >= g.origin[2]) && (p.z <= g.edge[2]);
 		return !in;
 	}
-	// the cell of a position and the position within it
-	__device__ __forceinline__ size_t cell(const V3 &p, double &fx, double &fy, double &fz) const {
-		double rx = div_cr(p.x - g.gridOrigin[0], g.spacing[0], g.invSpacing[0], g.fastDiv);
-		double ry = div_cr(p.y - g.gridOrigin[1], g.spacing[1], g.invSpacing[1], g.fastDiv);
-		double rz = div_cr(p.z - g.gridOrigin[2], g.spacing[2], g.invSpacing[2], g.fastDiv);
+	// the cell of a position and the position within it; Fast: without the divisions' range tests, `bad` is
+	// set where they are needed
+	template <bool Fast = false>
+	__device__ __forceinline__ size_t cell(const V3 &p, double &fx, double &fy, double &fz, bool *bad = nullptr) const {
+		double rx, ry, rz;
+		grid_position<Fast>(g, p, rx, ry, rz, bad);
 		int x0, x1, y0, y1, z0, z1;
 		periodic_clamp(rx, g.nx, g.invN[0], x0, x1, fx);
 		periodic_clamp(ry, g.ny, g.invN[1], y0, y1, fy);
@@ -624,6 +766,14 @@ struct FieldGridCells {
 		const size_t c = cell(p, fx, fy, fz);
 		return sum(reinterpret_cast<const float4 *>(cells + kCellFloats * c), fx, fy, fz);
 	}
+	// eval's straight line: the same value wherever it leaves `bad` alone
+	__device__ __forceinline__ V3 eval_fast(const V3 &p, bool &bad) const {
+		double fx, fy, fz;
+		const size_t c = cell<true>(p, fx, fy, fz, &bad);
+		const V3 b = sum(reinterpret_cast<const float4 *>(cells + kCellFloats * c), fx, fy, fz);
+		return outside(p) ? v3(0.0, 0.0, 0.0) : b;
+	}
+	__device__ __forceinline__ const FieldGridCells &lane_field() const { return *this; }
 	__device__ __forceinline__ float3 evalf(const V3 &p) const {
 		if (outside(p))
 			return make_float3(0.f, 0.f, 0.f);
@@ -806,21 +956,21 @@ struct FieldPlaneWaveLds : FieldPlaneWave {
 };
 
 // The field a propagation kernel evaluates for its argument: `make` is called once by every thread of
-// the workgroup; `lds` are kLdsPerWave bytes of dynamic LDS for each of its waves.  The FP64 plane waves
-// copy the cosine's 12 KB table to LDS: 64 lanes read 64 entries of it per mode, which as global loads
-// would be up to 128 line requests per mode and wave.  The mode loop is bound by FP64 issue: 65 vector
-// instructions a mode with this table against about 230 with the octant table and its selection; 2^18
-// particles x 300 steps x 256 modes in 52.7 ms against 147.5.
+// the workgroup; `lds` are lds_bytes() of dynamic LDS.  The FP64 plane waves copy the cosine's 12 KB table
+// to LDS: 64 lanes read 64 entries of it per mode, which as global loads would be up to 128 line requests per
+// mode and wave.  The mode loop is bound by FP64 issue: 65 vector instructions a mode with this table against
+// about 230 with the octant table and its selection; 2^18 particles x 300 steps x 256 modes in 52.7 ms
+// against 147.5.
 template <class F, bool MIX> struct KernelField {
 	typedef F type;
-	static constexpr int kLdsPerWave = 0;
+	static size_t lds_bytes(const F &, int) { return 0; }
 	static __device__ __forceinline__ type make(const F &f, char *) { return f; }
 };
 template <> struct KernelField<FieldPlaneWave, false> {
 	typedef FieldPlaneWaveLds type;
-	static constexpr int kLdsPerWave = 0;
-	static __device__ __forceinline__ type make(const FieldPlaneWave &f, char *) {
-		__shared__ double tab[2 * CRP_TURN_ENTRIES];
+	static size_t lds_bytes(const FieldPlaneWave &, int) { return 2 * CRP_TURN_ENTRIES * sizeof(double); }
+	static __device__ __forceinline__ type make(const FieldPlaneWave &f, char *lds) {
+		double *const tab = reinterpret_cast<double *>(lds);
 		for (int i = threadIdx.x; i < 2 * CRP_TURN_ENTRIES; i += blockDim.x)
 			tab[i] = crp_turn_tab[i];
 		__syncthreads();
@@ -830,7 +980,6 @@ template <> struct KernelField<FieldPlaneWave, false> {
 		return r;
 	}
 };
-
 // FieldGridCells whose cell lines are gathered by the wave together.  A lane that reads its own line does
 // it in six 16-byte loads, and each of them translates an address for every lane: once the table outgrows
 // the reach of the first-level translation cache (about 3 GB) all six miss, and random lines come at
@@ -865,10 +1014,10 @@ struct FieldGridCellsWave : FieldGridCells {
 			q[i] = *reinterpret_cast<const float4 *>(r + ((i ^ p) << 4));
 		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // and read before the next gather overwrites them
 	}
-	__device__ __forceinline__ V3 eval(const V3 &p) const {
+	__device__ __forceinline__ V3 eval_fast(const V3 &p, bool &bad) const {
 		double fx, fy, fz;
 		float4 q[6];
-		gather(cell(p, fx, fy, fz), q);
+		gather(cell<true>(p, fx, fy, fz, &bad), q);
 		const V3 b = sum(q, fx, fy, fz);
 		return outside(p) ? v3(0.0, 0.0, 0.0) : b;
 	}
@@ -887,11 +1036,11 @@ template <> struct WaveField<FieldGridCellsWave> {
 struct FieldGridCellsBig : FieldGridCells {};
 template <bool MIX> struct KernelField<FieldGridCellsBig, MIX> {
 	typedef FieldGridCellsWave type;
-	static constexpr int kLdsPerWave = FieldGridCellsWave::kLdsPerWave;
+	static size_t lds_bytes(const FieldGridCellsBig &, int block) { return (size_t)type::kLdsPerWave * (block / 64); }
 	static __device__ __forceinline__ type make(const FieldGridCellsBig &f, char *lds) {
 		type r;
 		static_cast<FieldGridCells &>(r) = f;
-		r.lds = lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kLdsPerWave;
+		r.lds = lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * type::kLdsPerWave;
 		return r;
 	}
 };
@@ -1044,9 +1193,84 @@ struct Y {
 	V3 x, u;
 };
 
-// PropagationBP::dY (src/module/PropagationBP.cpp:19-39)
+// Fields with eval_fast, whose values are FP32 numbers widened: their FP64 steps run without range tests and
+// are repeated with them where one would have failed
+template <class F> struct FastField {
+	static constexpr bool value = false;
+};
+template <> struct FastField<FieldGridCells> {
+	static constexpr bool value = true;
+};
+template <> struct FastField<FieldGrid> {
+	static constexpr bool value = true;
+};
+template <> struct FastField<FieldGridCellsWave> {
+	static constexpr bool value = true;
+};
+
+// Whether bp_dy_fast's quotients stay where div_fast is exact: nonzero field components are within
+// [2^-149, 2^128], so with these bounds B q/2 / m * step / c is 0 or within [2^-399, 2^390]
+__device__ __forceinline__ bool bp_in_range(double q, double m, double step) {
+	const double aq = __builtin_fabs(q);
+	return aq > 0x1p-100 && aq < 0x1p20 && m > 0x1p-150 && m < 0x1p60 && step > 0x1p-60 && step < 0x1p120;
+}
+
+// bp_dy below in one straight line; `bad` is set where its result may differ
 template <class F>
+__device__ __forceinline__ Y bp_dy_fast(const F &field, const V3 &pos0, const V3 &dir, double step, double q, double m,
+                                        double invm, bool &bad) {
+	V3 pos = v3(pos0.x + (dir.x * step) / 2., pos0.y + (dir.y * step) / 2., pos0.z + (dir.z * step) / 2.);
+	V3 B = field.eval_fast(pos, bad);
+	V3 t = v3(div_fast(div_fast((B.x * q) / 2, m, invm) * step, kCLight, kInvCLight),
+	          div_fast(div_fast((B.y * q) / 2, m, invm) * step, kCLight, kInvCLight),
+	          div_fast(div_fast((B.z * q) / 2, m, invm) * step, kCLight, kInvCLight));
+	double tt = (t.x * t.x + t.y * t.y) + t.z * t.z;
+	double den = 1 + tt;
+	bad |= !(den < 0x1p100); // NaN and infinities too
+	const double invden = rcp_rn(den);
+	V3 s = v3(div_fast(t.x * 2, den, invden), div_fast(t.y * 2, den, invden), div_fast(t.z * 2, den, invden));
+	V3 vh = v3(dir.x + (dir.y * t.z - t.y * dir.z), dir.y + (dir.z * t.x - t.z * dir.x),
+	           dir.z + (dir.x * t.y - t.x * dir.y));
+	V3 d = v3(dir.x + (vh.y * s.z - s.y * vh.z), dir.y + (vh.z * s.x - s.z * vh.x),
+	          dir.z + (vh.x * s.y - s.x * vh.y));
+	Y out;
+	out.x = v3(pos.x + (d.x * step) / 2., pos.y + (d.y * step) / 2., pos.z + (d.z * step) / 2.);
+	out.u = d;
+	return out;
+}
+
+// u / |u| twice, as setDirection(getUnitVector()) does
+__device__ __forceinline__ V3 unit_twice_tested(const V3 &u) {
+	const double n1 = norm(u), i1 = 1 / n1;
+	const V3 u1 = v3(div_rn(u.x, n1, i1), div_rn(u.y, n1, i1), div_rn(u.z, n1, i1));
+	const double n2 = norm(u1), i2 = 1 / n2;
+	return v3(div_rn(u1.x, n2, i2), div_rn(u1.y, n2, i2), div_rn(u1.z, n2, i2));
+}
+// in one straight line; `bad` is set where it may differ.  Rotated: |u| is 1 to a few ulps, as a Boris rotation
+// leaves it.  Components of u of magnitude 2^-400 and more, or 0, keep both divisions in range.
+template <bool Rotated> __device__ __forceinline__ V3 unit_twice_fast(const V3 &u, bool &bad) {
+	const double d1 = (u.x * u.x + u.y * u.y) + u.z * u.z;
+	const double n1 = Rotated ? sqrt_near_one(d1, bad) : __builtin_sqrt(d1);
+	const double i1 = Rotated ? rcp_near_one(n1, bad) : rcp_rn(n1);
+	const V3 u1 = v3(div_fast(u.x, n1, i1), div_fast(u.y, n1, i1), div_fast(u.z, n1, i1));
+	const double n2 = sqrt_near_one((u1.x * u1.x + u1.y * u1.y) + u1.z * u1.z, bad);
+	const double i2 = rcp_near_one(n2, bad); // 1 to an ulp or two
+	if (!Rotated)
+		bad |= !(n1 > 0x1p-80 && n1 < 0x1p80);
+	bad |= min(min(__builtin_amdgcn_frexp_exp(u.x), __builtin_amdgcn_frexp_exp(u.y)), __builtin_amdgcn_frexp_exp(u.z)) < -400;
+	return v3(div_fast(u1.x, n2, i2), div_fast(u1.y, n2, i2), div_fast(u1.z, n2, i2));
+}
+__device__ __forceinline__ V3 unit_twice(const V3 &u) {
+	bool bad = false;
+	V3 d = unit_twice_fast<false>(u, bad);
+	if (bad)
+		d = unit_twice_tested(u);
+	return d;
+}
+
+// PropagationBP::dY (src/module/PropagationBP.cpp:19-39)
 // (divisions as div_rn with shared reciprocals: invm = RN(1/m) from the caller)
+template <class F>
 __device__ __forceinline__ Y bp_dy(const F &field, const V3 &pos0, const V3 &dir, double step, double q, double m,
                                   double invm) {
 	V3 pos = v3(pos0.x + (dir.x * step) / 2., pos0.y + (dir.y * step) / 2., pos0.z + (dir.z * step) / 2.);
@@ -1074,9 +1298,8 @@ template <class F>
 __device__ __forceinline__ Y ck_dydt(const F &field, const Y &y, double qcE,
                                      CkB0Store<FloatValuedField<F>::value> *b0 = nullptr) {
 	Y d;
-	double n = norm(y.u);
-	const double invn = 1 / n;
-	d.x = v3(div_rn(y.u.x, n, invn) * kCLight, div_rn(y.u.y, n, invn) * kCLight, div_rn(y.u.z, n, invn) * kCLight);
+	const V3 v = unit_rn(y.u);
+	d.x = v3(v.x * kCLight, v.y * kCLight, v.z * kCLight);
 	V3 B;
 	if (WaveField<F>::value && b0) { // the whole wave evaluates while any lane needs it
 		if (__ballot(!b0->have)) {

@@ -143,6 +143,7 @@ struct crp_batch {
 };
 
 
+
 static Soa soa_of(const crp_batch *b) {
 	Soa s;
 	s.px = b->px; s.py = b->py; s.pz = b->pz;
@@ -404,7 +405,7 @@ static auto propagate_kernel() {
 }
 
 template <class F, int KIND, bool MIX>
-static int launch_propagate(const F &f, const crp_propagator *p, const Params &P0, crp_batch *b, int *launches) {
+static int launch_propagate(const F &f, const crp_propagator *p, const Params &Pin, crp_batch *b, int *launches) {
 	auto kern = propagate_kernel<F, KIND, MIX>();
 	const int ncu = num_cus();
 	if (ncu < 0)
@@ -413,16 +414,24 @@ static int launch_propagate(const F &f, const crp_propagator *p, const Params &P
 	int bpcMax = 0;
 	size_t lds = (size_t)kColdDoubles * block * sizeof(double);
 	if (KIND != PK_SDE)
-		lds += (size_t)KernelField<F, MIX>::kLdsPerWave * (block / 64);
+		lds += KernelField<F, MIX>::lds_bytes(f, block);
 	CRP_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&bpcMax, kern, block, lds));
 	if (bpcMax < 1)
 		bpcMax = 1;
 	const int bpc = p->blocksPerCU > 0 ? std::min(p->blocksPerCU, bpcMax) : bpcMax;
-	const size_t want = (b->n + block - 1) / block;
+	// A batch of fewer particles than the chip's SIMDs have lanes is spread over all of them, a wave taking
+	// `lanes` particles: every particle is one serial chain, and a wave with fewer of them waits for fewer
+	// lines per load and fewer rare branches.
+	const size_t waves = std::min<size_t>((size_t)ncu * bpc * (block / 64), (size_t)ncu * 4);
+	const int lanes = (int)std::min<size_t>(64, std::max<size_t>(1, (b->n + waves - 1) / waves));
+	const size_t perBlock = (size_t)lanes * (block / 64);
+	const size_t want = (b->n + perBlock - 1) / perBlock;
 	const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(want, (size_t)ncu * bpc));
 	p->lastGrid = grid;
 	p->lastBlock = (unsigned)block;
 	p->lastPPL = (double)b->n / ((double)grid * block);
+	Params P0 = Pin;
+	P0.lanes = lanes;
 	const Soa soa = soa_of(b);
 	const unsigned long long n = b->n;
 	const long long M = P0.maxSteps, S = p->stepsPerLaunch;
@@ -633,7 +642,7 @@ static int fill_grid_desc(GridDesc &g, const float *d_values, int nx, int ny, in
 	}
 	g.fastDiv = 1;
 	for (int a = 0; a < 3; a++)
-		g.fastDiv &= (spacing[a] >= 0x1p-500 && spacing[a] <= 0x1p500) ? 1 : 0;
+		g.fastDiv &= (spacing[a] >= 0x1p-300 && spacing[a] <= 0x1p300) ? 1 : 0;
 	return CRP_OK;
 }
 

@@ -75,6 +75,8 @@ struct Params {
 	const SdeAdvTerm *sdeAdvTerms;
 	int sdeAdvection;
 	uint32_t sdeSeed;
+	// lanes of a wave that take particles (launch_propagate)
+	int lanes;
 	int sdeMaxHalvings; // trials beyond this many halvings stop the particle (CTR_SDE_LIMIT)
 };
 
@@ -92,41 +94,48 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 // r^-0.2 of the step-size update (used as (step * 0.95) * r^-0.2, the
 // reference's order): correctly rounded on the FP64 path (the reference calls
 // glibc pow), the device libm on the mixed path
+// (tab: crp_logr_tab and crp_exp2_tab in LDS)
+constexpr int kPowTab = 3 * 256 + 2 * 256;
 template <bool MIX>
-__device__ __forceinline__ double pow_m02(double r) {
+__device__ __forceinline__ double pow_m02(double r, const double *tab) {
 	if (MIX)
 		return ::pow(r, -0.2);
-	return crp_pow_cr(r, -0.2);
+	return crp_pow_cr_quick(r, -0.2, tab, tab + 3 * 256);
 }
 
-// Register budget: the FP64 path through the cell table is asked for 3 waves per SIMD (<= 168
-// VGPRs; it needs 169 unconstrained and then runs at 2), gathered by waves on the mixed path for 2 (it
-// needs 257); everything else is left to the compiler.
-template <class F>
-struct WavesHint {
-	static constexpr int fp64 = 1, mixed = 1;
+// Register budget, in waves per SIMD asked of the compiler.  FP64 through the cell table: Cash-Karp 3 (it
+// fits 168 VGPRs and runs at 2 without the hint), adaptive Boris 2 (191; at 3 its two overlapping steps
+// spill).  Gathered by waves on the mixed path 2 (257 unconstrained).
+template <class F, int KIND, bool MIX> struct WavesHint {
+	static constexpr int value = 1;
 };
-template <>
-struct WavesHint<FieldGridCells> {
-	static constexpr int fp64 = 3, mixed = 1;
+template <int KIND> struct WavesHint<FieldGridCells, KIND, false> {
+	static constexpr int value = KIND == PK_BP_ADAPTIVE ? 2 : 3;
 };
-template <>
-struct WavesHint<FieldGridCellsBig> {
-	static constexpr int fp64 = 1, mixed = 2;
+template <int KIND> struct WavesHint<FieldGridCellsBig, KIND, true> {
+	static constexpr int value = 2;
 };
 
+// the field a lane evaluates by itself
+template <class F> __device__ __forceinline__ auto &&lane_field(const F &f) {
+	if constexpr (FastField<F>::value)
+		return f.lane_field();
+	else
+		return f;
+}
+
 template <class F, int KIND, bool MIX>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MIX ? WavesHint<F>::mixed : WavesHint<F>::fp64, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WavesHint<F, KIND, MIX>::value, 8)))
 k_propagate(F field0, Params P, Soa S, unsigned long long n,
                                                    unsigned long long *__restrict__ ctr) {
 	constexpr bool kCK = (KIND == PK_CK_FIXED || KIND == PK_CK_ADAPTIVE);
 	constexpr bool kAdaptive = (KIND == PK_BP_ADAPTIVE || KIND == PK_CK_ADAPTIVE);
 	constexpr unsigned long long kEvalsPerTrial = kCK ? 6 : (kAdaptive ? 3 : 1);
 	// fields whose evaluation is one computation of the whole wave: every lane takes part, busy or not
+	constexpr bool kFast = FastField<typename KernelField<F, MIX>::type>::value;
 	constexpr bool kWave = WaveField<typename KernelField<F, MIX>::type>::value;
 	const int lane = __lane_id();
-
-	bool have = false, exhausted = false, inProc = false;
+	bool have = false, exhausted = lane >= P.lanes, inProc = false;
 	CkB0Store<FloatValuedField<typename KernelField<F, MIX>::type>::value> b0; // the field at the trial sequence's start (adaptive CK), for retries
 	CkB0f b0f;
 	b0.have = false;
@@ -136,6 +145,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 	V3 pos = v3(0, 0, 0), dir = v3(0, 0, 0);
 	float3 dirf = make_float3(0.f, 0.f, 0.f);
 	double E = 0, q = 0, next = 0;
+	double m_ = 0, im_ = 0; // FP64 Boris: the particle's relativistic mass E/c^2 and RN(1/m)
 	double step = 0, newStep = 0;
 	// per-lane counters, flushed to ctr[] before they could wrap
 	unsigned nAcc = 0, nRej = 0, nEval = 0, nFin = 0, nPause = 0;
@@ -152,6 +162,14 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 	// the lane's copy: a field that reads the candidate's redshift binds it at refill
 	typename KernelField<F, MIX>::type field =
 	    KernelField<F, MIX>::make(field0, (char *)(crp_cold + kColdDoubles * blockDim.x));
+
+	// the tables of the step control's power: read from LDS, since every adaptive trial waits for them
+	__shared__ double powTab[kAdaptive && !MIX ? kPowTab : 1];
+	if (kAdaptive && !MIX) {
+		for (int i = threadIdx.x; i < kPowTab; i += blockDim.x)
+			powTab[i] = i < 3 * 256 ? crp_logr_tab[i] : crp_exp2_tab[i - 3 * 256];
+		__syncthreads();
+	}
 
 	for (;;) {
 		if (nEval > 0x80000000u) { // flush this lane's counters long before they wrap
@@ -181,6 +199,10 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 							dirf = make_float3((float)dir.x, (float)dir.y, (float)dir.z);
 						E = S.E[idx];
 						q = S.q[idx];
+						if (!kCK && !MIX) {
+							m_ = E / (kCLight * kCLight);
+							im_ = 1 / m_;
+						}
 						if (UsesRedshift<F>::value)
 							bind_redshift(field, S.z[idx]);
 						*cCur = S.cur[idx];
@@ -209,6 +231,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 		bool commit = false;
 		bool neutral = false;
 		Y yOut;          // FP64 path result
+		V3 nDir;         // FP64 Boris: its direction normalised, formed beside the error and the step control
 		V3 oPos;         // mixed path result
 		float3 oDir;
 		// rectilinear propagation for neutral particles (PropagationBP.cpp:74-80)
@@ -237,8 +260,17 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 					double eU;
 					ck_trystep(field, Y{pos, dir}, step / kCLight, (q * kCLight) / E, yOut, eU);
 				} else {
-					const double m_ = E / (kCLight * kCLight);
-					yOut = bp_dy(field, pos, dir, step, q, m_, 1 / m_);
+					if constexpr (kFast) {
+						bool bad = !bp_in_range(q, m_, step);
+						yOut = bp_dy_fast(field, pos, dir, step, q, m_, im_, bad);
+						nDir = unit_twice_fast<true>(yOut.u, bad);
+						if (bad) {
+							yOut = bp_dy(field.lane_field(), pos, dir, step, q, m_, im_);
+							nDir = unit_twice_tested(yOut.u);
+						}
+					} else {
+						yOut = bp_dy(field, pos, dir, step, q, m_, im_);
+					}
 				}
 			}
 		};
@@ -270,11 +302,23 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 				ck_trystep(field, Y{pos, dir}, step / kCLight, (q * kCLight) / E, yOut, eU, &b0);
 				return eU / P.tol;
 			}
-			const double m_ = E / (kCLight * kCLight);
-			const double im_ = 1 / m_;
-			yOut = bp_dy(field, pos, dir, step, q, m_, im_);
-			Y half = bp_dy(field, pos, dir, step / 2, q, m_, im_);
-			Y cmp = bp_dy(field, half.x, half.u, step / 2, q, m_, im_);
+			Y cmp;
+			bool bad = true;
+			if constexpr (kFast) {
+				bad = !(bp_in_range(q, m_, step) && bp_in_range(q, m_, step / 2));
+				yOut = bp_dy_fast(field, pos, dir, step, q, m_, im_, bad);
+				const Y half = bp_dy_fast(field, pos, dir, step / 2, q, m_, im_, bad);
+				cmp = bp_dy_fast(field, half.x, half.u, step / 2, q, m_, im_, bad);
+				nDir = unit_twice_fast<true>(yOut.u, bad);
+			}
+			if (!kFast || bad) {
+				auto &&f = lane_field(field);
+				yOut = bp_dy(f, pos, dir, step, q, m_, im_);
+				const Y half = bp_dy(f, pos, dir, step / 2, q, m_, im_);
+				cmp = bp_dy(f, half.x, half.u, step / 2, q, m_, im_);
+				if (kFast)
+					nDir = unit_twice_tested(yOut.u);
+			}
 			V3 d = v3(yOut.x.x - cmp.x.x, yOut.x.y - cmp.x.y, yOut.x.z - cmp.x.z);
 			double Sv = norm(d) / (step * (1 - 1 / 4.));
 			return __builtin_sqrt((Sv * Sv + Sv * Sv) + Sv * Sv) / P.tol;
@@ -287,14 +331,14 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 					commit = true;
 				} else {
 					nRej++;
-					newStep = step * 0.95 * pow_m02<MIX>(r);
+					newStep = step * 0.95 * pow_m02<MIX>(r, powTab);
 					newStep = dmax(newStep, 0.1 * step);
 					newStep = dmax(newStep, P.minStep);
 					step = newStep;
 				}
 			} else {
 				if (step != P.maxStep) {
-					newStep = step * 0.95 * pow_m02<MIX>(r);
+					newStep = step * 0.95 * pow_m02<MIX>(r, powTab);
 					newStep = dmin(newStep, 5 * step);
 					newStep = dmin(newStep, P.maxStep);
 				}
@@ -356,10 +400,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 		} else {
 			pos = yOut.x;
 			if (!neutral) {
-				const double n1 = norm(yOut.u), i1 = 1 / n1;
-				V3 u1 = v3(div_rn(yOut.u.x, n1, i1), div_rn(yOut.u.y, n1, i1), div_rn(yOut.u.z, n1, i1));
-				const double n2 = norm(u1), i2 = 1 / n2;
-				dir = v3(div_rn(u1.x, n2, i2), div_rn(u1.y, n2, i2), div_rn(u1.z, n2, i2));
+				dir = (kFast && !kCK) ? nDir : unit_twice(yOut.u);
 			}
 		}
 		if (P.box) {

@@ -38,13 +38,12 @@ constexpr int kSdeMaxHalvings = 20;
 
 // B / |B| * c_light (Vector3::getUnitVector, then the product)
 __device__ __forceinline__ V3 sde_unit_c(const V3 &b) {
-	const double r = norm(b), ir = 1 / r;
-	return v3(div_rn(b.x, r, ir) * kCLight, div_rn(b.y, r, ir) * kCLight, div_rn(b.z, r, ir) * kCLight);
+	const V3 u = unit_rn(b);
+	return v3(u.x * kCLight, u.y * kCLight, u.z * kCLight);
 }
 
 __device__ __forceinline__ V3 sde_unit(const V3 &b) {
-	const double r = norm(b), ir = 1 / r;
-	return v3(div_rn(b.x, r, ir), div_rn(b.y, r, ir), div_rn(b.z, r, ir));
+	return unit_rn(b);
 }
 
 // Vector3::cross (include/crpropa/Vector3.h:268-271)
@@ -57,16 +56,19 @@ __device__ __forceinline__ V3 sde_cross(const V3 &a, const V3 &b) {
 template <class F>
 __device__ __forceinline__ void sde_trystep(const F &field, const V3 &x, const V3 &k0, double t, V3 &out, V3 &err) {
 	const double e0 = CK::b0 - CK::s0, e1 = CK::b1 - CK::s1, e2 = CK::b2 - CK::s2, e3 = CK::b3 - CK::s3,
-	             e4 = CK::b4 - CK::s4, e5 = CK::b5 - CK::s5;
+	             e4 = CK::b4 - CK::s4, e5 = CK::b5 - CK::s5; // constants: the test of e folds
 	out = x;
 	err = v3(0.0, 0.0, 0.0);
 	auto acc = [&](const V3 &k, double b, double e) {
 		out.x += (k.x * b) * t;
 		out.y += (k.y * b) * t;
 		out.z += (k.z * b) * t;
-		err.x += div_rn((k.x * e) * t, kKpc, kInvKpc);
-		err.y += div_rn((k.y * e) * t, kKpc, kInvKpc);
-		err.z += div_rn((k.z * e) * t, kKpc, kInvKpc);
+		if (e != 0) { // e1 = 0: err is never -0, so adding 0 leaves it as it is (a NaN stage reaches the next ones)
+			const V3 d = div3_rn(v3((k.x * e) * t, (k.y * e) * t, (k.z * e) * t), kKpc, kInvKpc);
+			err.x += d.x;
+			err.y += d.y;
+			err.z += d.z;
+		}
 	};
 	// y_n = x + sum_j (k_j a_ij) t, in the reference's order
 	auto ax = [&](V3 &y, const V3 &k, double a) {
@@ -154,7 +156,7 @@ __device__ __forceinline__ V3 sde_randcone(crp_sde_rng &r, const V3 &mean, doubl
 // functions of the shock profiles stay out of the transport loop's registers.
 typedef __attribute__((address_space(4))) const SdeAdvTerm SdeAdvTermConst;
 
-__device__ __forceinline__ V3 sde_advection_velocity(const SdeAdvTerm *terms, int n, const V3 pos) {
+__device__ __attribute__((noinline)) V3 sde_advection_velocity(const SdeAdvTerm *terms, int n, const V3 pos) {
 	SdeAdvTermConst *T = (SdeAdvTermConst *)terms;
 	double vx = 0, vy = 0, vz = 0;
 	for (int t = 0; t < n; t++) {
@@ -247,7 +249,7 @@ __global__ void __launch_bounds__(256) k_sde(F field0, Params P, Soa S, unsigned
 	const double cosHalfPi = crp_cos_cr(3.14159265358979323846 / 2.);
 	const double minTime = P.minStep / kCLight; // minStep / c_light of the trial loop's test
 
-	bool have = false, exhausted = false;
+	bool have = false, exhausted = lane >= P.lanes;
 	unsigned idx = 0;
 	long long steps = 0;
 	int phase = SDE_BEGIN;
@@ -307,7 +309,7 @@ __global__ void __launch_bounds__(256) k_sde(F field0, Params P, Soa S, unsigned
 							// calculateBTensor (src/module/DiffusionSDE.cpp:258-266): constant per particle;
 							// pow(x, 0.5) correctly rounded is sqrt(x)
 							const double rig = S.E[idx] / q;
-							const double D = P.sdeScale * 6.1e24 * crp_pow_cr(__builtin_fabs(rig) / 4.0e9, P.sdeAlpha);
+							const double D = P.sdeScale * 6.1e24 * crp_pow_cr_cold(__builtin_fabs(rig) / 4.0e9, P.sdeAlpha);
 							B0 = __builtin_sqrt(2 * D);
 							B4 = __builtin_sqrt(2 * P.sdeEpsilon * D);
 						}

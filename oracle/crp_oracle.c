@@ -1406,6 +1406,13 @@ void orc_cos_turn_phases(const double *x, size_t n, int sine, double *quick, int
 	}
 }
 
+void orc_pow_phases(const double *x, double y, size_t n, double *quick, int32_t *decided, double *accurate) {
+	for (size_t i = 0; i < n; i++) {
+		decided[i] = crp_pow_quick(x[i], y, crp_logr_tab, crp_exp2_tab, &quick[i]);
+		accurate[i] = crp_pow_cr(x[i], y);
+	}
+}
+
 void orc_philox4x32_10(const uint32_t ctr[4], const uint32_t key[2], uint32_t out[4]) {
 	crp_philox_ctr c;
 	for (int i = 0; i < 4; i++)

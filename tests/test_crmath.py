@@ -103,6 +103,20 @@ def test_cos_turn_phase_agrees_with_accurate_phase(sine):
     assert not dec[4:].any()
 
 
+@pytest.mark.parametrize("y", [-0.2, 1 / 3., -1.0, 0.9])
+def test_pow_quick_phase_agrees_with_double_double(y):
+    """Every value that the quick phase decides equals the double-double one (7e7 arguments checked the same way
+    during development); zero, subnormal, negative, infinite and NaN arguments are left to it."""
+    rng = np.random.default_rng(29)
+    n = 200000
+    x = np.concatenate([np.exp(rng.uniform(-10, 10, n)), np.exp(rng.uniform(-600, 600, n)), 1 + rng.uniform(-1e-3, 1e-3, n),
+                        np.ldexp(1 + np.arange(4096) / 4096., rng.integers(-40, 40, 4096)), np.array([1.0, 2.0, 0.5])])
+    q, dec, a = O.pow_phases(x, y)
+    assert dec.mean() > 0.99
+    assert np.array_equal(q[dec].view(np.uint64), a[dec].view(np.uint64))
+    assert not O.pow_phases(np.array([0.0, -0.0, 5e-324, 1e-310, -1.0, np.inf, -np.inf, np.nan]), y)[1].any()
+
+
 def test_philox_known_answers():
     """Philox4x32-10 known-answer vectors (Salmon et al., SC'11, the Random123 distribution)."""
     assert O.philox4x32_10([0, 0, 0, 0], [0, 0]) == [0x6627e8d5, 0xe169c58d, 0xbc57ac4c, 0x9b00dbd8]

@@ -171,6 +171,7 @@ struct PlaneWaveDesc {
 	int nm;
 	const PwMode64 *m64;   // [nm]
 	const PwModeMixed *mm; // [nm]
+	double reach;          // mixed path: |x| + |y| + |z| below which every phase is below 2^18 turns
 };
 
 struct FieldUniform {
@@ -955,6 +956,35 @@ struct FieldPlaneWaveLds : FieldPlaneWave {
 	__device__ __forceinline__ V3 eval(const V3 &p) const { return sum(p, tab); }
 };
 
+// The mixed path's mode loop in a propagation kernel.  A vector instruction reads one scalar pair, so the
+// phase's start value (the bias) comes from LDS, read by all lanes at once, instead of two moves a mode; it
+// carries 1.5 x 2^20, after which the low word of the phase is its fraction in units of 2^-32 turns, rounded
+// there (2^-33 turns; FP32 fractions have 2^-25), and a conversion and a product replace the FP64 fraction
+// and its narrowing.  Positions whose phases leave 2^18 turns take FieldPlaneWave's loop.  Bound by vector
+// issue: 46.6 cycles a mode and wave against 58.6.
+struct FieldPlaneWaveMix : FieldPlaneWave {
+	static constexpr int kModesMax = 2048; // 16 KB of LDS
+	static constexpr double kBias = 1.5 * 1048576.0;
+	const double *bias; // bt + kBias in LDS
+
+	__device__ __forceinline__ float3 evalf(const V3 &p) const {
+		if (!(__builtin_fabs(p.x) + __builtin_fabs(p.y) + __builtin_fabs(p.z) < w.reach))
+			return FieldPlaneWave::evalf(p);
+		float bx = 0.f, by = 0.f, bz = 0.f;
+		PwModeMixedConst *m = (PwModeMixedConst *)w.mm;
+		const int nm = w.nm;
+#pragma unroll 8
+		for (int i = 0; i < nm; i++) {
+			const double t = __builtin_fma(p.z, m[i].ktz, __builtin_fma(p.y, m[i].kty, __builtin_fma(p.x, m[i].ktx, bias[i])));
+			const float c = __builtin_amdgcn_cosf((float)__double2loint(t) * 0x1p-32f);
+			bx = __builtin_fmaf(m[i].ax, c, bx);
+			by = __builtin_fmaf(m[i].ay, c, by);
+			bz = __builtin_fmaf(m[i].az, c, bz);
+		}
+		return make_float3(bx, by, bz);
+	}
+};
+
 // The field a propagation kernel evaluates for its argument: `make` is called once by every thread of
 // the workgroup; `lds` are lds_bytes() of dynamic LDS.  The FP64 plane waves copy the cosine's 12 KB table
 // to LDS: 64 lanes read 64 entries of it per mode, which as global loads would be up to 128 line requests per
@@ -980,6 +1010,27 @@ template <> struct KernelField<FieldPlaneWave, false> {
 		return r;
 	}
 };
+template <> struct KernelField<FieldPlaneWave, true> {
+	typedef FieldPlaneWaveMix type;
+	static size_t lds_bytes(const FieldPlaneWave &f, int) {
+		return f.w.nm <= type::kModesMax ? f.w.nm * sizeof(double) : 0;
+	}
+	static __device__ __forceinline__ type make(const FieldPlaneWave &f, char *lds) {
+		double *const bias = reinterpret_cast<double *>(lds);
+		type r;
+		r.w = f.w;
+		r.bias = bias;
+		if (f.w.nm > type::kModesMax) {
+			r.w.reach = 0;
+			return r;
+		}
+		for (int i = threadIdx.x; i < f.w.nm; i += blockDim.x)
+			bias[i] = f.w.mm[i].bt + type::kBias;
+		__syncthreads();
+		return r;
+	}
+};
+
 // FieldGridCells whose cell lines are gathered by the wave together.  A lane that reads its own line does
 // it in six 16-byte loads, and each of them translates an address for every lane: once the table outgrows
 // the reach of the first-level translation cache (about 3 GB) all six miss, and random lines come at

@@ -1380,6 +1380,10 @@ int crp_field_create_planewave(int nm, const double *k, const double *Ak, const 
 		}
 		f->owned[j] = d;
 	}
+	double most = 0; // the largest phase gradient; a phase of 2^18 turns holds the bias too
+	for (int i = 0; i < nm; i++)
+		most = std::max({most, std::fabs(mm[i].ktx), std::fabs(mm[i].kty), std::fabs(mm[i].ktz), std::fabs(mm[i].bt) > 0x1p17 ? HUGE_VAL : 0.0});
+	f->pw.reach = most > 0 && most < HUGE_VAL ? 0x1p17 / most : 0.0;
 	f->pw.nm = nm;
 	f->pw.m64 = (const PwMode64 *)f->owned[0];
 	f->pw.mm = (const PwModeMixed *)f->owned[1];

@@ -905,6 +905,184 @@ struct FieldGridAny {
 	}
 };
 
+// Fields of which a group of lanes evaluates one position together: the lanes of a group (aligned, this
+// many) hold the same particle
+template <class F> struct LaneGroup {
+	static constexpr int value = 1;
+};
+
+// the value of lane K of the quad
+template <int K> __device__ __forceinline__ int quad_lane(int v) {
+	return __builtin_amdgcn_mov_dpp(v, K * 0x55, 0xf, 0xf, true);
+}
+template <int K> __device__ __forceinline__ float quad_lane(float v) {
+	return __int_as_float(quad_lane<K>(__float_as_int(v)));
+}
+// v[k] of lane j <- v[j] of lane k
+__device__ __forceinline__ void quad_transpose(float v[4], bool odd, bool high) {
+	constexpr int swap1 = 0xb1, swap2 = 0x4e; // quad_perm [1,0,3,2] and [2,3,0,1]
+#pragma unroll
+	for (int i = 0; i < 4; i += 2) {
+		const float a = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[i]), swap1, 0xf, 0xf, true));
+		const float b = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[i + 1]), swap1, 0xf, 0xf, true));
+		v[i] = odd ? b : v[i];
+		v[i + 1] = odd ? v[i + 1] : a;
+	}
+#pragma unroll
+	for (int i = 0; i < 2; i++) {
+		const float a = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[i]), swap2, 0xf, 0xf, true));
+		const float b = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[i + 2]), swap2, 0xf, 0xf, true));
+		v[i] = high ? b : v[i];
+		v[i + 2] = high ? v[i + 2] : a;
+	}
+}
+
+// A Grid3f read tricubic, four lanes to a particle (the same operations as grid_tricubic, so the same bits).
+// One lane's 64 points lie in 16 rows of four; a load in which every lane reads a point of its own row costs
+// the address unit a cycle a lane, 4096 cycles a wave for 64 particles, and one particle a lane leaves one
+// wave of 330 registers on a SIMD.  Here the four lanes of a quad read the four points of a row together
+// (48 bytes, one or two lines), and the quad shares the cubics: lane j takes the z-cubics of row y_j of
+// every plane, the y-cubics of plane x_j, and all four the last one; values change lanes by DPP.
+struct FieldTricubic {
+	GridDesc g;
+
+	template <bool Fast> __device__ __forceinline__ V3 value(const V3 &p, bool *bad) const {
+		const int j = __lane_id() & 3;
+		const bool odd = j & 1, high = j & 2;
+		double r[3];
+		grid_position<Fast>(g, p, r[0], r[1], r[2], bad);
+		int own[3];
+		float t[3], t2[3], t3[3];
+#pragma unroll
+		for (int a = 0; a < 3; a++) {
+			const int i0 = (int)__builtin_floor(r[a]);
+			const double f = r[a] - (double)i0;
+			t[a] = (float)f;
+			t2[a] = (float)(f * f);
+			t3[a] = (float)(f * f * f);
+			own[a] = i0 - 1 + j; // this lane's neighbour on the axis
+		}
+		const unsigned zo = (unsigned)cubic_index(own[2], g.nz, g.invN[2], g.reflective);
+		const int yo = (int)((unsigned)cubic_index(own[1], g.ny, g.invN[1], g.reflective) * (unsigned)g.nz);
+		const int xo = (int)((unsigned)cubic_index(own[0], g.nx, g.invN[0], g.reflective) * (unsigned)g.ny * (unsigned)g.nz);
+		const unsigned Y[4] = {(unsigned)quad_lane<0>(yo), (unsigned)quad_lane<1>(yo), (unsigned)quad_lane<2>(yo),
+		                       (unsigned)quad_lane<3>(yo)};
+		const unsigned X[4] = {(unsigned)quad_lane<0>(xo), (unsigned)quad_lane<1>(xo), (unsigned)quad_lane<2>(xo),
+		                       (unsigned)quad_lane<3>(xo)};
+		float v[4][4][3]; // plane, row, component: this lane's point
+#pragma unroll
+		for (int a = 0; a < 4; a++)
+#pragma unroll
+			for (int b = 0; b < 4; b++) {
+				const unsigned off = 12u * (X[a] + Y[b] + zo); // below 4 GiB (grid_tricubic_fits)
+				const float *q = reinterpret_cast<const float *>(reinterpret_cast<const char *>(g.values) + off);
+#pragma unroll
+				for (int l = 0; l < 3; l++)
+					v[a][b][l] = q[l];
+			}
+		float vx[3];
+#pragma unroll
+		for (int l = 0; l < 3; l++) {
+			float w[4]; // plane a: row y_j after its z-cubic
+#pragma unroll
+			for (int a = 0; a < 4; a++) {
+				float z[4] = {v[a][0][l], v[a][1][l], v[a][2][l], v[a][3][l]};
+				quad_transpose(z, odd, high);
+				w[a] = cubic_f32(z[0], z[1], z[2], z[3], t[2], t2[2], t3[2]);
+			}
+			quad_transpose(w, odd, high); // rows of plane x_j
+			vx[l] = cubic_f32(w[0], w[1], w[2], w[3], t[1], t2[1], t3[1]);
+		}
+		float b[3];
+#pragma unroll
+		for (int l = 0; l < 3; l++)
+			b[l] = cubic_f32(quad_lane<0>(vx[l]), quad_lane<1>(vx[l]), quad_lane<2>(vx[l]), quad_lane<3>(vx[l]), t[0],
+			                 t2[0], t3[0]);
+		return v3((double)b[0], (double)b[1], (double)b[2]);
+	}
+	__device__ __forceinline__ bool outside(const V3 &p) const { return g.clip && !in_clip_box(g, p); }
+	__device__ __forceinline__ V3 eval(const V3 &p) const {
+		if (outside(p))
+			return v3(0.0, 0.0, 0.0);
+		return value<false>(p, nullptr);
+	}
+	__device__ __forceinline__ V3 eval_fast(const V3 &p, bool &bad) const {
+		const V3 b = value<true>(p, &bad);
+		return outside(p) ? v3(0.0, 0.0, 0.0) : b;
+	}
+	__device__ __forceinline__ const FieldTricubic &lane_field() const { return *this; }
+	__device__ __forceinline__ float3 evalf(const V3 &p) const {
+		const V3 b = eval(p);
+		return make_float3((float)b.x, (float)b.y, (float)b.z);
+	}
+};
+template <> struct LaneGroup<FieldTricubic> {
+	static constexpr int value = 4;
+};
+
+// A periodic Grid3f read tricubic through a table of row pairs: entry (x, y, z) holds the points z .. z + 3 of
+// rows y and y + 1 (wrapped) as 24 floats in a 128-byte line, so the 64 points come from 8 lines instead of the
+// 21.5 that 16 rows of 48 bytes touch; where a batch fills the chip the rate of line requests bounds it.  A run
+// builds the table for itself (the grid may be the caller's memory and change between runs).
+struct FieldTricubicTable {
+	GridDesc g;
+	const float *rows; // [nx*ny*nz][32]
+
+	__device__ __forceinline__ V3 value(const V3 &p) const {
+		double r[3];
+		grid_position<false>(g, p, r[0], r[1], r[2], nullptr);
+		int i0[3];
+		float t[3], t2[3], t3[3];
+#pragma unroll
+		for (int a = 0; a < 3; a++) {
+			i0[a] = (int)__builtin_floor(r[a]);
+			const double f = r[a] - (double)i0[a];
+			t[a] = (float)f;
+			t2[a] = (float)(f * f);
+			t3[a] = (float)(f * f * f);
+		}
+		const size_t z = (size_t)wrap_index(i0[2] - 1, g.nz, g.invN[2]);
+		const size_t y0 = (size_t)wrap_index(i0[1] - 1, g.ny, g.invN[1]) * g.nz + z;
+		const size_t y1 = (size_t)wrap_index(i0[1] + 1, g.ny, g.invN[1]) * g.nz + z;
+		float vx[4][3];
+#pragma unroll
+		for (int a = 0; a < 4; a++) {
+			const size_t x = (size_t)wrap_index(i0[0] - 1 + a, g.nx, g.invN[0]) * g.ny * g.nz;
+			float w[4][3];
+#pragma unroll
+			for (int h = 0; h < 2; h++) {
+				const float4 *c = reinterpret_cast<const float4 *>(rows + 32 * (x + (h ? y1 : y0)));
+				const float4 q0 = c[0], q1 = c[1], q2 = c[2], q3 = c[3], q4 = c[4], q5 = c[5];
+				const float v[24] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x, q2.y, q2.z, q2.w,
+				                     q3.x, q3.y, q3.z, q3.w, q4.x, q4.y, q4.z, q4.w, q5.x, q5.y, q5.z, q5.w};
+#pragma unroll
+				for (int l = 0; l < 3; l++) {
+					w[2 * h][l] = cubic_f32(v[l], v[3 + l], v[6 + l], v[9 + l], t[2], t2[2], t3[2]);
+					w[2 * h + 1][l] = cubic_f32(v[12 + l], v[15 + l], v[18 + l], v[21 + l], t[2], t2[2], t3[2]);
+				}
+			}
+#pragma unroll
+			for (int l = 0; l < 3; l++)
+				vx[a][l] = cubic_f32(w[0][l], w[1][l], w[2][l], w[3][l], t[1], t2[1], t3[1]);
+		}
+		float b[3];
+#pragma unroll
+		for (int l = 0; l < 3; l++)
+			b[l] = cubic_f32(vx[0][l], vx[1][l], vx[2][l], vx[3][l], t[0], t2[0], t3[0]);
+		return v3((double)b[0], (double)b[1], (double)b[2]);
+	}
+	__device__ __forceinline__ bool outside(const V3 &p) const { return g.clip && !in_clip_box(g, p); }
+	__device__ __forceinline__ V3 eval(const V3 &p) const {
+		if (outside(p))
+			return v3(0.0, 0.0, 0.0);
+		return value(p);
+	}
+	__device__ __forceinline__ float3 evalf(const V3 &p) const {
+		const V3 b = eval(p);
+		return make_float3((float)b.x, (float)b.y, (float)b.z);
+	}
+};
+
 struct FieldPlaneWave {
 	PlaneWaveDesc w;
 
@@ -1145,6 +1323,12 @@ template <> struct FloatValuedField<FieldGridCells> {
 template <> struct FloatValuedField<FieldGrid> {
 	static constexpr bool value = true;
 };
+template <> struct FloatValuedField<FieldTricubicTable> {
+	static constexpr bool value = true;
+};
+template <> struct FloatValuedField<FieldTricubic> {
+	static constexpr bool value = true;
+};
 template <> struct FloatValuedField<FieldGridCellsWave> {
 	static constexpr bool value = true;
 };
@@ -1253,6 +1437,9 @@ template <> struct FastField<FieldGridCells> {
 	static constexpr bool value = true;
 };
 template <> struct FastField<FieldGrid> {
+	static constexpr bool value = true;
+};
+template <> struct FastField<FieldTricubic> {
 	static constexpr bool value = true;
 };
 template <> struct FastField<FieldGridCellsWave> {

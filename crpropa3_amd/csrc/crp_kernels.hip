@@ -135,6 +135,8 @@ struct crp_batch {
 	uint64_t *sdeStream; // DiffusionSDE random stream per particle (main allocation, 8-byte aligned)
 	double *snap;     // detection snapshots [snapK][kSnapDoubles][cap], allocated on first use
 	int snapK;
+	float *rows;      // FieldTricubicTable's table, built by each run that reads it; kept for the next
+	size_t rowsBytes;
 	// captured launch sequence of the last graph-enabled call, keyed by the exact bytes of every
 	// kernel argument and launch dimension it holds
 	hipGraphExec_t gexec;
@@ -209,6 +211,34 @@ __global__ void __launch_bounds__(256) k_build_cells(const float *__restrict__ g
 		float4 *o = reinterpret_cast<float4 *>(cells + (size_t)kCellFloats * c);
 #pragma unroll
 		for (int k = 0; k < 8; k++)
+			o[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+	}
+}
+
+// FieldTricubicTable's row pairs
+__global__ void __launch_bounds__(256) k_build_rows(const float *__restrict__ g, float *__restrict__ rows, int nx, int ny,
+                                                    int nz) {
+	const size_t total = (size_t)nx * ny * nz, stride = (size_t)gridDim.x * blockDim.x;
+	for (size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x; c < total; c += stride) {
+		const int z = (int)(c % nz);
+		const size_t t = c / nz;
+		const int y = (int)(t % ny);
+		const size_t x = t / ny;
+		float v[24];
+#pragma unroll
+		for (int h = 0; h < 2; h++) {
+			const size_t row = (x * ny + (y + h) % ny) * nz;
+#pragma unroll
+			for (int k = 0; k < 4; k++) {
+				const float *s = g + 3 * (row + (z + k) % nz);
+				v[12 * h + 3 * k] = s[0];
+				v[12 * h + 3 * k + 1] = s[1];
+				v[12 * h + 3 * k + 2] = s[2];
+			}
+		}
+		float4 *o = reinterpret_cast<float4 *>(rows + 32 * c);
+#pragma unroll
+		for (int k = 0; k < 6; k++)
 			o[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
 	}
 }
@@ -422,9 +452,10 @@ static int launch_propagate(const F &f, const crp_propagator *p, const Params &P
 	// A batch of fewer particles than the chip's SIMDs have lanes is spread over all of them, a wave taking
 	// `lanes` particles: every particle is one serial chain, and a wave with fewer of them waits for fewer
 	// lines per load and fewer rare branches.
+	constexpr size_t group = KIND == PK_SDE ? 1 : LaneGroup<typename KernelField<F, MIX>::type>::value;
 	const size_t waves = std::min<size_t>((size_t)ncu * bpc * (block / 64), (size_t)ncu * 4);
-	const int lanes = (int)std::min<size_t>(64, std::max<size_t>(1, (b->n + waves - 1) / waves));
-	const size_t perBlock = (size_t)lanes * (block / 64);
+	const int lanes = (int)std::min<size_t>(64, group * std::max<size_t>(1, (b->n + waves - 1) / waves));
+	const size_t perBlock = (size_t)lanes / group * (block / 64);
 	const size_t want = (b->n + perBlock - 1) / perBlock;
 	const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(want, (size_t)ncu * bpc));
 	p->lastGrid = grid;
@@ -567,6 +598,41 @@ static int dispatch_cells(const FieldGridCells &f, const crp_propagator *p, cons
 	                                           : dispatch_kind_p<FieldGridCellsBig, false>(big, p, P, b, launches);
 }
 
+// Tricubic grids.  Up to kQuadParticles a batch leaves lanes idle and is bound by each particle's chain: four
+// lanes share a particle (128^3 grid, 300 Boris steps: 1000 to 16384 particles in 1.5 - 2.0 ms against 3.9, 32768
+// in 3.8 against 4.4); above, by the rate of line requests (65536: 7.2 ms with quads, 6.1 a lane each), and a table
+// of row pairs pays where the run evaluates the field more often than the table has entries.
+constexpr size_t kQuadParticles = 32768;
+constexpr size_t kRowsBytesMax = (size_t)2 << 30;
+
+// whether this run reads a row-pair table; builds it on the batch's stream
+static bool tricubic_rows(const GridDesc &g, const crp_propagator *p, const Params &P, crp_batch *b) {
+	const size_t ncell = (size_t)g.nx * g.ny * g.nz, bytes = ncell * 32 * sizeof(float);
+	if (g.interp != kInterpTricubic || g.reflective || b->n <= kQuadParticles || bytes > kRowsBytesMax)
+		return false;
+	const double evals = p->type == 1 ? 6 : (P.minStep == P.maxStep ? 1 : 3);
+	double steps = P.maxSteps >= 0 ? (double)P.maxSteps : HUGE_VAL;
+	if (P.maxLen > 0 && P.maxStep > 0)
+		steps = std::min(steps, P.maxLen / P.maxStep); // at least
+	if (steps * evals * (double)b->n < 2.0 * (double)ncell)
+		return false;
+	if (b->rowsBytes < bytes) {
+		if (b->rows)
+			(void)hipFree(b->rows);
+		b->rows = nullptr;
+		b->rowsBytes = 0;
+		if (hipMalloc((void **)&b->rows, bytes) != hipSuccess) {
+			(void)hipGetLastError();
+			b->rows = nullptr;
+			return false;
+		}
+		b->rowsBytes = bytes;
+	}
+	const unsigned blocks = (unsigned)std::min<size_t>((ncell + 255) / 256, 65536);
+	hipLaunchKernelGGL(k_build_rows, dim3(blocks), dim3(256), 0, b->stream, g.values, b->rows, g.nx, g.ny, g.nz);
+	return hipGetLastError() == hipSuccess;
+}
+
 // ------------------------------------------------------------------ C ABI
 extern "C" {
 
@@ -687,6 +753,11 @@ static bool any_interp(const crp_field *f) {
 	if (f->kind == FK_MODULATED)
 		return f->grid.interp != kInterpTrilinear || f->mod.interp != kInterpTrilinear;
 	return false;
+}
+
+// a grid that FieldTricubic reads: tricubic, its byte offsets within 32 bits
+static bool grid_tricubic_fits(const GridDesc &g) {
+	return g.interp == kInterpTricubic && (size_t)g.nx * g.ny * g.nz * 12 <= 0xffffffffull;
 }
 
 // a JF12 field whose turbulent grid is not read trilinear: FieldJF12Any
@@ -2000,6 +2071,8 @@ int crp_batch_destroy(crp_batch_t *b) {
 	(void)hipFree(b->base);
 	if (b->snap)
 		(void)hipFree(b->snap);
+	if (b->rows)
+		(void)hipFree(b->rows);
 	delete b;
 	return CRP_OK;
 }
@@ -2268,7 +2341,19 @@ int crp_propagate(const crp_propagator_t *p, crp_batch_t *b, long long max_steps
 	int rc;
 	const crp_field *f = p->field;
 	switch (any_interp(f) ? -1 : (f ? f->kind : FK_NONE)) {
-	case -1: rc = dispatch_kind(grid_any(f), p, P, b, &st.launches); break;
+	case -1:
+		if (p->type != 2 && f->kind == FK_GRID && tricubic_rows(f->grid, p, P, b)) {
+			const FieldTricubicTable t{f->grid, b->rows};
+			rc = p->precision == CRP_PRECISION_MIXED ? dispatch_kind_p<FieldTricubicTable, true>(t, p, P, b, &st.launches)
+			                                         : dispatch_kind_p<FieldTricubicTable, false>(t, p, P, b, &st.launches);
+		} else if (p->type != 2 && f->kind == FK_GRID && grid_tricubic_fits(f->grid) && b->n <= kQuadParticles) {
+			const FieldTricubic t{f->grid};
+			rc = p->precision == CRP_PRECISION_MIXED ? dispatch_kind_p<FieldTricubic, true>(t, p, P, b, &st.launches)
+			                                         : dispatch_kind_p<FieldTricubic, false>(t, p, P, b, &st.launches);
+		} else {
+			rc = dispatch_kind(grid_any(f), p, P, b, &st.launches);
+		}
+		break;
 	case FK_UNIFORM: rc = dispatch_kind(f->uniform, p, P, b, &st.launches); break;
 	case FK_GRID:
 		if (p->precision == CRP_PRECISION_MIXED && f->cells16)

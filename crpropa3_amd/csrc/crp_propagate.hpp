@@ -135,6 +135,11 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 	constexpr bool kFast = FastField<typename KernelField<F, MIX>::type>::value;
 	constexpr bool kWave = WaveField<typename KernelField<F, MIX>::type>::value;
 	const int lane = __lane_id();
+	// lanes that hold one particle together: all its state is the same in them, they store the same values and
+	// the first of them counts
+	constexpr int kGroup = LaneGroup<typename KernelField<F, MIX>::type>::value;
+	const bool first = lane % kGroup == 0;
+
 	bool have = false, exhausted = lane >= P.lanes, inProc = false;
 	CkB0Store<FloatValuedField<typename KernelField<F, MIX>::type>::value> b0; // the field at the trial sequence's start (adaptive CK), for retries
 	CkB0f b0f;
@@ -173,9 +178,11 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 
 	for (;;) {
 		if (nEval > 0x80000000u) { // flush this lane's counters long before they wrap
-			atomicAdd(&ctr[CTR_ACCEPTED], (unsigned long long)nAcc);
-			atomicAdd(&ctr[CTR_REJECTED], (unsigned long long)nRej);
-			atomicAdd(&ctr[CTR_EVALS], (unsigned long long)nEval);
+			if (first) {
+				atomicAdd(&ctr[CTR_ACCEPTED], (unsigned long long)nAcc);
+				atomicAdd(&ctr[CTR_REJECTED], (unsigned long long)nRej);
+				atomicAdd(&ctr[CTR_EVALS], (unsigned long long)nEval);
+			}
 			nAcc = nRej = nEval = 0;
 		}
 		// ---- refill lanes without a particle from the queue
@@ -185,10 +192,11 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 			const int leader = __ffsll((long long)m) - 1;
 			unsigned long long base = 0;
 			if (lane == leader)
-				base = atomicAdd(&ctr[CTR_QUEUE], (unsigned long long)__popcll(m));
+				base = atomicAdd(&ctr[CTR_QUEUE], (unsigned long long)__popcll(m) / kGroup);
 			base = __shfl(base, leader);
 			if (need) {
-				const unsigned long long my = base + (unsigned long long)__popcll(m & ((1ull << lane) - 1ull));
+				const unsigned long long below = m & ((1ull << (lane & ~(kGroup - 1))) - 1ull);
+				const unsigned long long my = base + (unsigned long long)__popcll(below) / kGroup;
 				if (my < n) {
 					idx = S.order[my];
 					have = S.active[idx] != 0;
@@ -489,6 +497,8 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 			have = false;
 		}
 	}
+	if (!first)
+		nAcc = nRej = nEval = nFin = nPause = 0;
 	const unsigned long long tAcc = wave_sum(nAcc), tRej = wave_sum(nRej), tEval = wave_sum(nEval),
 	                         tFin = wave_sum(nFin), tPause = wave_sum(nPause);
 	if (lane == 0) {

@@ -171,3 +171,36 @@ def test_staged_eval(n, precision):
     assert same(got, want)
     if precision == capi.PRECISION_FP64:
         assert same(got, O.OracleField.grid(g, [0, 0, 0], 1.0).eval(pos))
+
+
+@pytest.mark.parametrize("shape,clip", [((1, 1, 1), False), ((2, 3, 5), False), ((4, 4, 4), True), ((9, 6, 19), False)])
+@pytest.mark.parametrize("kind,fixed", [("BP", True), ("BP", False), ("CK", True), ("CK", False)])
+def test_tricubic_row_table(kind, fixed, shape, clip):
+    """Batches that fill the chip read a table of row pairs built by the run: copies of the same particles, every
+    wrap; then the caller's grid changes and the next run of the same batch sees it."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(17)
+    m, n = 1003, 33100
+    sp = [20 * KPC] * 3
+    L = np.array(shape) * 20 * KPC
+    pos, d, E = rng.uniform(-0.6, 1.6, (m, 3)) * L, rng.normal(size=(m, 3)), 10 ** rng.uniform(0, 2, m) * EEV
+    q = np.where(np.arange(m) % 6 == 1, 0.0, EPLUS)
+    lo, hi = (20 * KPC, 20 * KPC) if fixed else (KPC, 60 * KPC)
+    idx = np.arange(n) % m
+    dev = torch.empty(tuple(shape) + (3,), dtype=torch.float32, device="cuda:0")
+    f = capi.Field.grid3f_device(dev.data_ptr(), shape, [0, 0, 0], sp, clip_volume=clip, keep=dev)
+    f.set_interpolation("TRICUBIC")
+    p, b = capi.Propagator(kind, f, 1e-3, lo, hi), capi.Batch(n)
+    for seed in (3, 4):
+        g = noise(shape, seed)
+        dev.copy_(torch.from_numpy(g))
+        torch.cuda.synchronize()
+        ref = O.OracleState(pos, d, E, q)
+        O.propagate(O.OracleField.grid(g, [0, 0, 0], sp, False, clip, interp=O.GRID_TRICUBIC),
+                    O.PROP_BP if kind == "BP" else O.PROP_CK, ref, 8, tolerance=1e-3, min_step=lo, max_step=hi,
+                    libm=O.LIBM_CR)
+        b.upload(pos[idx], O.normalise(d)[idx], E[idx], q[idx])
+        p.propagate(b, max_steps=8)
+        out = b.download()
+        for k in ("pos", "dir", "next_step", "trajectory_length"):
+            assert same(out[k], getattr(ref, k)[idx]), k

@@ -64,20 +64,6 @@ struct CompositeDesc {
 	CompLeaf leaves[kCompMaxLeaves];
 };
 
-// A trivially copyable value read from immutable device memory through the constant address space,
-// so that wave-uniform reads become scalar loads.
-template <class T> __device__ __forceinline__ T ld_const(const T *p) {
-	static_assert(sizeof(T) % 4 == 0, "ld_const: size must be a multiple of 4");
-	typedef __attribute__((address_space(4))) const uint32_t cu32;
-	cu32 *src = (cu32 *)p;
-	T out;
-	uint32_t *dst = reinterpret_cast<uint32_t *>(&out);
-#pragma unroll
-	for (unsigned i = 0; i < sizeof(T) / 4; i++)
-		dst[i] = src[i];
-	return out;
-}
-
 template <class T> __device__ __forceinline__ T slot_get(const T &s0, const T &s1, const T &s2, const T &s3, int i) {
 	return i == 0 ? s0 : (i == 1 ? s1 : (i == 2 ? s2 : s3));
 }

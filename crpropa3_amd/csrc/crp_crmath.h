@@ -580,17 +580,8 @@ CRP_MATH_FN double crp_sin_cr(double x) {
  * 0 when it does not decide: 2e-4 of arguments.  `tab` is crp_turn_tab or a copy of it.
  */
 #define CRP_TURN_ENTRIES 768
-CRP_MATH_FN int crp_cos_turn(double x, int shift, const double *tab, double *out) {
-	const double big = 6755399441055744.0; /* 1.5 * 2^52: the sum's low bits are the nearest integer */
-	const double kb = __builtin_fma(x, CRP_TURN_INV, big);
-	const uint32_t ki = (uint32_t)crp_as_u64(kb) - (uint32_t)shift;
-	const double k = kb - big;
-	const double r0 = __builtin_fma(-k, CRP_TURN_P1, x); /* exact */
-	const double t = k * CRP_TURN_P2, te = __builtin_fma(k, CRP_TURN_P2, -t);
-	const double rh = r0 - t;
-	const double rl = __builtin_fma(-k, CRP_TURN_P3, ((r0 - rh) - t) - te);
-	const double *const e = tab + 2 * (ki & 511u);
-	const double Sh = e[0], Sl = e[1], Ch = e[512], Cl = e[513];
+/* C cos r - S sin r and its rounding test */
+CRP_MATH_FN int crp_turn_sum(double rh, double rl, double Sh, double Sl, double Ch, double Cl, double *out) {
 	const double z = rh * rh;
 	const double c4 = (z * z) * __builtin_fma(z, -1.0 / 720, 1.0 / 24); /* cos r - 1 + z/2 */
 	/* sin r - rh */
@@ -607,7 +598,23 @@ CRP_MATH_FN int crp_cos_turn(double x, int shift, const double *tab, double *out
 	const double as = __builtin_fabs(s.hi);
 	const double y = s.hi + __builtin_fma(as, 1.25 * 0x1p-67, lo);
 	const double y2 = s.hi + __builtin_fma(as, -1.25 * 0x1p-67, lo);
-	if (!(y == y2 && as > 0x1p-28 && __builtin_fabs(x) < 0x1p30))
+	*out = y;
+	return y == y2 && as > 0x1p-28;
+}
+
+CRP_MATH_FN int crp_cos_turn(double x, int shift, const double *tab, double *out) {
+	const double big = 6755399441055744.0; /* 1.5 * 2^52: the sum's low bits are the nearest integer */
+	const double kb = __builtin_fma(x, CRP_TURN_INV, big);
+	const uint32_t ki = (uint32_t)crp_as_u64(kb) - (uint32_t)shift;
+	const double k = kb - big;
+	const double r0 = __builtin_fma(-k, CRP_TURN_P1, x); /* exact */
+	const double t = k * CRP_TURN_P2, te = __builtin_fma(k, CRP_TURN_P2, -t);
+	const double rh = r0 - t;
+	const double rl = __builtin_fma(-k, CRP_TURN_P3, ((r0 - rh) - t) - te);
+	const double *const e = tab + 2 * (ki & 511u);
+	const double Sh = e[0], Sl = e[1], Ch = e[512], Cl = e[513];
+	double y;
+	if (!(crp_turn_sum(rh, rl, Sh, Sl, Ch, Cl, &y) && __builtin_fabs(x) < 0x1p30))
 		return 0;
 	*out = crp_from_u64(crp_as_u64(y) ^ ((uint64_t)((ki << 22) & 0x80000000u) << 32));
 	return 1;
@@ -629,12 +636,33 @@ CRP_MATH_FN double crp_cos_cr_turn(double x, const double *tab) {
 	return crp_cos_cr_cold(x, 0);
 }
 
-/* sin(x) likewise: sin x = cos(x - pi/2), a quarter turn is 256 entries */
-CRP_MATH_FN double crp_sin_cr_turn(double x, const double *tab) {
-	double v;
-	if (crp_cos_turn(x, 256, tab, &v))
-		return v;
-	return crp_cos_cr_cold(x, 3);
+/* sin(x) and cos(x) by the quick phase, from one reduction: sin x = S cos r + C sin r is crp_turn_sum with
+ * C, -S for S, C.  Returns 0 when either is undecided. */
+CRP_MATH_FN int crp_sincos_turn(double x, double *sin_out, double *cos_out) {
+	const double big = 6755399441055744.0;
+	const double kb = __builtin_fma(x, CRP_TURN_INV, big);
+	const uint32_t ki = (uint32_t)crp_as_u64(kb);
+	const double k = kb - big;
+	const double r0 = __builtin_fma(-k, CRP_TURN_P1, x);
+	const double t = k * CRP_TURN_P2, te = __builtin_fma(k, CRP_TURN_P2, -t);
+	const double rh = r0 - t;
+	const double rl = __builtin_fma(-k, CRP_TURN_P3, ((r0 - rh) - t) - te);
+	const double *const e = crp_turn_tab + 2 * (ki & 511u);
+	const double Sh = e[0], Sl = e[1], Ch = e[512], Cl = e[513];
+	const uint64_t sign = (uint64_t)((ki << 22) & 0x80000000u) << 32;
+	double s, c;
+	const int cs = crp_turn_sum(rh, rl, -Ch, -Cl, Sh, Sl, &s), cc = crp_turn_sum(rh, rl, Sh, Sl, Ch, Cl, &c);
+	*sin_out = crp_from_u64(crp_as_u64(s) ^ sign);
+	*cos_out = crp_from_u64(crp_as_u64(c) ^ sign);
+	return cs & cc & (__builtin_fabs(x) < 0x1p30);
+}
+
+/* sin(x) (hi) and cos(x) (lo), correctly rounded */
+CRP_MATH_COLD crp_dd crp_sincos_cr(double x) {
+	double s, c;
+	if (crp_sincos_turn(x, &s, &c))
+		return crp_mkdd(s, c);
+	return crp_mkdd(crp_cos_cr_cold(x, 3), crp_cos_cr_cold(x, 0));
 }
 
 /* log(x) for finite x > 0: the double-double logarithm (absolute error about 2^-104)

@@ -125,6 +125,20 @@ __device__ __forceinline__ V3 div3_rn(const V3 &v, double s, double invs) {
 	return r;
 }
 
+// A trivially copyable value read from immutable device memory through the constant address space,
+// so that wave-uniform reads become scalar loads.
+template <class T> __device__ __forceinline__ T ld_const(const T *p) {
+	static_assert(sizeof(T) % 4 == 0, "ld_const: size must be a multiple of 4");
+	typedef __attribute__((address_space(4))) const uint32_t cu32;
+	cu32 *src = (cu32 *)p;
+	T out;
+	uint32_t *dst = reinterpret_cast<uint32_t *>(&out);
+#pragma unroll
+	for (unsigned i = 0; i < sizeof(T) / 4; i++)
+		dst[i] = src[i];
+	return out;
+}
+
 // u / |u|, one range test
 __device__ __forceinline__ V3 unit_rn(const V3 &u) {
 	const double n = norm(u), invn = rcp_rn(n);
@@ -313,6 +327,11 @@ __device__ __forceinline__ int reflect_index(int i, int n) {
 	return (m < n) ? m : p - 1 - m;
 }
 
+// fmod(x, n), which is x itself for |x| < n: most positions lie within a box of the origin, and the loop of
+// the general case is left to the others
+__device__ __attribute__((noinline)) inline double fmod_far(double x, double n) { return __builtin_fmod(x, n); }
+__device__ __forceinline__ double fmod_near(double x, double n) { return __builtin_fabs(x) < n ? x : fmod_far(x, n); }
+
 // Grid::closestValue (include/crpropa/Grid.h:383-405): flat index of the grid point nearest to p,
 // mirrored (reflective) or wrapped (periodic) into the grid
 __device__ inline size_t grid_closest(const GridDesc &g, const V3 &p) {
@@ -326,9 +345,9 @@ __device__ inline size_t grid_closest(const GridDesc &g, const V3 &p) {
 		iz = reflect_index((int)round_sym(rz), g.nz);
 	} else {
 		// fmod(r, n) lies in (-n, n), its rounding in [-n, n]: (i + n * (i < 0)) % n is one correction each way
-		ix = (int)round_sym(__builtin_fmod(rx, (double)g.nx));
-		iy = (int)round_sym(__builtin_fmod(ry, (double)g.ny));
-		iz = (int)round_sym(__builtin_fmod(rz, (double)g.nz));
+		ix = (int)round_sym(fmod_near(rx, (double)g.nx));
+		iy = (int)round_sym(fmod_near(ry, (double)g.ny));
+		iz = (int)round_sym(fmod_near(rz, (double)g.nz));
 		ix += (ix < 0) ? g.nx : 0;
 		iy += (iy < 0) ? g.ny : 0;
 		iz += (iz < 0) ? g.nz : 0;

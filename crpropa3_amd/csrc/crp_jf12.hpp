@@ -13,6 +13,27 @@ namespace crp {
 constexpr double kJKpc = 1e3 * (648000 / 3.14159265358979323846 * 149597870700.0);
 constexpr double kJPi = 3.14159265358979323846;
 
+// exp and atan2 for the arguments that their quick phases leave open
+static __device__ __attribute__((noinline)) double jf12_exp(double x) { return crp_exp_rn(x); }
+static __device__ __attribute__((noinline)) double jf12_atan2(double y, double x) { return crp_atan2_rn(y, x); }
+// five exponentials side by side, one copy of the code
+struct Exp5 {
+	double a, b, c, d, e;
+};
+static __device__ __attribute__((noinline)) Exp5 jf12_exp5(double a, double b, double c, double d, double e) {
+	const double x[5] = {a, b, c, d, e};
+	double v[5];
+	bool ok[5];
+#pragma unroll
+	for (int i = 0; i < 5; i++)
+		ok[i] = crp_exp_quick(x[i], &v[i]) && x[i] >= -708.0 && x[i] <= 708.0;
+#pragma unroll
+	for (int i = 0; i < 5; i++)
+		if (!ok[i])
+			v[i] = jf12_exp(x[i]);
+	return Exp5{v[0], v[1], v[2], v[3], v[4]};
+}
+
 // Grid<float>::closestValue (include/crpropa/Grid.h:383-405): nearest point, reflective or periodic
 __device__ __forceinline__ float scalar_grid_closest(const GridDesc &g, const V3 &p) { return g.values[grid_closest(g, p)]; }
 
@@ -24,62 +45,95 @@ struct FieldJF12 {
 	// pow(x, 2.) as the reference's build evaluates it: GCC rewrites the call as x * x
 	__device__ __forceinline__ static double sq(double x) { return x * x; }
 
-	// JF12Field::logisticFunction (JF12Field.cpp:188-190)
-	__device__ __forceinline__ double logistic(double x, double x0, double w) const {
-		return 1. / (1. + crp_exp_rn(-2. * (__builtin_fabs(x) - x0) / w));
+	// JF12Field::logisticFunction (JF12Field.cpp:188-190): 1 / (1 + exp(logistic_arg))
+	__device__ __forceinline__ static double logistic_arg(double x, double x0, double w) {
+		return -2. * (__builtin_fabs(x) - x0) / w;
 	}
 
-	// radius where the arm through (r, phi) crosses the negative x-axis, tried for three windings
-	__device__ __forceinline__ double r_negx(double r, double phi) const {
-		double rn = r * crp_exp_rn(-(phi - kJPi) / p.tan90_minus_pitch);
-		if (rn > p.r_arms[7])
-			rn = r * crp_exp_rn(-(phi + kJPi) / p.tan90_minus_pitch);
-		if (rn > p.r_arms[7])
-			rn = r * crp_exp_rn(-(phi + 3 * kJPi) / p.tan90_minus_pitch);
-		return rn;
-	}
-
-	// What getRegularField and getTurbulentStrength both compute from the position, once per evaluation
-	// (the same operations, so the same bits): |pos|, the in-plane radius, the azimuth (Vector3::getPhi,
-	// include/crpropa/Vector3.h:136-142) and the arm radius r_negx when r >= 5 kpc.
+	// What an evaluation takes from the position: the transcendental functions of every part, each correctly
+	// rounded.  They are formed side by side, whether or not this position's branches read all of them: a
+	// batch has about one wave to a SIMD, where every instruction waits for the one before, and two azimuths,
+	// two sines and cosines and ten exponentials one after the other were most of an evaluation.
+	enum { E_DISK, E_HALO, E_HALO_R, E_X, E_TURB_DISK, E_TURB_R, E_TURB_HALO, E_ARM0, E_ARM1, E_ARM2, E_COUNT };
 	struct Geo {
-		double d, r, phi, rn;
-		bool haveRn;
+		double d, r, rn, rc, rp;
+		double sinPhi, cosPhi, sinThetaX, cosThetaX;
+		double e[E_COUNT];
 	};
 	__device__ __forceinline__ Geo geo(const V3 &pos) const {
 		Geo g;
+		const double z = pos.z, az = __builtin_fabs(z);
 		g.d = norm(pos);
 		g.r = __builtin_sqrt(pos.x * pos.x + pos.y * pos.y);
+		// X field (:252-300): rp and the angle inside rc
+		g.rc = p.r_xc + az / p.tan_theta_x0;
+		const bool inner = g.r < g.rc;
+		g.rp = inner ? g.r * p.r_xc / g.rc : g.r - az / p.tan_theta_x0;
+		// azimuth (Vector3::getPhi, include/crpropa/Vector3.h:136-142) and theta_X
 		const double eps = 2.2250738585072014e-308; // numeric_limits<double>::min()
-		g.phi = (__builtin_fabs(pos.x) < eps && __builtin_fabs(pos.y) < eps) ? 0.0 : crp_atan2_rn(pos.y, pos.x);
-		g.haveRn = false;
-		g.rn = 0;
-		return g;
-	}
-	__device__ __forceinline__ double arm_radius(Geo &g) const {
-		if (!g.haveRn) {
-			g.rn = r_negx(g.r, g.phi);
-			g.haveRn = true;
+		const bool axis = __builtin_fabs(pos.x) < eps && __builtin_fabs(pos.y) < eps;
+		const double tx = g.r - g.rp;
+		double phi = 0, theta = 0;
+		const bool okPhi = pos.x == pos.x && pos.y == pos.y && pos.x != 0 && pos.y != 0 && crp_atan2_quick(pos.y, pos.x, &phi);
+		const bool okTheta = az == az && tx == tx && az != 0 && tx != 0 && crp_atan2_quick(az, tx, &theta);
+		if (!okPhi && !axis)
+			phi = jf12_atan2(pos.y, pos.x);
+		if (axis)
+			phi = 0.0;
+		const bool useTheta = p.use_x && inner && g.r * g.r + z * z > 1 * kJKpc * kJKpc;
+		if (!okTheta && useTheta && z != 0)
+			theta = jf12_atan2(az, tx);
+		if (z == 0)
+			theta = kJPi / 2.;
+		// exponentials
+		double x[E_COUNT];
+		x[E_DISK] = logistic_arg(z, p.h_disk, p.w_disk);
+		x[E_HALO] = -az / p.z0;
+		x[E_HALO_R] = logistic_arg(g.r, z >= 0 ? p.r_north : p.r_south, p.w_halo);
+		x[E_X] = -g.rp / p.r_x;
+		x[E_TURB_DISK] = p.use_turbulent ? -0.5 * sq(z / p.z_disk_turb) : 0.0;
+		x[E_TURB_R] = p.use_turbulent ? -g.r / p.r_halo_turb : 0.0;
+		x[E_TURB_HALO] = p.use_turbulent ? -0.5 * sq(z / p.z_halo_turb) : 0.0;
+		x[E_ARM0] = -(phi - kJPi) / p.tan90_minus_pitch;
+		x[E_ARM1] = -(phi + kJPi) / p.tan90_minus_pitch;
+		x[E_ARM2] = -(phi + 3 * kJPi) / p.tan90_minus_pitch;
+		const Exp5 e0 = jf12_exp5(x[0], x[1], x[2], x[3], x[4]), e1 = jf12_exp5(x[5], x[6], x[7], x[8], x[9]);
+		const double e[E_COUNT] = {e0.a, e0.b, e0.c, e0.d, e0.e, e1.a, e1.b, e1.c, e1.d, e1.e};
+#pragma unroll
+		for (int i = 0; i < E_COUNT; i++)
+			g.e[i] = e[i];
+		const bool okP = crp_sincos_turn(phi, &g.sinPhi, &g.cosPhi);
+		const bool okT = crp_sincos_turn(theta, &g.sinThetaX, &g.cosThetaX);
+		if (!okP) {
+			const crp_dd sc = crp_sincos_cr(phi);
+			g.sinPhi = sc.hi;
+			g.cosPhi = sc.lo;
 		}
-		return g.rn;
+		if (!okT) {
+			const crp_dd sc = crp_sincos_cr(theta);
+			g.sinThetaX = sc.hi;
+			g.cosThetaX = sc.lo;
+		}
+		// radius where the arm through (r, phi) crosses the negative x-axis, tried for three windings
+		g.rn = g.r * g.e[E_ARM0];
+		if (g.rn > p.r_arms[7])
+			g.rn = g.r * g.e[E_ARM1];
+		if (g.rn > p.r_arms[7])
+			g.rn = g.r * g.e[E_ARM2];
+		return g;
 	}
 
 	// JF12Field::getRegularField with getDiskField, getToroidalHaloField, getXField (:192-300)
-	__device__ V3 regular(const V3 &pos, Geo &gm) const {
+	__device__ __forceinline__ V3 regular(const V3 &pos, const Geo &gm) const {
 		double bx = 0, by = 0, bz = 0;
-		const double d = gm.d;
-		if (d < 20 * kJKpc) {
+		if (gm.d < 20 * kJKpc) {
 			const double r = gm.r;
-			const double phi = gm.phi;
-			const double sinPhi = crp_sin_cr(phi), cosPhi = crp_cos_cr(phi);
+			const double sinPhi = gm.sinPhi, cosPhi = gm.cosPhi;
 			const double z = pos.z;
-			// the disk's logistic factor, shared by the disk and the toroidal halo
-			const bool needLf = p.use_disk || (p.use_toroidal_halo && (r * r + z * z > 1 * kJKpc * kJKpc));
-			const double lfShared = needLf ? logistic(z, p.h_disk, p.w_disk) : 0.0;
+			const double lfDisk = 1. / (1. + gm.e[E_DISK]);
 			// disk
 			double dx = 0, dy = 0;
 			if (p.use_disk) {
-				const double lfDisk = lfShared;
 				if (r > 3 * kJKpc) {
 					double bMag = 0;
 					if (r < 5 * kJKpc) {
@@ -87,7 +141,7 @@ struct FieldJF12 {
 						dx += -bMag * sinPhi;
 						dy += bMag * cosPhi;
 					} else {
-						const double rn = arm_radius(gm);
+						const double rn = gm.rn;
 						for (int i = 7; i >= 0; i--)
 							if (rn < p.r_arms[i])
 								bMag = p.b_disk[i];
@@ -103,12 +157,12 @@ struct FieldJF12 {
 			// toroidal halo
 			double hx = 0, hy = 0;
 			if (p.use_toroidal_halo && (r * r + z * z > 1 * kJKpc * kJKpc)) {
-				const double lfDisk = lfShared;
-				double bMagH = crp_exp_rn(-__builtin_fabs(z) / p.z0) * lfDisk;
+				double bMagH = gm.e[E_HALO] * lfDisk;
+				const double lfR = 1. / (1. + gm.e[E_HALO_R]);
 				if (z >= 0)
-					bMagH *= p.b_north * (1 - logistic(r, p.r_north, p.w_halo));
+					bMagH *= p.b_north * (1 - lfR);
 				else
-					bMagH *= p.b_south * (1 - logistic(r, p.r_south, p.w_halo));
+					bMagH *= p.b_south * (1 - lfR);
 				hx += -bMagH * sinPhi;
 				hy += bMagH * cosPhi;
 			}
@@ -118,19 +172,14 @@ struct FieldJF12 {
 			// X field
 			double xx = 0, xy = 0, xz = 0;
 			if (p.use_x && (r * r + z * z > 1 * kJKpc * kJKpc)) {
-				double bMagX, sinThetaX, cosThetaX, rp;
-				const double rc = p.r_xc + __builtin_fabs(z) / p.tan_theta_x0;
+				double bMagX, sinThetaX, cosThetaX;
+				const double rc = gm.rc, rp = gm.rp;
 				if (r < rc) {
-					rp = r * p.r_xc / rc;
-					bMagX = p.b_x * crp_exp_rn(-1 * rp / p.r_x) * sq(p.r_xc / rc);
-					double thetaX = crp_atan2_rn(__builtin_fabs(z), (r - rp));
-					if (z == 0)
-						thetaX = kJPi / 2.;
-					sinThetaX = crp_sin_cr(thetaX);
-					cosThetaX = crp_cos_cr(thetaX);
+					bMagX = p.b_x * gm.e[E_X] * sq(p.r_xc / rc);
+					sinThetaX = gm.sinThetaX;
+					cosThetaX = gm.cosThetaX;
 				} else {
-					rp = r - __builtin_fabs(z) / p.tan_theta_x0;
-					bMagX = p.b_x * crp_exp_rn(-rp / p.r_x) * (rp / r);
+					bMagX = p.b_x * gm.e[E_X] * (rp / r);
 					sinThetaX = p.sin_theta_x0;
 					cosThetaX = p.cos_theta_x0;
 				}
@@ -147,7 +196,7 @@ struct FieldJF12 {
 	}
 
 	// JF12Field::getTurbulentStrength (:307-331)
-	__device__ double turbulent_strength(const V3 &pos, Geo &gm) const {
+	__device__ __forceinline__ double turbulent_strength(const Geo &gm) const {
 		if (gm.d > 20 * kJKpc)
 			return 0;
 		const double r = gm.r;
@@ -155,43 +204,58 @@ struct FieldJF12 {
 		if (r < 5 * kJKpc) {
 			bDisk = p.b_disk_turb5;
 		} else {
-			const double rn = arm_radius(gm);
 			for (int i = 7; i >= 0; i--)
-				if (rn < p.r_arms[i])
+				if (gm.rn < p.r_arms[i])
 					bDisk = p.b_disk_turb[i];
 			bDisk *= (5 * kJKpc) / r;
 		}
-		bDisk *= crp_exp_rn(-0.5 * sq(pos.z / p.z_disk_turb));
-		const double bHalo = p.b_halo_turb * crp_exp_rn(-r / p.r_halo_turb) *
-		                     crp_exp_rn(-0.5 * sq(pos.z / p.z_halo_turb));
+		bDisk *= gm.e[E_TURB_DISK];
+		const double bHalo = p.b_halo_turb * gm.e[E_TURB_R] * gm.e[E_TURB_HALO];
 		return __builtin_sqrt(sq(bDisk) + sq(bHalo));
 	}
 
-	// JF12Field::getField (:337-346); the turbulent term is Vector3f * (float)strength in float.
+	// JF12Field::getField (:337-346) with the model read by three sections (jf12_eval); the turbulent term is
+	// Vector3f * (float)strength in float, and every part ends 20 kpc from the centre (:230-231, 307-308).
 	// AnyInterp: the turbulent grid may be read tricubic or nearest-neighbour (Grid::interpolate).
-	template <bool AnyInterp> __device__ __forceinline__ V3 eval_impl(const V3 &pos) const {
-		double bx = 0, by = 0, bz = 0;
-		Geo gm = geo(pos);
-		if (p.use_turbulent) {
-			const V3 g = AnyInterp ? grid_interpolate(turbulent, pos) : FieldGrid{turbulent}.eval(pos);
-			const float s = (float)turbulent_strength(pos, gm);
-			bx += (double)((float)g.x * s);
-			by += (double)((float)g.y * s);
-			bz += (double)((float)g.z * s);
+	template <bool AnyInterp, class M>
+	static __device__ __forceinline__ V3 sum_parts(const V3 &pos, M &&model) {
+		const bool in = !(norm(pos) > 20 * kJKpc);
+		Geo gm;
+		V3 r = v3(0, 0, 0);
+		float strength = 0.f;
+		if (in) {
+			{
+				const FieldJF12 f = model();
+				gm = f.geo(pos);
+			}
+			const FieldJF12 f = model();
+			if (f.p.use_striated || f.p.use_regular)
+				r = f.regular(pos, gm);
+			if (f.p.use_turbulent)
+				strength = (float)f.turbulent_strength(gm);
 		}
-		if (p.use_striated) {
-			const V3 b = regular(pos, gm);
-			const double f = 1. + p.sqrt_beta * (double)scalar_grid_closest(striated, pos);
-			bx += b.x * f;
-			by += b.y * f;
-			bz += b.z * f;
-		} else if (p.use_regular) {
-			const V3 b = regular(pos, gm);
-			bx += b.x;
-			by += b.y;
-			bz += b.z;
+		double bx = 0, by = 0, bz = 0;
+		const FieldJF12 f = model();
+		if (f.p.use_turbulent) {
+			const V3 g = AnyInterp ? grid_interpolate(f.turbulent, pos) : FieldGrid{f.turbulent}.eval(pos);
+			bx += (double)((float)g.x * strength);
+			by += (double)((float)g.y * strength);
+			bz += (double)((float)g.z * strength);
+		}
+		if (f.p.use_striated) {
+			const double s = 1. + f.p.sqrt_beta * (double)scalar_grid_closest(f.striated, pos);
+			bx += r.x * s;
+			by += r.y * s;
+			bz += r.z * s;
+		} else if (f.p.use_regular) {
+			bx += r.x;
+			by += r.y;
+			bz += r.z;
 		}
 		return v3(bx, by, bz);
+	}
+	template <bool AnyInterp> __device__ __forceinline__ V3 eval_impl(const V3 &pos) const {
+		return sum_parts<AnyInterp>(pos, [&]() { return *this; });
 	}
 	// Out of line: one copy serves the six stages of a Cash-Karp step.
 	__device__ __attribute__((noinline)) V3 eval(const V3 &pos) const { return eval_impl<false>(pos); }
@@ -210,6 +274,29 @@ struct FieldJF12Any {
 	__device__ __forceinline__ V3 eval(const V3 &pos) const { return f.eval_any(pos); }
 	__device__ __forceinline__ float3 evalf(const V3 &pos) const {
 		const V3 b = f.eval_any(pos);
+		return make_float3((float)b.x, (float)b.y, (float)b.z);
+	}
+};
+
+// The same fields in the propagation kernels, which read the model's hundred parameters from device memory
+// through scalar loads.  As a kernel argument the model was copied to scratch, since its out-of-line
+// evaluation takes an address, and every parameter came back as a 64-lane scratch load.
+template <bool AnyInterp>
+static __device__ __attribute__((noinline)) V3 jf12_eval(const FieldJF12 *model, const V3 pos) {
+	const uint64_t a = (uint64_t)model; // the same in every lane
+	const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+	                   (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32;
+	return FieldJF12::sum_parts<AnyInterp>(pos, [&]() {
+		uint64_t v = u; // each section loads what it reads: all at once, most of it would be spilled
+		asm volatile("" : "+s"(v));
+		return ld_const((const FieldJF12 *)v);
+	});
+}
+template <bool AnyInterp> struct FieldJF12Ref {
+	const FieldJF12 *model;
+	__device__ __forceinline__ V3 eval(const V3 &pos) const { return jf12_eval<AnyInterp>(model, pos); }
+	__device__ __forceinline__ float3 evalf(const V3 &pos) const {
+		const V3 b = eval(pos);
 		return make_float3((float)b.x, (float)b.y, (float)b.z);
 	}
 };

@@ -68,6 +68,7 @@ struct crp_field {
 	GridDesc grid;
 	GridDesc mod; // FK_MODULATED: the Grid1f modulation, one float per point
 	FieldJF12 jf12; // FK_JF12: parameters and grids
+	mutable FieldJF12 *djf12; // their copy on the device, made by the first propagation (jf12_device)
 	PlaneWaveDesc pw;
 	float *cells; // cell-major corner table (periodic grids), or nullptr
 	unsigned char *cells16; // FP16 corner table with brick scales (mixed path), or nullptr
@@ -760,6 +761,23 @@ static bool grid_tricubic_fits(const GridDesc &g) {
 	return g.interp == kInterpTricubic && (size_t)g.nx * g.ny * g.nz * 12 <= 0xffffffffull;
 }
 
+// the device copy of a JF12 field's parameters
+static int jf12_device(const crp_field *f) {
+	static std::mutex lock;
+	std::lock_guard<std::mutex> g(lock);
+	if (f->djf12)
+		return CRP_OK;
+	FieldJF12 *d = nullptr;
+	CRP_HIP_TRY(hipMalloc((void **)&d, sizeof(FieldJF12)));
+	const hipError_t e = hipMemcpy(d, &f->jf12, sizeof(FieldJF12), hipMemcpyHostToDevice);
+	if (e != hipSuccess) {
+		(void)hipFree(d);
+		return fail(CRP_E_HIP, std::string("crp_propagate: JF12 parameters: ") + hipGetErrorString(e));
+	}
+	f->djf12 = d;
+	return CRP_OK;
+}
+
 // a JF12 field whose turbulent grid is not read trilinear: FieldJF12Any
 static bool jf12_any(const crp_field *f) {
 	return f && f->kind == FK_JF12 && f->jf12.turbulent.interp != kInterpTrilinear;
@@ -1077,6 +1095,11 @@ int crp_field_set_grid_interpolation(crp_field_t *f, int grid, int type) {
 	if (g->interp == type)
 		return CRP_OK;
 	g->interp = type;
+	if (f->kind == FK_JF12 && f->djf12) { // runs in flight read the device copy: the next one makes another
+		CRP_HIP_TRY(hipDeviceSynchronize());
+		CRP_HIP_TRY(hipFree(f->djf12));
+		f->djf12 = nullptr;
+	}
 	if (g != &f->grid)
 		return CRP_OK;
 	if (type == CRP_GRID_TRILINEAR)
@@ -1474,6 +1497,8 @@ int crp_field_destroy(crp_field_t *f) {
 		(void)hipFree(f->cells16);
 	if (f->dcomp)
 		(void)hipFree(f->dcomp);
+	if (f->djf12)
+		(void)hipFree(f->djf12);
 	delete f->hcomp;
 	delete f;
 	return CRP_OK;
@@ -2337,6 +2362,9 @@ int crp_propagate(const crp_propagator_t *p, crp_batch_t *b, long long max_steps
 	}
 	if (int rc0 = field_prepare(p->field)) // a decorator's program, before the timed region
 		return rc0;
+	if (p->field && p->field->kind == FK_JF12)
+		if (int rc0 = jf12_device(p->field))
+			return rc0;
 	CRP_HIP_TRY(hipEventRecord(b->ev0, b->stream));
 	int rc;
 	const crp_field *f = p->field;
@@ -2369,8 +2397,8 @@ int crp_propagate(const crp_propagator_t *p, crp_batch_t *b, long long max_steps
 		              : dispatch_kind(FieldModulated<FieldGrid>{FieldGrid{f->grid}, f->mod}, p, P, b, &st.launches);
 		break;
 	case FK_JF12:
-		rc = jf12_any(f) ? dispatch_kind(FieldJF12Any{f->jf12}, p, P, b, &st.launches)
-		                 : dispatch_kind(f->jf12, p, P, b, &st.launches);
+		rc = jf12_any(f) ? dispatch_kind(FieldJF12Ref<true>{f->djf12}, p, P, b, &st.launches)
+		                 : dispatch_kind(FieldJF12Ref<false>{f->djf12}, p, P, b, &st.launches);
 		break;
 	case FK_COMPOSITE: rc = dispatch_kind(FieldComposite{f->dcomp, 1.0}, p, P, b, &st.launches); break;
 	default: rc = dispatch_kind(FieldNone{}, p, P, b, &st.launches); break;

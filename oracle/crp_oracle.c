@@ -1406,6 +1406,14 @@ void orc_cos_turn_phases(const double *x, size_t n, int sine, double *quick, int
 	}
 }
 
+void orc_sincos_cr(const double *x, size_t n, double *s, double *c) {
+	for (size_t i = 0; i < n; i++) {
+		const crp_dd r = crp_sincos_cr(x[i]);
+		s[i] = r.hi;
+		c[i] = r.lo;
+	}
+}
+
 void orc_pow_phases(const double *x, double y, size_t n, double *quick, int32_t *decided, double *accurate) {
 	for (size_t i = 0; i < n; i++) {
 		decided[i] = crp_pow_quick(x[i], y, crp_logr_tab, crp_exp2_tab, &quick[i]);

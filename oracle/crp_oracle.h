@@ -179,6 +179,7 @@ void orc_sin_log_batch(const double *x, size_t n, double *sin_out, double *log_o
 
 /* the two phases of the correctly rounded cos separately: quick[i] valid where decided[i] != 0 */
 void orc_cos_phases(const double *x, size_t n, double *quick, int32_t *decided, double *accurate);
+void orc_sincos_cr(const double *x, size_t n, double *s, double *c);
 void orc_pow_phases(const double *x, double y, size_t n, double *quick, int32_t *decided, double *accurate);
 void orc_cos_turn_phases(const double *x, size_t n, int sine, double *quick, int32_t *decided, double *accurate);
 

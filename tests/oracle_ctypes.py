@@ -135,6 +135,7 @@ def lib():
         L.orc_noise_grid.argtypes = [C.c_uint32, C.c_int, C.c_int, C.c_int, C.c_double, _fp]
         L.orc_rng_randint_batch.argtypes = [C.c_uint32, C.c_size_t, _P(C.c_uint32)]
         L.orc_cos_phases.argtypes = [_dp, C.c_size_t, _dp, _P(C.c_int32), _dp]
+        L.orc_sincos_cr.argtypes = [_dp, C.c_size_t, _dp, _dp]
         L.orc_pow_phases.argtypes = [_dp, C.c_double, C.c_size_t, _dp, _P(C.c_int32), _dp]
         L.orc_cos_turn_phases.argtypes = [_dp, C.c_size_t, C.c_int, _dp, _P(C.c_int32), _dp]
         L.orc_philox4x32_10.argtypes = [_P(C.c_uint32), _P(C.c_uint32), _P(C.c_uint32)]
@@ -604,6 +605,14 @@ def cos_phases(x):
     d = np.zeros(x.shape, dtype=np.int32)
     lib().orc_cos_phases(ptr(x), x.size, ptr(q), d.ctypes.data_as(_P(C.c_int32)), ptr(a))
     return q, d.astype(bool), a
+
+
+def sincos_cr(x):
+    """(sin, cos) of the joint evaluation, correctly rounded."""
+    x = np.ascontiguousarray(x, dtype=np.float64)
+    s, c = np.zeros_like(x), np.zeros_like(x)
+    lib().orc_sincos_cr(ptr(x), x.size, ptr(s), ptr(c))
+    return s, c
 
 
 def pow_phases(x, y):

@@ -103,6 +103,16 @@ def test_cos_turn_phase_agrees_with_accurate_phase(sine):
     assert not dec[4:].any()
 
 
+def test_sincos_joint_evaluation():
+    rng = np.random.default_rng(23)
+    x = np.concatenate([rng.uniform(-4, 4, 100000), rng.uniform(-1e7, 1e7, 100000), np.linspace(-7, 7, 20001),
+                        np.array([0.0, -0.0, 1e-300, 2.0 ** 30, 1e300, np.inf, -np.inf, np.nan])])
+    s, c = O.sincos_cr(x)
+    for got, sine in ((s, True), (c, False)):
+        want = O.cos_turn_phases(x, sine)[2]
+        assert ((got.view(np.uint64) == want.view(np.uint64)) | (np.isnan(got) & np.isnan(want))).all()
+
+
 @pytest.mark.parametrize("y", [-0.2, 1 / 3., -1.0, 0.9])
 def test_pow_quick_phase_agrees_with_double_double(y):
     """Every value that the quick phase decides equals the double-double one (7e7 arguments checked the same way

@@ -2775,12 +2775,19 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 		CRP_HIP_TRY(hipGetLastError());
 		return CRP_OK;
 	}
-	// stream A (the caller's) runs the reverse sweeps, block after block; stream B the recompute of
-	// the block after (in backward order), stream C the accumulation of the block before: the three
-	// are bound by FP64 issue at one wave per SIMD, the random-line rate of the cell gathers and LDS
-	// atomics respectively
+	// stream A (the caller's) runs the reverse sweeps, block after block, stream C the accumulation of the
+	// block before.  The recompute of the next block goes to a stream of its own, B, where the reverse sweep
+	// leaves half the SIMDs idle or more; where it has a wave on nearly all, the two beside each other take longer
+	// (2.3 ms a block of 65536 particles) than one after the other (1.28 + 0.69), and the recompute runs on
+	// stream A before its sweep, beside the accumulation
 	hipStream_t sb, sc;
 	CRP_HIP_TRY(adj_side_streams(&sb, &sc));
+	const int ncu = num_cus();
+	if (ncu < 0)
+		return CRP_E_HIP;
+	const bool apart = n <= (size_t)ncu * 4 * 64 / 2;
+	if (!apart)
+		sb = sa;
 	AdjEvents E;
 	const int NB = P.nblocks;
 	std::vector<hipEvent_t> recomputed(NB), reversed(NB), sorted(NB);
@@ -2825,7 +2832,8 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 	auto recompute = [&](int b, hipStream_t st) {
 		const AdjBlock Bk = block(b);
 		const size_t nc = (size_t)Bk.npg * T;
-		hipLaunchKernelGGL(k_dep_zero, dim3((unsigned)((nc + kAdjGroup - 1) / kAdjGroup)), dim3(kAdjGroup), 0, st, Bk);
+		if (b >= NB - 2) // a buffer's first block; the reverse sweeps clear the counts for the later ones
+			hipLaunchKernelGGL(k_dep_zero, dim3((unsigned)((nc + kAdjGroup - 1) / kAdjGroup)), dim3(kAdjGroup), 0, st, Bk);
 		const dim3 grid((unsigned)((size_t)Bk.nseg * Bk.npg));
 		if (P.tileShift == 3)
 			hipLaunchKernelGGL((k_adj_recompute<3, kAdjSub>), grid, dim3(kAdjGroup), T * sizeof(uint32_t), st, A, Bk);
@@ -2856,19 +2864,24 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 	CRP_HIP_TRY(hipEventRecord(start, sa));
 	CRP_HIP_TRY(hipStreamWaitEvent(sb, start, 0));
 	CRP_HIP_TRY(hipStreamWaitEvent(sc, start, 0));
-	recompute(NB - 1, sb);
-	CRP_HIP_TRY(hipEventRecord(recomputed[NB - 1], sb));
+	if (apart) {
+		recompute(NB - 1, sb);
+		CRP_HIP_TRY(hipEventRecord(recomputed[NB - 1], sb));
+	}
 	for (int b = NB - 1; b >= 0; b--) {
 		// A: reverse sweep of block b once its sub-checkpoints and counts are there and the accumulation
 		// of block b + 2 (the same record buffer) has read its records
-		CRP_HIP_TRY(hipStreamWaitEvent(sa, recomputed[b], 0));
+		if (apart)
+			CRP_HIP_TRY(hipStreamWaitEvent(sa, recomputed[b], 0));
 		if (b + 2 < NB)
 			CRP_HIP_TRY(hipStreamWaitEvent(sa, sorted[b + 2], 0));
+		if (!apart) // into the buffers that block b + 2 has finished with
+			recompute(b, sa);
 		reverse(b, sa);
 		CRP_HIP_TRY(hipEventRecord(reversed[b], sa));
 		// B: recompute of block b - 1 into the buffers that the reverse sweep of block b + 1 has
 		// finished with (its counts were last read by the accumulation of block b + 1)
-		if (b > 0) {
+		if (apart && b > 0) {
 			if (b + 1 < NB) {
 				CRP_HIP_TRY(hipStreamWaitEvent(sb, reversed[b + 1], 0));
 				CRP_HIP_TRY(hipStreamWaitEvent(sb, sorted[b + 1], 0));

@@ -17,12 +17,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "crp_device.hpp"
@@ -146,6 +148,49 @@ struct crp_batch {
 };
 
 
+// Pinned slots through which field samples and batches cross the bus.  A call takes what it needs and gives
+// it back; at most kSlotsMax stay idle, and all are freed when the last field and batch are destroyed.
+constexpr size_t kSlotBytes = 2u << 20;
+constexpr int kSlotsMax = 8;
+static struct PinnedPool {
+	std::mutex lock;
+	void *idle[kSlotsMax];
+	int nidle = 0, objects = 0;
+
+	void *take() { // nullptr: no pinned memory to be had
+		{
+			std::lock_guard<std::mutex> g(lock);
+			if (nidle > 0)
+				return idle[--nidle];
+		}
+		void *p = nullptr;
+		if (hipHostMalloc(&p, kSlotBytes, hipHostMallocPortable) != hipSuccess) {
+			(void)hipGetLastError();
+			return nullptr;
+		}
+		return p;
+	}
+	void give(void *p) {
+		{
+			std::lock_guard<std::mutex> g(lock);
+			if (objects > 0 && nidle < kSlotsMax) {
+				idle[nidle++] = p;
+				return;
+			}
+		}
+		(void)hipHostFree(p);
+	}
+	void created() {
+		std::lock_guard<std::mutex> g(lock);
+		objects++;
+	}
+	void destroyed() {
+		std::lock_guard<std::mutex> g(lock);
+		if (--objects == 0)
+			while (nidle > 0)
+				(void)hipHostFree(idle[--nidle]);
+	}
+} gPinned;
 
 static Soa soa_of(const crp_batch *b) {
 	Soa s;
@@ -181,6 +226,50 @@ __global__ void __launch_bounds__(256) k_copy_f64(const double *__restrict__ src
 	const size_t stride = (size_t)gridDim.x * blockDim.x;
 	for (; i < n; i += stride)
 		dst[i] = src[i];
+}
+
+// crp_batch_download's gather: particles [first, first + m) of the requested arrays, section after section,
+// into pinned host memory.  A section is 3 arrays interleaved (x, y, z per particle), one array of doubles or
+// one of 4-byte words; consecutive threads write consecutive words, since a store to host memory is one
+// transaction over the bus however few of its bytes it fills.
+struct PackArgs {
+	const double *v3[6][3];
+	const double *d1[6];
+	const uint32_t *w1[3];
+	int n3, n1, nw;
+};
+__global__ void __launch_bounds__(256) k_pack(PackArgs A, size_t first, unsigned m, double *__restrict__ out) {
+	const unsigned t0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+	const int sec = blockIdx.y;
+	if (sec < A.n3) {
+		double *const o = out + (size_t)3 * m * sec;
+		const double *const x = A.v3[sec][0] + first, *const y = A.v3[sec][1] + first, *const z = A.v3[sec][2] + first;
+		for (unsigned t = t0; t < 3 * m; t += stride) {
+			const unsigned i = t / 3, c = t - 3 * i;
+			o[t] = c == 0 ? x[i] : (c == 1 ? y[i] : z[i]);
+		}
+	} else if (sec < A.n3 + A.n1) {
+		double *const o = out + (size_t)3 * m * A.n3 + (size_t)m * (sec - A.n3);
+		const double *const x = A.d1[sec - A.n3] + first;
+		for (unsigned t = t0; t < m; t += stride)
+			o[t] = x[t];
+	} else {
+		uint32_t *const o = (uint32_t *)(out + (size_t)m * (3 * A.n3 + A.n1)) + (size_t)m * (sec - A.n3 - A.n1);
+		const uint32_t *const x = A.w1[sec - A.n3 - A.n1] + first;
+		for (unsigned t = t0; t < m; t += stride)
+			o[t] = x[t];
+	}
+}
+
+// crp_batch_detections' gather: detection k of m particles, 9 doubles each, NaN where it did not happen
+__global__ void __launch_bounds__(256) k_pack_snap(const double *__restrict__ snap, size_t cap,
+                                                   const int32_t *__restrict__ det, int k, unsigned m,
+                                                   double *__restrict__ out) {
+	const unsigned stride = gridDim.x * blockDim.x;
+	for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < m * kSnapDoubles; t += stride) {
+		const unsigned i = t / kSnapDoubles, c = t - i * kSnapDoubles;
+		out[t] = k < det[i] ? snap[c * cap + i] : __builtin_nan("");
+	}
 }
 
 // Cell-major corner table of a periodic grid: cell (x0,y0,z0) stores the values
@@ -311,28 +400,46 @@ __global__ void __launch_bounds__(256) k_build_cells16(const float *__restrict__
 	}
 }
 
-template <class F>
-__global__ void k_field_evalf(F field, const double *__restrict__ pos, double *__restrict__ B, size_t n) {
-	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	V3 p = v3(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]);
-	float3 b = field.evalf(p);
-	B[3 * i] = b.x;
-	B[3 * i + 1] = b.y;
-	B[3 * i + 2] = b.z;
+// Field samples, 256 positions a workgroup.  Positions and values may lie in pinned host memory: they pass
+// through LDS, so that each of their 64-byte pieces crosses the bus once (a lane reading its own 24 bytes
+// would ask for every piece three times).
+template <class F, bool MIX>
+__device__ __forceinline__ void field_eval_block(const F &field, const double *__restrict__ pos, double *__restrict__ B,
+                                                 size_t n) {
+	__shared__ double buf[3 * 256];
+	const size_t first = (size_t)blockIdx.x * 256;
+	const int m = (int)min(n - first, (size_t)256);
+	for (int t = threadIdx.x; t < 3 * m; t += 256)
+		buf[t] = pos[3 * first + t];
+	__syncthreads();
+	double *const mine = buf + 3 * threadIdx.x;
+	if ((int)threadIdx.x < m) {
+		const V3 p = v3(mine[0], mine[1], mine[2]);
+		if (MIX) {
+			const float3 b = field.evalf(p);
+			mine[0] = b.x;
+			mine[1] = b.y;
+			mine[2] = b.z;
+		} else {
+			const V3 b = field.eval(p);
+			mine[0] = b.x;
+			mine[1] = b.y;
+			mine[2] = b.z;
+		}
+	}
+	__syncthreads();
+	for (int t = threadIdx.x; t < 3 * m; t += 256)
+		B[3 * first + t] = buf[t];
 }
-
 template <class F>
-__global__ void k_field_eval(F field, const double *__restrict__ pos, double *__restrict__ B, size_t n) {
-	size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	V3 p = v3(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]);
-	V3 b = field.eval(p);
-	B[3 * i] = b.x;
-	B[3 * i + 1] = b.y;
-	B[3 * i + 2] = b.z;
+__global__ void __launch_bounds__(256) k_field_evalf(F field, const double *__restrict__ pos, double *__restrict__ B,
+                                                     size_t n) {
+	field_eval_block<F, true>(field, pos, B, n);
+}
+template <class F>
+__global__ void __launch_bounds__(256) k_field_eval(F field, const double *__restrict__ pos, double *__restrict__ B,
+                                                    size_t n) {
+	field_eval_block<F, false>(field, pos, B, n);
 }
 
 // The reference's public per-step functions on n phase points (PropagationBP::dY / tryStep,
@@ -665,7 +772,13 @@ static crp_field *new_field(int kind) {
 	std::memset(f, 0, sizeof(*f));
 	f->kind = kind;
 	(void)hipGetDevice(&f->device);
+	gPinned.created();
 	return f;
+}
+// a field whose creation failed
+static void drop_field(crp_field *f) {
+	delete f;
+	gPinned.destroyed();
 }
 
 int crp_field_create_uniform(const double B[3], crp_field_t **out) {
@@ -803,20 +916,20 @@ int crp_field_create_grid3f(const float *values, int nx, int ny, int nz, const d
 		return fail(CRP_E_NOMEM, "crp_field_create_grid3f: out of host memory");
 	int rc = fill_grid_desc(f->grid, nullptr, nx, ny, nz, origin, spacing, reflective, clip_volume);
 	if (rc != CRP_OK) {
-		delete f;
+		drop_field(f);
 		return rc;
 	}
 	size_t bytes = (size_t)nx * ny * nz * 3 * sizeof(float);
 	void *d = nullptr;
 	hipError_t e = hipMalloc(&d, bytes);
 	if (e != hipSuccess) {
-		delete f;
+		drop_field(f);
 		return fail(CRP_E_NOMEM, std::string("crp_field_create_grid3f: hipMalloc: ") + hipGetErrorString(e));
 	}
 	e = hipMemcpy(d, values, bytes, hipMemcpyHostToDevice);
 	if (e != hipSuccess) {
 		(void)hipFree(d);
-		delete f;
+		drop_field(f);
 		return fail(CRP_E_HIP, std::string("crp_field_create_grid3f: hipMemcpy: ") + hipGetErrorString(e));
 	}
 	f->grid.values = (const float *)d;
@@ -834,7 +947,7 @@ int crp_field_create_grid3f_device(const float *d_values, int nx, int ny, int nz
 		return fail(CRP_E_NOMEM, "crp_field_create_grid3f_device: out of host memory");
 	int rc = fill_grid_desc(f->grid, d_values, nx, ny, nz, origin, spacing, reflective, clip_volume);
 	if (rc != CRP_OK) {
-		delete f;
+		drop_field(f);
 		return rc;
 	}
 	*out = f;
@@ -1326,6 +1439,30 @@ static hipError_t launch_field_eval(const crp_field_t *f, const double *dpos, do
 	return hipGetLastError();
 }
 
+// Field samples through a pinned slot: the kernel reads the positions and writes the values over the bus, so
+// a call is one launch and one wait (two allocations, two copies and two frees around the launch took 38 us
+// for 1000 positions, this
+// takes EVAL_US).  On the null stream, as the copies were.
+static int eval_staged(const crp_field_t *f, const double *pos, size_t n, double *B, int precision, double *slot) {
+	constexpr size_t kMost = kSlotBytes / (6 * sizeof(double));
+	hipError_t e = hipSuccess;
+	for (size_t i0 = 0; i0 < n && e == hipSuccess; i0 += kMost) {
+		const size_t m = std::min(kMost, n - i0);
+		double *const out = slot + 3 * m;
+		std::memcpy(slot, pos + 3 * i0, 3 * m * sizeof(double));
+		e = launch_field_eval(f, slot, out, m, precision);
+		const hipError_t w = hipStreamSynchronize(0);
+		if (e == hipSuccess)
+			e = w;
+		if (e == hipSuccess)
+			std::memcpy(B + 3 * i0, out, 3 * m * sizeof(double));
+	}
+	gPinned.give(slot);
+	if (e != hipSuccess)
+		return fail(CRP_E_HIP, std::string("crp_field_eval: ") + hipGetErrorString(e));
+	return CRP_OK;
+}
+
 int crp_field_eval_ex(const crp_field_t *f, const double *pos, size_t n, double *B, int precision) {
 	if (precision == CRP_PRECISION_FP64)
 		return crp_field_eval(f, pos, n, B);
@@ -1337,6 +1474,8 @@ int crp_field_eval_ex(const crp_field_t *f, const double *pos, size_t n, double 
 		return CRP_OK;
 	if (int rc = field_prepare(f))
 		return rc;
+	if (void *slot = gPinned.take())
+		return eval_staged(f, pos, n, B, CRP_PRECISION_MIXED, (double *)slot);
 	double *dpos = nullptr, *dB = nullptr;
 	CRP_HIP_TRY(hipMalloc(&dpos, 3 * n * sizeof(double)));
 	hipError_t e = hipMalloc(&dB, 3 * n * sizeof(double));
@@ -1469,7 +1608,7 @@ int crp_field_create_planewave(int nm, const double *k, const double *Ak, const 
 				(void)hipFree(d);
 			for (int i = 0; i < j; i++)
 				(void)hipFree(f->owned[i]);
-			delete f;
+			drop_field(f);
 			return fail(CRP_E_HIP, std::string("crp_field_create_planewave: ") + hipGetErrorString(e));
 		}
 		f->owned[j] = d;
@@ -1500,7 +1639,7 @@ int crp_field_destroy(crp_field_t *f) {
 	if (f->djf12)
 		(void)hipFree(f->djf12);
 	delete f->hcomp;
-	delete f;
+	drop_field(f);
 	return CRP_OK;
 }
 
@@ -1516,7 +1655,7 @@ static int new_composite(int deco, crp_field_t **out, crp_field **res) {
 		if (e == hipSuccess)
 			(void)hipFree(f->dcomp);
 		delete f->hcomp;
-		delete f;
+		drop_field(f);
 		return fail(CRP_E_NOMEM, "field decorator: device or host memory");
 	}
 	std::memset(f->hcomp, 0xff, sizeof(CompositeDesc)); // differs from any program: the first use uploads
@@ -1740,6 +1879,8 @@ int crp_field_eval(const crp_field_t *f, const double *pos, size_t n, double *B)
 		return CRP_OK;
 	if (int rc = field_prepare(f))
 		return rc;
+	if (void *slot = gPinned.take())
+		return eval_staged(f, pos, n, B, CRP_PRECISION_FP64, (double *)slot);
 	double *dpos = nullptr, *dB = nullptr;
 	CRP_HIP_TRY(hipMalloc(&dpos, 3 * n * sizeof(double)));
 	hipError_t e = hipMalloc(&dB, 3 * n * sizeof(double));
@@ -2080,6 +2221,7 @@ int crp_batch_create(size_t capacity, crp_batch_t **out) {
 		delete b;
 		return fail(CRP_E_HIP, std::string("crp_batch_create: ") + hipGetErrorString(e));
 	}
+	gPinned.created();
 	*out = b;
 	return CRP_OK;
 }
@@ -2099,6 +2241,7 @@ int crp_batch_destroy(crp_batch_t *b) {
 	if (b->rows)
 		(void)hipFree(b->rows);
 	delete b;
+	gPinned.destroyed();
 	return CRP_OK;
 }
 
@@ -2194,39 +2337,96 @@ int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 	const size_t n = b->n;
 	if (n == 0)
 		return CRP_OK;
-	CRP_HIP_TRY(hipStreamSynchronize(b->stream));
-	std::vector<double> tmp(n);
-	const double *src3[12] = {b->px, b->py, b->pz, b->dx, b->dy, b->dz, b->ppx, b->ppy, b->ppz, b->pdx, b->pdy, b->pdz};
-	double *dstv[4] = {s->pos, s->dir, s->prev_pos, s->prev_dir};
-	for (int c = 0; c < 12; c++) {
-		double *dst = dstv[c / 3];
-		if (!dst)
-			continue;
-		CRP_HIP_TRY(hipMemcpy(tmp.data(), src3[c], n * sizeof(double), hipMemcpyDeviceToHost));
-		for (size_t i = 0; i < n; i++)
-			dst[3 * i + (c % 3)] = tmp[i];
-	}
+	// The arrays cross the bus packed by k_pack: one launch and one wait per chunk of particles instead of a
+	// copy, a wait and a strided host loop per array.  The host's part, filling fresh pages of the caller's
+	// arrays, is the slow one (about 5 GB/s a thread), so large batches are taken by several threads, each
+	// with a slot and the next chunk.
+	PackArgs A;
+	std::memset(&A, 0, sizeof(A));
+	const double *src3[6][3] = {{b->px, b->py, b->pz},    {b->dx, b->dy, b->dz}, {b->ppx, b->ppy, b->ppz},
+	                            {b->pdx, b->pdy, b->pdz}, {b->sx, b->sy, b->sz}, {b->cx, b->cy, b->cz}};
+	double *const want3[6] = {s->pos, s->dir, s->prev_pos, s->prev_dir, s->source_pos, s->created_pos};
 	const double *src1[6] = {b->E, b->q, b->cur, b->next, b->len, b->time};
-	double *dst1[6] = {s->energy, s->charge, s->current_step, s->next_step, s->trajectory_length, s->time};
-	for (int c = 0; c < 6; c++)
-		if (dst1[c])
-			CRP_HIP_TRY(hipMemcpy(dst1[c], src1[c], n * sizeof(double), hipMemcpyDeviceToHost));
-	if (s->active)
-		CRP_HIP_TRY(hipMemcpy(s->active, b->active, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-	if (s->detection_index)
-		CRP_HIP_TRY(hipMemcpy(s->detection_index, b->det, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-	if (s->sde_step)
-		CRP_HIP_TRY(hipMemcpy(s->sde_step, b->sdeStep, n * sizeof(uint32_t), hipMemcpyDeviceToHost));
-	const double *srcv[6] = {b->sx, b->sy, b->sz, b->cx, b->cy, b->cz};
-	double *dstv2[2] = {s->source_pos, s->created_pos};
-	for (int c = 0; c < 6; c++) {
-		double *dst = dstv2[c / 3];
-		if (!dst)
-			continue;
-		CRP_HIP_TRY(hipMemcpy(tmp.data(), srcv[c], n * sizeof(double), hipMemcpyDeviceToHost));
-		for (size_t i = 0; i < n; i++)
-			dst[3 * i + (c % 3)] = tmp[i];
+	double *const want1[6] = {s->energy, s->charge, s->current_step, s->next_step, s->trajectory_length, s->time};
+	const void *srcw[3] = {b->active, b->det, b->sdeStep};
+	void *const wantw[3] = {s->active, s->detection_index, s->sde_step};
+	double *dst3[6], *dst1[6];
+	char *dstw[3];
+	for (int k = 0; k < 6; k++)
+		if (want3[k]) {
+			std::memcpy(A.v3[A.n3], src3[k], sizeof(src3[k]));
+			dst3[A.n3++] = want3[k];
+		}
+	for (int k = 0; k < 6; k++)
+		if (want1[k]) {
+			A.d1[A.n1] = src1[k];
+			dst1[A.n1++] = want1[k];
+		}
+	for (int k = 0; k < 3; k++)
+		if (wantw[k]) {
+			A.w1[A.nw] = (const uint32_t *)srcw[k];
+			dstw[A.nw++] = (char *)wantw[k];
+		}
+	const size_t per = 8 * (size_t)(3 * A.n3 + A.n1) + 4 * (size_t)A.nw; // bytes of a particle
+	if (per == 0) {
+		CRP_HIP_TRY(hipStreamSynchronize(b->stream));
+		return CRP_OK;
 	}
+	const size_t chunk = std::min(n, kSlotBytes / per), nchunk = (n + chunk - 1) / chunk;
+	const unsigned cpus = std::max(1u, std::thread::hardware_concurrency());
+	const int nthread = (int)std::min<size_t>(std::min<size_t>(kSlotsMax, cpus), (nchunk + 1) / 2);
+	std::atomic<size_t> nextChunk{0};
+	std::atomic<int> err{(int)hipSuccess};
+	auto worker = [&](int w) {
+		double *const slot = (double *)gPinned.take();
+		hipEvent_t ev = nullptr;
+		hipError_t e = slot ? hipSetDevice(b->device) : hipErrorOutOfMemory;
+		if (e == hipSuccess)
+			e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+		const bool ready = e == hipSuccess;
+		for (size_t c; e == hipSuccess && (c = nextChunk++) < nchunk;) {
+			const size_t i0 = c * chunk, m = std::min(chunk, n - i0);
+			const unsigned blocks = (unsigned)std::min<size_t>(256, (3 * m + 255) / 256);
+			hipLaunchKernelGGL(k_pack, dim3(blocks, A.n3 + A.n1 + A.nw), dim3(256), 0, b->stream, A, i0, (unsigned)m, slot);
+			e = hipGetLastError();
+			if (e == hipSuccess)
+				e = hipEventRecord(ev, b->stream);
+			if (e == hipSuccess)
+				e = hipEventSynchronize(ev);
+			if (e != hipSuccess)
+				break;
+			const double *p = slot;
+			for (int k = 0; k < A.n3; k++, p += 3 * m)
+				std::memcpy(dst3[k] + 3 * i0, p, 3 * m * sizeof(double));
+			for (int k = 0; k < A.n1; k++, p += m)
+				std::memcpy(dst1[k] + i0, p, m * sizeof(double));
+			const char *pw = (const char *)p;
+			for (int k = 0; k < A.nw; k++, pw += 4 * m)
+				std::memcpy(dstw[k] + 4 * i0, pw, 4 * m);
+		}
+		if (ev)
+			(void)hipEventDestroy(ev);
+		if (e != hipSuccess && ready)
+			(void)hipStreamSynchronize(b->stream); // nothing writes to the slot any more
+		if (slot)
+			gPinned.give(slot);
+		if (e != hipSuccess && (ready || w == 0)) // a helper that could not start leaves its chunks to the others
+			err = (int)e;
+	};
+	int caller = 0;
+	CRP_HIP_TRY(hipGetDevice(&caller));
+	std::vector<std::thread> team;
+	try {
+		for (int w = 1; w < nthread; w++)
+			team.emplace_back(worker, w);
+	} catch (...) { // no more threads: those there are take all chunks
+	}
+	worker(0);
+	for (std::thread &t : team)
+		t.join();
+	CRP_HIP_TRY(hipSetDevice(caller));
+	if (err != (int)hipSuccess)
+		return fail(CRP_E_HIP, std::string("crp_batch_download: ") + hipGetErrorString((hipError_t)err.load()));
 	return CRP_OK;
 }
 
@@ -2251,20 +2451,28 @@ int crp_batch_detections(const crp_batch_t *b, int ntimes, double *out) {
 	const size_t n = b->n;
 	if (n == 0 || ntimes == 0)
 		return CRP_OK;
-	CRP_HIP_TRY(hipStreamSynchronize(b->stream));
-	std::vector<int32_t> det(n);
-	CRP_HIP_TRY(hipMemcpy(det.data(), b->det, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-	std::fill(out, out + (size_t)ntimes * n * kSnapDoubles, NAN);
 	const int kk = std::min(ntimes, b->snap ? b->snapK : 0);
-	std::vector<double> col(n);
-	for (int k = 0; k < kk; k++)
-		for (int c = 0; c < kSnapDoubles; c++) {
-			CRP_HIP_TRY(hipMemcpy(col.data(), b->snap + ((size_t)k * kSnapDoubles + c) * b->cap, n * sizeof(double),
-			                      hipMemcpyDeviceToHost));
-			for (size_t i = 0; i < n; i++)
-				if (k < det[i])
-					out[((size_t)k * n + i) * kSnapDoubles + c] = col[i];
+	const size_t rec = kSnapDoubles * sizeof(double), chunk = std::min(n, kSlotBytes / rec);
+	double *const slot = (double *)gPinned.take();
+	if (!slot)
+		return fail(CRP_E_NOMEM, "crp_batch_detections: no pinned memory");
+	hipError_t e = hipSuccess;
+	for (int k = 0; k < kk && e == hipSuccess; k++)
+		for (size_t i0 = 0; i0 < n && e == hipSuccess; i0 += chunk) {
+			const size_t m = std::min(chunk, n - i0);
+			const unsigned blocks = (unsigned)std::min<size_t>(1024, (m * kSnapDoubles + 255) / 256);
+			hipLaunchKernelGGL(k_pack_snap, dim3(blocks), dim3(256), 0, b->stream,
+			                   b->snap + (size_t)k * kSnapDoubles * b->cap + i0, b->cap, b->det + i0, k, (unsigned)m, slot);
+			e = hipGetLastError();
+			if (e == hipSuccess)
+				e = hipStreamSynchronize(b->stream);
+			if (e == hipSuccess)
+				std::memcpy(out + ((size_t)k * n + i0) * kSnapDoubles, slot, m * rec);
 		}
+	gPinned.give(slot);
+	if (e != hipSuccess)
+		return fail(CRP_E_HIP, std::string("crp_batch_detections: ") + hipGetErrorString(e));
+	std::fill(out + (size_t)kk * n * kSnapDoubles, out + (size_t)ntimes * n * kSnapDoubles, NAN);
 	return CRP_OK;
 }
 

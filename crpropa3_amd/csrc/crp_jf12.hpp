@@ -16,22 +16,22 @@ constexpr double kJPi = 3.14159265358979323846;
 // exp and atan2 for the arguments that their quick phases leave open
 static __device__ __attribute__((noinline)) double jf12_exp(double x) { return crp_exp_rn(x); }
 static __device__ __attribute__((noinline)) double jf12_atan2(double y, double x) { return crp_atan2_rn(y, x); }
-// five exponentials side by side, one copy of the code
-struct Exp5 {
-	double a, b, c, d, e;
+// four exponentials side by side, one copy of the code
+struct Exp4 {
+	double a, b, c, d;
 };
-static __device__ __attribute__((noinline)) Exp5 jf12_exp5(double a, double b, double c, double d, double e) {
-	const double x[5] = {a, b, c, d, e};
-	double v[5];
-	bool ok[5];
+static __device__ __attribute__((noinline)) Exp4 jf12_exp4(double a, double b, double c, double d) {
+	const double x[4] = {a, b, c, d};
+	double v[4];
+	bool ok[4];
 #pragma unroll
-	for (int i = 0; i < 5; i++)
+	for (int i = 0; i < 4; i++)
 		ok[i] = crp_exp_quick(x[i], &v[i]) && x[i] >= -708.0 && x[i] <= 708.0;
 #pragma unroll
-	for (int i = 0; i < 5; i++)
+	for (int i = 0; i < 4; i++)
 		if (!ok[i])
 			v[i] = jf12_exp(x[i]);
-	return Exp5{v[0], v[1], v[2], v[3], v[4]};
+	return Exp4{v[0], v[1], v[2], v[3]};
 }
 
 // Grid<float>::closestValue (include/crpropa/Grid.h:383-405): nearest point, reflective or periodic
@@ -51,10 +51,11 @@ struct FieldJF12 {
 	}
 
 	// What an evaluation takes from the position: the transcendental functions of every part, each correctly
-	// rounded.  They are formed side by side, whether or not this position's branches read all of them: a
-	// batch has about one wave to a SIMD, where every instruction waits for the one before, and two azimuths,
-	// two sines and cosines and ten exponentials one after the other were most of an evaluation.
-	enum { E_DISK, E_HALO, E_HALO_R, E_X, E_TURB_DISK, E_TURB_R, E_TURB_HALO, E_ARM0, E_ARM1, E_ARM2, E_COUNT };
+	// rounded.  The azimuth, its sine and cosine and the eight exponentials that most positions read are formed
+	// side by side, whether or not this one reads all of them: a batch has about one wave to a SIMD, where every
+	// instruction waits for the one before.  The angle inside rc and the other two windings are left to the
+	// positions that have them.
+	enum { E_DISK, E_HALO, E_HALO_R, E_X, E_TURB_DISK, E_TURB_R, E_TURB_HALO, E_ARM, E_COUNT };
 	struct Geo {
 		double d, r, rn, rc, rp;
 		double sinPhi, cosPhi, sinThetaX, cosThetaX;
@@ -75,16 +76,13 @@ struct FieldJF12 {
 		const double tx = g.r - g.rp;
 		double phi = 0, theta = 0;
 		const bool okPhi = pos.x == pos.x && pos.y == pos.y && pos.x != 0 && pos.y != 0 && crp_atan2_quick(pos.y, pos.x, &phi);
-		const bool okTheta = az == az && tx == tx && az != 0 && tx != 0 && crp_atan2_quick(az, tx, &theta);
 		if (!okPhi && !axis)
 			phi = jf12_atan2(pos.y, pos.x);
 		if (axis)
 			phi = 0.0;
 		const bool useTheta = p.use_x && inner && g.r * g.r + z * z > 1 * kJKpc * kJKpc;
-		if (!okTheta && useTheta && z != 0)
-			theta = jf12_atan2(az, tx);
-		if (z == 0)
-			theta = kJPi / 2.;
+		if (useTheta)
+			theta = z == 0 ? kJPi / 2. : jf12_atan2(az, tx);
 		// exponentials
 		double x[E_COUNT];
 		x[E_DISK] = logistic_arg(z, p.h_disk, p.w_disk);
@@ -94,32 +92,30 @@ struct FieldJF12 {
 		x[E_TURB_DISK] = p.use_turbulent ? -0.5 * sq(z / p.z_disk_turb) : 0.0;
 		x[E_TURB_R] = p.use_turbulent ? -g.r / p.r_halo_turb : 0.0;
 		x[E_TURB_HALO] = p.use_turbulent ? -0.5 * sq(z / p.z_halo_turb) : 0.0;
-		x[E_ARM0] = -(phi - kJPi) / p.tan90_minus_pitch;
-		x[E_ARM1] = -(phi + kJPi) / p.tan90_minus_pitch;
-		x[E_ARM2] = -(phi + 3 * kJPi) / p.tan90_minus_pitch;
-		const Exp5 e0 = jf12_exp5(x[0], x[1], x[2], x[3], x[4]), e1 = jf12_exp5(x[5], x[6], x[7], x[8], x[9]);
-		const double e[E_COUNT] = {e0.a, e0.b, e0.c, e0.d, e0.e, e1.a, e1.b, e1.c, e1.d, e1.e};
+		x[E_ARM] = -(phi - kJPi) / p.tan90_minus_pitch;
+		const Exp4 e0 = jf12_exp4(x[0], x[1], x[2], x[3]), e1 = jf12_exp4(x[4], x[5], x[6], x[7]);
+		const double e[E_COUNT] = {e0.a, e0.b, e0.c, e0.d, e1.a, e1.b, e1.c, e1.d};
 #pragma unroll
 		for (int i = 0; i < E_COUNT; i++)
 			g.e[i] = e[i];
 		const bool okP = crp_sincos_turn(phi, &g.sinPhi, &g.cosPhi);
-		const bool okT = crp_sincos_turn(theta, &g.sinThetaX, &g.cosThetaX);
+		g.sinThetaX = g.cosThetaX = 0;
+		if (useTheta) {
+			const crp_dd sc = crp_sincos_cr(theta);
+			g.sinThetaX = sc.hi;
+			g.cosThetaX = sc.lo;
+		}
 		if (!okP) {
 			const crp_dd sc = crp_sincos_cr(phi);
 			g.sinPhi = sc.hi;
 			g.cosPhi = sc.lo;
 		}
-		if (!okT) {
-			const crp_dd sc = crp_sincos_cr(theta);
-			g.sinThetaX = sc.hi;
-			g.cosThetaX = sc.lo;
-		}
 		// radius where the arm through (r, phi) crosses the negative x-axis, tried for three windings
-		g.rn = g.r * g.e[E_ARM0];
+		g.rn = g.r * g.e[E_ARM];
 		if (g.rn > p.r_arms[7])
-			g.rn = g.r * g.e[E_ARM1];
+			g.rn = g.r * jf12_exp(-(phi + kJPi) / p.tan90_minus_pitch);
 		if (g.rn > p.r_arms[7])
-			g.rn = g.r * g.e[E_ARM2];
+			g.rn = g.r * jf12_exp(-(phi + 3 * kJPi) / p.tan90_minus_pitch);
 		return g;
 	}
 

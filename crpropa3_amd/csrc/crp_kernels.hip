@@ -542,6 +542,13 @@ static auto propagate_kernel() {
 		return k_propagate<F, KIND, MIX>;
 }
 
+template <class F> struct BigCode {
+	static constexpr bool value = false;
+};
+template <bool Any> struct BigCode<FieldJF12Ref<Any>> {
+	static constexpr bool value = true;
+};
+
 template <class F, int KIND, bool MIX>
 static int launch_propagate(const F &f, const crp_propagator *p, const Params &Pin, crp_batch *b, int *launches) {
 	auto kern = propagate_kernel<F, KIND, MIX>();
@@ -561,9 +568,20 @@ static int launch_propagate(const F &f, const crp_propagator *p, const Params &P
 	// `lanes` particles: every particle is one serial chain, and a wave with fewer of them waits for fewer
 	// lines per load and fewer rare branches.
 	constexpr size_t group = KIND == PK_SDE ? 1 : LaneGroup<typename KernelField<F, MIX>::type>::value;
-	const size_t waves = std::min<size_t>((size_t)ncu * bpc * (block / 64), (size_t)ncu * 4);
+	// Field types whose code crowds the instruction cache that two CUs share run better with fewer waves there:
+	// these get one wave to a CU, and two and four once all have 64 particles (JF12, 64 to 8192 particles: 46 us
+	// a step with one wave to a CU, 76 to 104 with four; 65536 fill four, 42 us).
+	const int perBlockWaves = block / 64;
+	int perCU = 4;
+	if (BigCode<F>::value) {
+		perCU = 1;
+		while (perCU < 4 && (size_t)ncu * perCU * 64 < b->n)
+			perCU *= 2;
+	}
+	const int active = std::min(perBlockWaves, perCU); // waves of a workgroup that take particles
+	const size_t waves = std::min<size_t>((size_t)ncu * bpc * active, (size_t)ncu * perCU);
 	const int lanes = (int)std::min<size_t>(64, group * std::max<size_t>(1, (b->n + waves - 1) / waves));
-	const size_t perBlock = (size_t)lanes / group * (block / 64);
+	const size_t perBlock = (size_t)lanes / group * active;
 	const size_t want = (b->n + perBlock - 1) / perBlock;
 	const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(want, (size_t)ncu * bpc));
 	p->lastGrid = grid;
@@ -571,6 +589,7 @@ static int launch_propagate(const F &f, const crp_propagator *p, const Params &P
 	p->lastPPL = (double)b->n / ((double)grid * block);
 	Params P0 = Pin;
 	P0.lanes = lanes;
+	P0.waves = active;
 	const Soa soa = soa_of(b);
 	const unsigned long long n = b->n;
 	const long long M = P0.maxSteps, S = p->stepsPerLaunch;
@@ -1441,8 +1460,8 @@ static hipError_t launch_field_eval(const crp_field_t *f, const double *dpos, do
 
 // Field samples through a pinned slot: the kernel reads the positions and writes the values over the bus, so
 // a call is one launch and one wait (two allocations, two copies and two frees around the launch took 38 us
-// for 1000 positions, this
-// takes EVAL_US).  On the null stream, as the copies were.
+// for 1000 positions, this takes
+// 22).  On the null stream, as the copies were.
 static int eval_staged(const crp_field_t *f, const double *pos, size_t n, double *B, int precision, double *slot) {
 	constexpr size_t kMost = kSlotBytes / (6 * sizeof(double));
 	hipError_t e = hipSuccess;

@@ -75,8 +75,8 @@ struct Params {
 	const SdeAdvTerm *sdeAdvTerms;
 	int sdeAdvection;
 	uint32_t sdeSeed;
-	// lanes of a wave that take particles (launch_propagate)
-	int lanes;
+	// lanes of a wave, and waves of a workgroup, that take particles (launch_propagate)
+	int lanes, waves;
 	int sdeMaxHalvings; // trials beyond this many halvings stop the particle (CTR_SDE_LIMIT)
 };
 
@@ -140,7 +140,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 	constexpr int kGroup = LaneGroup<typename KernelField<F, MIX>::type>::value;
 	const bool first = lane % kGroup == 0;
 
-	bool have = false, exhausted = lane >= P.lanes, inProc = false;
+	bool have = false, exhausted = lane >= P.lanes || (int)(threadIdx.x >> 6) >= P.waves, inProc = false;
 	CkB0Store<FloatValuedField<typename KernelField<F, MIX>::type>::value> b0; // the field at the trial sequence's start (adaptive CK), for retries
 	CkB0f b0f;
 	b0.have = false;

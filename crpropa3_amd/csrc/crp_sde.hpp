@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(256) k_sde(F field0, Params P, Soa S, unsigned
 	const double cosHalfPi = crp_cos_cr(3.14159265358979323846 / 2.);
 	const double minTime = P.minStep / kCLight; // minStep / c_light of the trial loop's test
 
-	bool have = false, exhausted = lane >= P.lanes;
+	bool have = false, exhausted = lane >= P.lanes || (int)(threadIdx.x >> 6) >= P.waves;
 	unsigned idx = 0;
 	long long steps = 0;
 	int phase = SDE_BEGIN;

@@ -83,6 +83,34 @@ def test_jf12_trajectories_bit_exact_vs_oracle(launch):
         assert np.mean(rel < 1e-9) >= near[si], si
 
 
+@pytest.mark.parametrize("n,block", [(1, 256), (64, 256), (257, 64), (8193, 128), (16384, 256), (16385, 256), (32769, 256),
+                                     (16385, 64)])
+def test_jf12_batches_spread_over_compute_units(n, block):
+    """A particle's steps do not depend on how many waves of a workgroup and lanes of a wave the batch takes (one
+    wave to a compute unit up to 64 particles each, then two and four), at positions on the plane and the axis, inside
+    and outside the X field's inner cone, and with arm radii of every winding."""
+    rng = np.random.default_rng(17)
+    m = 512
+    dev, orc = fields(O.load_case("jf12"), "full")
+    r, phi = 10 ** rng.uniform(-1, np.log10(25), m), rng.uniform(-np.pi, np.pi, m)
+    pos = np.stack([r * np.cos(phi), r * np.sin(phi), rng.normal(size=m) * 3], axis=1) * O.kpc
+    pos[::7, 2] = 0.0
+    pos[3::31, :2] = 0.0
+    d, E, q = rng.normal(size=(m, 3)), 10 ** rng.uniform(0, 2, m) * O.EeV, np.full(m, -O.eplus)
+    ref = O.OracleState(pos, d, E, q)
+    O.propagate(orc, O.PROP_CK, ref, 4, tolerance=1e-4, min_step=0.1 * O.pc, max_step=100 * O.pc, libm=O.LIBM_CR)
+    i = np.arange(n) % m
+    b = capi.Batch(n)
+    b.upload(pos[i], O.normalise(d)[i], E[i], q[i])
+    p = capi.Propagator("CK", dev, 1e-4, 0.1 * O.pc, 100 * O.pc)
+    p.set_launch(block=block)
+    st = p.propagate(b, max_steps=4)
+    out = b.download()
+    assert st.accepted_steps == 4 * n
+    for key in ("pos", "dir", "next_step", "trajectory_length"):
+        assert bits_equal(out[key], getattr(ref, key)[i]), key
+
+
 def test_python_jf12_classes():
     """JF12Field / PlanckJF12bField from Python: getField and the parts equal the C-ABI field; a
     ModuleList run with PropagationCK equals the oracle"""

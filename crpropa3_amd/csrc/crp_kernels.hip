@@ -542,13 +542,6 @@ static auto propagate_kernel() {
 		return k_propagate<F, KIND, MIX>;
 }
 
-template <class F> struct BigCode {
-	static constexpr bool value = false;
-};
-template <bool Any> struct BigCode<FieldJF12Ref<Any>> {
-	static constexpr bool value = true;
-};
-
 template <class F, int KIND, bool MIX>
 static int launch_propagate(const F &f, const crp_propagator *p, const Params &Pin, crp_batch *b, int *launches) {
 	auto kern = propagate_kernel<F, KIND, MIX>();
@@ -564,23 +557,21 @@ static int launch_propagate(const F &f, const crp_propagator *p, const Params &P
 	if (bpcMax < 1)
 		bpcMax = 1;
 	const int bpc = p->blocksPerCU > 0 ? std::min(p->blocksPerCU, bpcMax) : bpcMax;
-	// A batch of fewer particles than the chip's SIMDs have lanes is spread over all of them, a wave taking
+	// A batch of fewer particles than the chip's SIMDs have lanes is spread over them, a wave taking
 	// `lanes` particles: every particle is one serial chain, and a wave with fewer of them waits for fewer
-	// lines per load and fewer rare branches.
+	// lines per load and fewer rare branches.  Waves of fewer than 16 particles slow each other down on a compute
+	// unit (8192 particles in waves of 8, four to a unit: a Cash-Karp step takes 76 us in JF12 and 32 in a grid,
+	// in waves of 16 41 and 22; 64 particles one to a wave: 104 us in JF12, 46 with one wave to a unit): below 16
+	// particles to a unit, each has one wave, and from there on waves of 16 or more (2048 particles: the grid's
+	// step 49 us with one wave to a unit, 53 in waves of 16; plane waves 11 and 14; at 4096 10.8 and 9.1).
+	// Groups of lanes on a particle always fill their waves (1000 particles, a tricubic Boris step: 3.1 us, 3.6
+	// with fewer).
 	constexpr size_t group = KIND == PK_SDE ? 1 : LaneGroup<typename KernelField<F, MIX>::type>::value;
-	// Field types whose code crowds the instruction cache that two CUs share run better with fewer waves there:
-	// these get one wave to a CU, and two and four once all have 64 particles (JF12, 64 to 8192 particles: 46 us
-	// a step with one wave to a CU, 76 to 104 with four; 65536 fill four, 42 us).
-	const int perBlockWaves = block / 64;
-	int perCU = 4;
-	if (BigCode<F>::value) {
-		perCU = 1;
-		while (perCU < 4 && (size_t)ncu * perCU * 64 < b->n)
-			perCU *= 2;
-	}
-	const int active = std::min(perBlockWaves, perCU); // waves of a workgroup that take particles
-	const size_t waves = std::min<size_t>((size_t)ncu * bpc * active, (size_t)ncu * perCU);
-	const int lanes = (int)std::min<size_t>(64, group * std::max<size_t>(1, (b->n + waves - 1) / waves));
+	const bool lone = group == 1 && b->n < (size_t)ncu * 16;
+	const int active = lone ? 1 : block / 64; // waves of a workgroup that take particles
+	const size_t waves = std::min<size_t>((size_t)ncu * bpc * active, (size_t)ncu * (lone ? 1 : 4));
+	const size_t least = lone ? 1 : 16;
+	const int lanes = (int)std::min<size_t>(64, group * std::max<size_t>(least, (b->n + waves - 1) / waves));
 	const size_t perBlock = (size_t)lanes / group * active;
 	const size_t want = (b->n + perBlock - 1) / perBlock;
 	const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>(want, (size_t)ncu * bpc));

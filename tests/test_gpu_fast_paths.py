@@ -94,7 +94,7 @@ def test_mirror_fold(shape):
     assert same(capi.Field.grid3f(g, o, sp, reflective=True).eval(pos), want)
 
 
-@pytest.mark.parametrize("n", [1, 5, 63, 1023, 1025, 4097, 66000])
+@pytest.mark.parametrize("n", [1, 5, 63, 1023, 1025, 4095, 4096, 4097, 66000])
 @pytest.mark.parametrize("kind", ["BP", "CK"])
 def test_spread_batches(kind, n):
     """A particle's steps do not depend on how many share its wave."""

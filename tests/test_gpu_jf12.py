@@ -83,11 +83,11 @@ def test_jf12_trajectories_bit_exact_vs_oracle(launch):
         assert np.mean(rel < 1e-9) >= near[si], si
 
 
-@pytest.mark.parametrize("n,block", [(1, 256), (64, 256), (257, 64), (8193, 128), (16384, 256), (16385, 256), (32769, 256),
-                                     (16385, 64)])
+@pytest.mark.parametrize("n,block", [(1, 256), (64, 256), (257, 64), (4095, 256), (4096, 256), (4097, 128), (16385, 256),
+                                     (32769, 64)])
 def test_jf12_batches_spread_over_compute_units(n, block):
     """A particle's steps do not depend on how many waves of a workgroup and lanes of a wave the batch takes (one
-    wave to a compute unit up to 64 particles each, then two and four), at positions on the plane and the axis, inside
+    wave to a compute unit below 16 particles each, waves of 16 and more from there on), at positions on the plane and the axis, inside
     and outside the X field's inner cone, and with arm radii of every winding."""
     rng = np.random.default_rng(17)
     m = 512

@@ -324,10 +324,11 @@ __global__ void __launch_bounds__(256) k_adjoint_backward(AdjArgs A) {
 // The checkpointed backward above walks every particle's segments one after the other: each
 // segment's recompute and reverse sweep wait on one gather per step at one wave per SIMD, and
 // every reverse step adds 24 FP64 atomics into the grid gradient.  The blocked backward instead
-//   1. recomputes a block of segments of every particle at once (segments x n independent lanes),
-//      stores the state (x, u) before every kAdjSub-th step of the block (sub-checkpoints, 6 doubles
-//      per kAdjSub steps) and counts, per workgroup, the steps whose half-step position falls in each
-//      tile of 2^S cells per axis;
+//   1. takes the state (x, u) before every kAdjSub-th step of the block (sub-checkpoints, 6 doubles
+//      per kAdjSub steps) and, per particle group, the number of steps whose half-step position falls in
+//      each tile of 2^S cells per axis.  The forward keeps both where all of them fit the buffer budget
+//      (k_adjoint_forward_keep); else a block of segments of every particle is recomputed at once
+//      (segments x n independent lanes);
 //   2. scans the counts into every tile's start and every particle group's place within each tile;
 //   3. runs the reverse steps of the block per particle (one lane per particle, the only sequential
 //      part): for each run of kAdjSub steps, from the last to the first, it recomputes the run from
@@ -369,12 +370,16 @@ struct AdjBlock {
 	int s0, s1;          // steps [s0, s1)
 	int first, last;     // first block of the backward (reads the output adjoints); last block
 	int npg;             // particle groups: ceil(n / kAdjGroup)
-	double *sub;         // [q / kAdjSub][6][n]: x, u before step s0 + q, q a multiple of kAdjSub
+	const double *sub;   // [q / kAdjSub][6][n]: x, u before step s0 + q, q a multiple of kAdjSub
 	double *carry;       // [6][n]: adjoint (x, u) between blocks
 	DepRec *srec;        // [m], grouped by tile
-	uint32_t *counts;    // [npg][ntiles]: records per particle group and tile, then their offsets
+	const uint32_t *counts; // [npg][ntiles]: records per particle group and tile
+	uint32_t *offs;      // [npg][ntiles]: their offsets (the counts' own buffer when those are recomputed)
 	uint32_t *tileStart; // [ntiles + 1]
 	uint32_t *wgStart;   // [ntiles + 1]: first accumulating workgroup of every tile
+	// the scans take blockIdx.y blocks at once: 32-bit words from one block's counts and offsets, and from one's
+	// starts, to the next one's
+	size_t countStride, startStride;
 	int ntx, nty, ntz, ntiles;
 	size_t m;            // records of the block: (s1 - s0) * n
 };
@@ -382,7 +387,7 @@ struct AdjBlock {
 __global__ void __launch_bounds__(kAdjGroup) k_dep_zero(AdjBlock Bk) {
 	const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
 	if (k < (size_t)Bk.npg * Bk.ntiles)
-		Bk.counts[k] = 0u;
+		Bk.offs[k] = 0u;
 }
 
 // the record key of a cell: tile << 3S | cell in tile (x << 2S | y << S | z)
@@ -392,6 +397,76 @@ __device__ __forceinline__ uint32_t adj_key(const AdjBlock &Bk, const TriPoint &
 	const uint32_t tile = (uint32_t)(((cx >> S) * Bk.nty + (cy >> S)) * Bk.ntz + (cz >> S));
 	const uint32_t m = (1u << S) - 1;
 	return (tile << (3 * S)) | (((uint32_t)cx & m) << (2 * S)) | (((uint32_t)cy & m) << S) | ((uint32_t)cz & m);
+}
+
+__device__ __forceinline__ void adj_store_sub(double *o, size_t n, const V3 &x, const V3 &u) {
+	__builtin_nontemporal_store(x.x, o);
+	__builtin_nontemporal_store(x.y, o + n);
+	__builtin_nontemporal_store(x.z, o + 2 * n);
+	__builtin_nontemporal_store(u.x, o + 3 * n);
+	__builtin_nontemporal_store(u.y, o + 4 * n);
+	__builtin_nontemporal_store(u.z, o + 5 * n);
+}
+
+// the forward's kept sub-checkpoints and counts, block after block of `steps` steps
+struct AdjKeep {
+	int steps, nty, ntz, ntiles, npg;
+	size_t subStride;    // doubles from one block's sub-checkpoints to the next one's
+	size_t countStride;  // words from one block's counts to the next one's
+	double *sub;
+	uint32_t *counts;
+};
+
+// The forward that leaves what the backward's blocks start from: the sub-checkpoints of every block and, per
+// particle group (a workgroup), the tile counts, which are formed in LDS and written once a block.  The step is
+// bound by its serial chain at one wave to a SIMD, beside which the LDS count and 6 stores in L steps cost
+// little (4096 steps of 65536 particles: 5.66 ms, 5.75 without); the backward then has no step to run a third time (loss and
+// gradient of that batch 31.0 -> 24.7 ms).
+template <int S, int L>
+__global__ void __launch_bounds__(kAdjGroup) k_adjoint_forward_keep(AdjArgs A, AdjKeep Kp) {
+	extern __shared__ uint32_t hist[];
+	const int T = Kp.ntiles;
+	for (int k = threadIdx.x; k < T; k += blockDim.x)
+		hist[k] = 0u;
+	__syncthreads();
+	const size_t n = A.n, i = (size_t)blockIdx.x * kAdjGroup + threadIdx.x;
+	const bool live = i < n;
+	const size_t il = live ? i : n - 1;
+	V3 x = v3(A.x0[3 * il], A.x0[3 * il + 1], A.x0[3 * il + 2]);
+	V3 u = v3(A.u0[3 * il], A.u0[3 * il + 1], A.u0[3 * il + 2]);
+	const double kq = A.kq[il];
+	AdjBlock Bk; // adj_key reads the tile counts per axis
+	Bk.nty = Kp.nty;
+	Bk.ntz = Kp.ntz;
+	for (int b = 0, s0 = 0; s0 < A.nsteps; b++, s0 += Kp.steps) {
+		const int m = min(Kp.steps, A.nsteps - s0);
+		if (live) {
+			double *o = Kp.sub + (size_t)b * Kp.subStride + i;
+			for (int q = 0; q < m; q++) {
+				if (q % L == 0) {
+					adj_store_sub(o, n, x, u);
+					o += 6 * n;
+				}
+				const V3 x1 = vadd(x, vmul(u, A.h / 2));
+				TriPoint tp;
+				adj_cell(A.G, x1, tp);
+				const V3 Tv = adj_interp(A.G, tp);
+				atomicAdd(&hist[adj_key<S>(Bk, tp) >> (3 * S)], 1u);
+				adj_push(A.G, A.h, kq, Tv, x1, x, u);
+			}
+		}
+		__syncthreads();
+		uint32_t *cnt = Kp.counts + (size_t)b * Kp.countStride + (size_t)blockIdx.x * T;
+		for (int k = threadIdx.x; k < T; k += blockDim.x) {
+			cnt[k] = hist[k];
+			hist[k] = 0u;
+		}
+		__syncthreads();
+	}
+	if (live) {
+		A.xout[3 * i] = x.x; A.xout[3 * i + 1] = x.y; A.xout[3 * i + 2] = x.z;
+		A.uout[3 * i] = u.x; A.uout[3 * i + 1] = u.y; A.uout[3 * i + 2] = u.z;
+	}
 }
 
 // One lane per (segment, particle); a workgroup holds kAdjGroup particles of one segment.  Every step
@@ -416,13 +491,7 @@ __global__ void __launch_bounds__(kAdjGroup) k_adj_recompute(AdjArgs A, AdjBlock
 		int q = seg * A.K - Bk.s0;
 		for (int j = 0; j < len; j++, q++) {
 			if (q % L == 0) {
-				double *o = Bk.sub + (size_t)(q / L) * 6 * n + i;
-				__builtin_nontemporal_store(x.x, o);
-				__builtin_nontemporal_store(x.y, o + n);
-				__builtin_nontemporal_store(x.z, o + 2 * n);
-				__builtin_nontemporal_store(u.x, o + 3 * n);
-				__builtin_nontemporal_store(u.y, o + 4 * n);
-				__builtin_nontemporal_store(u.z, o + 5 * n);
+				adj_store_sub(const_cast<double *>(Bk.sub) + (size_t)(q / L) * 6 * n + i, n, x, u);
 			}
 			const V3 x1 = vadd(x, vmul(u, A.h / 2));
 			TriPoint tp;
@@ -433,7 +502,7 @@ __global__ void __launch_bounds__(kAdjGroup) k_adj_recompute(AdjArgs A, AdjBlock
 		}
 	}
 	__syncthreads();
-	uint32_t *cnt = Bk.counts + (size_t)pg * T;
+	uint32_t *cnt = Bk.offs + (size_t)pg * T;
 	for (int k = threadIdx.x; k < T; k += blockDim.x)
 		if (hist[k])
 			atomicAdd(cnt + k, hist[k]);
@@ -446,20 +515,22 @@ __global__ void __launch_bounds__(256) k_dep_scan_chunks(AdjBlock Bk) {
 	const int t = blockIdx.x * blockDim.x + threadIdx.x;
 	if (t >= Bk.ntiles)
 		return;
+	const uint32_t *counts = Bk.counts + blockIdx.y * Bk.countStride;
+	uint32_t *offs = Bk.offs + blockIdx.y * Bk.countStride;
 	uint32_t acc = 0;
 	for (int c0 = 0; c0 < Bk.npg; c0 += kScanBatch) {
 		uint32_t v[kScanBatch];
 #pragma unroll
 		for (int k = 0; k < kScanBatch; k++)
-			v[k] = (c0 + k < Bk.npg) ? Bk.counts[(size_t)(c0 + k) * Bk.ntiles + t] : 0u;
+			v[k] = (c0 + k < Bk.npg) ? counts[(size_t)(c0 + k) * Bk.ntiles + t] : 0u;
 #pragma unroll
 		for (int k = 0; k < kScanBatch; k++) {
 			if (c0 + k < Bk.npg)
-				Bk.counts[(size_t)(c0 + k) * Bk.ntiles + t] = acc;
+				offs[(size_t)(c0 + k) * Bk.ntiles + t] = acc;
 			acc += v[k];
 		}
 	}
-	Bk.tileStart[t + 1] = acc;
+	Bk.tileStart[blockIdx.y * Bk.startStride + t + 1] = acc;
 }
 
 // exclusive scans of the tile totals into tile starts and of the tiles' workgroup counts into
@@ -471,12 +542,13 @@ __global__ void __launch_bounds__(1024) k_dep_scan_tiles(AdjBlock Bk) {
 	__shared__ uint32_t part[1024], partw[1024];
 	const int T = Bk.ntiles;
 	const int per = (T + 1023) / 1024;
+	uint32_t *tileStart = Bk.tileStart + blockIdx.y * Bk.startStride, *wgStart = Bk.wgStart + blockIdx.y * Bk.startStride;
 	const int b = threadIdx.x * per, e = min(b + per, T);
 	uint32_t v[kScanPer];
 	uint32_t sum = 0, sumw = 0;
 #pragma unroll
 	for (int k = 0; k < kScanPer; k++) {
-		v[k] = (b + k < e) ? Bk.tileStart[b + k + 1] : 0u;
+		v[k] = (b + k < e) ? tileStart[b + k + 1] : 0u;
 		sum += v[k];
 		sumw += (v[k] + kDepPerGroup - 1) / kDepPerGroup;
 	}
@@ -498,15 +570,15 @@ __global__ void __launch_bounds__(1024) k_dep_scan_tiles(AdjBlock Bk) {
 #pragma unroll
 	for (int k = 0; k < kScanPer; k++) {
 		if (b + k < e) {
-			Bk.tileStart[b + k] = acc;
-			Bk.wgStart[b + k] = accw;
+			tileStart[b + k] = acc;
+			wgStart[b + k] = accw;
 			acc += v[k];
 			accw += (v[k] + kDepPerGroup - 1) / kDepPerGroup;
 		}
 	}
 	if (e == T && b < e) {
-		Bk.tileStart[T] = acc;
-		Bk.wgStart[T] = accw;
+		tileStart[T] = acc;
+		wgStart[T] = accw;
 	}
 }
 
@@ -578,7 +650,7 @@ __device__ __forceinline__ V3 adj_reverse_stored(const AdjGrid &G, double h, dou
 }
 
 // One lane per particle, kAdjGroup particles per workgroup; each step's record goes to its tile's range
-// at the group's offset (counts, from the scans) plus its rank among the group's records of the tile.
+// at the group's offset (offs, from the scans) plus its rank among the group's records of the tile.
 // one wave per SIMD (n / 64 waves in all): the kernel may use the whole register file, and holds a run
 // of L steps' stored values in it (the step and reverse-step arithmetic, FP64 at one wave per SIMD,
 // is what bounds it, not the run's gathers)
@@ -587,10 +659,10 @@ __global__ void __launch_bounds__(kAdjGroup) __attribute__((amdgpu_waves_per_eu(
 	extern __shared__ uint32_t lds[];
 	const int T = Bk.ntiles;
 	uint32_t *base = lds, *rank = lds + T;
-	uint32_t *off = Bk.counts + (size_t)blockIdx.x * T;
+	uint32_t *off = Bk.offs + (size_t)blockIdx.x * T;
 	for (int t = threadIdx.x; t < T; t += blockDim.x) {
 		base[t] = Bk.tileStart[t] + off[t];
-		off[t] = 0u; // for the block that counts in this buffer next
+		off[t] = 0u; // for the block that is recomputed into this buffer next
 		rank[t] = 0u;
 	}
 	__syncthreads();

@@ -2811,6 +2811,13 @@ struct AdjPlan {
 	size_t maxRecords; // records of the largest block
 	// byte offsets into the scratch
 	size_t oCarry, oSub[2], oSRec[2], oCounts[2], oTileStart[2], oWgStart[2], total;
+	// The forward keeps the sub-checkpoints and counts of all blocks where they fit the budget (per step
+	// and particle 6 bytes, and 4 per tile, group and block): the blocks' offsets and starts are then in the scratch
+	// side by side, countStride and startStride words apart, and the checkpoint buffer holds
+	// [nblocks][subPerBlock][6][n] states, then from oKeptCounts [nblocks][npg][ntiles] counts, in place of the
+	// segments' states
+	bool keep;
+	size_t subPerBlock, countStride, startStride, oKeptCounts, keptBytes;
 };
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -2856,14 +2863,27 @@ static AdjPlan adj_plan(const crp_adjoint_config *cfg, size_t n) {
 	P.nblocks = (P.nseg + P.segPerBlock - 1) / P.segPerBlock;
 	P.segPerBlock = (P.nseg + P.nblocks - 1) / P.nblocks; // the same number of segments in every block
 	P.maxRecords = (size_t)P.segPerBlock * K * n;
+	P.subPerBlock = ((size_t)P.segPerBlock * K + kAdjSub - 1) / kAdjSub;
+	P.countStride = (size_t)P.npg * P.ntiles;
+	P.startStride = align256(((size_t)P.ntiles + 1) * sizeof(uint32_t)) / sizeof(uint32_t);
+	P.oKeptCounts = align256((size_t)P.nblocks * P.subPerBlock * 6 * n * sizeof(double));
+	P.keptBytes = P.oKeptCounts + align256((size_t)P.nblocks * P.countStride * sizeof(uint32_t));
+	P.keep = (double)P.keptBytes <= budget && P.nblocks <= 65535;
 	size_t o = 0;
 	P.oCarry = o;      o += align256(6 * n * sizeof(double));
 	for (int k = 0; k < 2; k++) {
-		P.oSub[k] = o;        o += align256(((size_t)P.segPerBlock * K + kAdjSub - 1) / kAdjSub * 6 * n * sizeof(double));
 		P.oSRec[k] = o;       o += align256(P.maxRecords * sizeof(DepRec));
-		P.oCounts[k] = o;     o += align256((size_t)P.npg * P.ntiles * sizeof(uint32_t));
-		P.oTileStart[k] = o;  o += align256(((size_t)P.ntiles + 1) * sizeof(uint32_t));
-		P.oWgStart[k] = o;    o += align256(((size_t)P.ntiles + 1) * sizeof(uint32_t));
+		if (P.keep)
+			continue;
+		P.oSub[k] = o;        o += align256(P.subPerBlock * 6 * n * sizeof(double));
+		P.oCounts[k] = o;     o += align256(P.countStride * sizeof(uint32_t));
+		P.oTileStart[k] = o;  o += P.startStride * sizeof(uint32_t);
+		P.oWgStart[k] = o;    o += P.startStride * sizeof(uint32_t);
+	}
+	if (P.keep) {
+		P.oCounts[0] = o;     o += align256((size_t)P.nblocks * P.countStride * sizeof(uint32_t));
+		P.oTileStart[0] = o;  o += (size_t)P.nblocks * P.startStride * sizeof(uint32_t);
+		P.oWgStart[0] = o;    o += (size_t)P.nblocks * P.startStride * sizeof(uint32_t);
 	}
 	P.total = o;
 	return P;
@@ -2903,7 +2923,9 @@ static size_t adj_cells_bytes(const crp_adjoint_config *cfg) {
 	return b <= kAdjCellsMax ? b : 0;
 }
 
-static size_t adj_checkpoint_bytes(const crp_adjoint_config *cfg, size_t n) {
+static size_t adj_checkpoint_bytes(const crp_adjoint_config *cfg, size_t n, const AdjPlan &P) {
+	if (P.keep)
+		return P.keptBytes;
 	const size_t nseg = ((size_t)cfg->nsteps + cfg->checkpoint_every - 1) / cfg->checkpoint_every;
 	return align256((nseg > 0 ? nseg : 1) * 6 * n * sizeof(double));
 }
@@ -2913,10 +2935,11 @@ int crp_adjoint_workspace(const crp_adjoint_config *cfg, size_t n, size_t *check
 	int rc = adj_args(cfg, n, A);
 	if (rc != CRP_OK)
 		return rc;
+	const AdjPlan P = adj_plan(cfg, n);
 	if (checkpoint_bytes)
-		*checkpoint_bytes = adj_checkpoint_bytes(cfg, n) + adj_cells_bytes(cfg);
+		*checkpoint_bytes = adj_checkpoint_bytes(cfg, n, P) + adj_cells_bytes(cfg);
 	if (scratch_bytes)
-		*scratch_bytes = std::max<size_t>(adj_plan(cfg, n).total, 8);
+		*scratch_bytes = std::max<size_t>(P.total, 8);
 	return CRP_OK;
 }
 
@@ -2936,15 +2959,33 @@ int crp_adjoint_forward(const crp_adjoint_config *cfg, size_t n, const double *x
 	A.ckpt = checkpoints;
 	A.xout = x_out;
 	A.uout = u_out;
+	const AdjPlan P = adj_plan(cfg, n);
 	if (adj_cells_bytes(cfg)) {
-		float *cells = reinterpret_cast<float *>(reinterpret_cast<char *>(checkpoints) + adj_checkpoint_bytes(cfg, n));
+		float *cells = reinterpret_cast<float *>(reinterpret_cast<char *>(checkpoints) + adj_checkpoint_bytes(cfg, n, P));
 		const size_t ncell = (size_t)cfg->nx * cfg->ny * cfg->nz;
 		const unsigned blocks = (unsigned)std::min<size_t>((ncell + 255) / 256, 65535);
 		hipLaunchKernelGGL(k_build_cells, dim3(blocks), dim3(256), 0, (hipStream_t)stream, cfg->grid, cells, cfg->nx,
 		                   cfg->ny, cfg->nz);
 		A.G.cells = cells;
 	}
-	hipLaunchKernelGGL(k_adjoint_forward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, A);
+	if (P.keep) {
+		AdjKeep Kp;
+		Kp.steps = P.segPerBlock * A.K;
+		Kp.nty = P.nty;
+		Kp.ntz = P.ntz;
+		Kp.ntiles = P.ntiles;
+		Kp.npg = P.npg;
+		Kp.subStride = P.subPerBlock * 6 * n;
+		Kp.countStride = P.countStride;
+		Kp.sub = checkpoints;
+		Kp.counts = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(checkpoints) + P.oKeptCounts);
+		const size_t lb = (size_t)P.ntiles * sizeof(uint32_t);
+		if (P.tileShift == 3)
+			hipLaunchKernelGGL((k_adjoint_forward_keep<3, kAdjSub>), dim3((unsigned)P.npg), dim3(kAdjGroup), lb, (hipStream_t)stream, A, Kp);
+		else
+			hipLaunchKernelGGL((k_adjoint_forward_keep<4, kAdjSub>), dim3((unsigned)P.npg), dim3(kAdjGroup), lb, (hipStream_t)stream, A, Kp);
+	} else
+		hipLaunchKernelGGL(k_adjoint_forward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, A);
 	CRP_HIP_TRY(hipGetLastError());
 	return CRP_OK;
 }
@@ -2984,10 +3025,10 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 	A.gradX0 = grad_x0;
 	A.gradU0 = grad_u0;
 	A.gradScale = grad_scale;
-	if (adj_cells_bytes(cfg))
-		A.G.cells = reinterpret_cast<const float *>(reinterpret_cast<const char *>(checkpoints) + adj_checkpoint_bytes(cfg, n));
-	hipStream_t sa = (hipStream_t)stream;
 	const AdjPlan P = adj_plan(cfg, n);
+	if (adj_cells_bytes(cfg))
+		A.G.cells = reinterpret_cast<const float *>(reinterpret_cast<const char *>(checkpoints) + adj_checkpoint_bytes(cfg, n, P));
+	hipStream_t sa = (hipStream_t)stream;
 	if (!P.blocked) {
 		hipLaunchKernelGGL(k_adjoint_backward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, sa, A);
 		CRP_HIP_TRY(hipGetLastError());
@@ -2997,13 +3038,14 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 	// block before.  The recompute of the next block goes to a stream of its own, B, where the reverse sweep
 	// leaves half the SIMDs idle or more; where it has a wave on nearly all, the two beside each other take longer
 	// (2.3 ms a block of 65536 particles) than one after the other (1.28 + 0.69), and the recompute runs on
-	// stream A before its sweep, beside the accumulation
+	// stream A before its sweep, beside the accumulation.  With the forward's sub-checkpoints and counts there is
+	// nothing to recompute, and the scans of all blocks are the first launches
 	hipStream_t sb, sc;
 	CRP_HIP_TRY(adj_side_streams(&sb, &sc));
 	const int ncu = num_cus();
 	if (ncu < 0)
 		return CRP_E_HIP;
-	const bool apart = n <= (size_t)ncu * 4 * 64 / 2;
+	const bool apart = !P.keep && n <= (size_t)ncu * 4 * 64 / 2;
 	if (!apart)
 		sb = sa;
 	AdjEvents E;
@@ -3025,11 +3067,22 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 		std::memset(&Bk, 0, sizeof(Bk));
 		const int buf = b & 1;
 		Bk.carry = reinterpret_cast<double *>(base + P.oCarry);
-		Bk.sub = reinterpret_cast<double *>(base + P.oSub[buf]);
 		Bk.srec = reinterpret_cast<DepRec *>(base + P.oSRec[buf]);
-		Bk.counts = reinterpret_cast<uint32_t *>(base + P.oCounts[buf]);
-		Bk.tileStart = reinterpret_cast<uint32_t *>(base + P.oTileStart[buf]);
-		Bk.wgStart = reinterpret_cast<uint32_t *>(base + P.oWgStart[buf]);
+		Bk.countStride = P.countStride;
+		Bk.startStride = P.startStride;
+		const int set = P.keep ? 0 : buf;
+		const size_t place = P.keep ? b : 0; // of the block's offsets and starts in their set
+		Bk.offs = reinterpret_cast<uint32_t *>(base + P.oCounts[set]) + place * P.countStride;
+		Bk.tileStart = reinterpret_cast<uint32_t *>(base + P.oTileStart[set]) + place * P.startStride;
+		Bk.wgStart = reinterpret_cast<uint32_t *>(base + P.oWgStart[set]) + place * P.startStride;
+		if (P.keep) {
+			Bk.sub = checkpoints + place * P.subPerBlock * 6 * n;
+			Bk.counts = reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(checkpoints) + P.oKeptCounts) +
+			            place * P.countStride;
+		} else {
+			Bk.sub = reinterpret_cast<const double *>(base + P.oSub[buf]);
+			Bk.counts = Bk.offs;
+		}
 		Bk.npg = P.npg;
 		Bk.ntx = P.ntx;
 		Bk.nty = P.nty;
@@ -3045,6 +3098,10 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 		return Bk;
 	};
 	const size_t T = (size_t)P.ntiles;
+	auto scan = [&](const AdjBlock &Bk, int blocks, hipStream_t st) {
+		hipLaunchKernelGGL(k_dep_scan_chunks, dim3((unsigned)((T + 255) / 256), (unsigned)blocks), dim3(256), 0, st, Bk);
+		hipLaunchKernelGGL(k_dep_scan_tiles, dim3(1, (unsigned)blocks), dim3(1024), 0, st, Bk);
+	};
 	// recompute of block b: its sub-checkpoints, the records' counts per particle group and tile, and
 	// the scans
 	auto recompute = [&](int b, hipStream_t st) {
@@ -3057,8 +3114,7 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 			hipLaunchKernelGGL((k_adj_recompute<3, kAdjSub>), grid, dim3(kAdjGroup), T * sizeof(uint32_t), st, A, Bk);
 		else
 			hipLaunchKernelGGL((k_adj_recompute<4, kAdjSub>), grid, dim3(kAdjGroup), T * sizeof(uint32_t), st, A, Bk);
-		hipLaunchKernelGGL(k_dep_scan_chunks, dim3((unsigned)((T + 255) / 256)), dim3(256), 0, st, Bk);
-		hipLaunchKernelGGL(k_dep_scan_tiles, dim3(1), dim3(1024), 0, st, Bk);
+		scan(Bk, 1, st);
 	};
 	auto reverse = [&](int b, hipStream_t st) {
 		const AdjBlock Bk = block(b);
@@ -3082,6 +3138,8 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 	CRP_HIP_TRY(hipEventRecord(start, sa));
 	CRP_HIP_TRY(hipStreamWaitEvent(sb, start, 0));
 	CRP_HIP_TRY(hipStreamWaitEvent(sc, start, 0));
+	if (P.keep)
+		scan(block(0), NB, sa);
 	if (apart) {
 		recompute(NB - 1, sb);
 		CRP_HIP_TRY(hipEventRecord(recomputed[NB - 1], sb));
@@ -3093,7 +3151,7 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 			CRP_HIP_TRY(hipStreamWaitEvent(sa, recomputed[b], 0));
 		if (b + 2 < NB)
 			CRP_HIP_TRY(hipStreamWaitEvent(sa, sorted[b + 2], 0));
-		if (!apart) // into the buffers that block b + 2 has finished with
+		if (!P.keep && !apart) // into the buffers that block b + 2 has finished with
 			recompute(b, sa);
 		reverse(b, sa);
 		CRP_HIP_TRY(hipEventRecord(reversed[b], sa));

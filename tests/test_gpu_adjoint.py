@@ -216,3 +216,36 @@ def test_adjoint_large_grid_uses_16_cell_tiles():
     assert rel < 1e-6
     assert np.allclose(got[5], ref[5], rtol=1e-7, atol=1e-8 * np.abs(ref[5]).max())
     assert got[6] == pytest.approx(ref[6], rel=1e-8)
+
+
+@pytest.mark.parametrize("n,nsteps,K,budget", [(1, 1, 1, None), (256, 64, 8, None), (257, 111, 13, None), (600, 111, 13, None),
+                                               (600, 111, 13, "4e5"), (257, 111, 13, "1.5e5")])
+def test_adjoint_kept_and_recomputed_sub_checkpoints(n, nsteps, K, budget, monkeypatch):
+    """The forward keeps the blocks' sub-checkpoints and tile counts where they fit the buffer budget;
+    beyond it (4e5 bytes where the states of 600 particles take 5.2e5; 1.5e5 of 2.2e5) the backward
+    recomputes them.  Both against the oracle at full and partial particle groups, with segments that are no
+    multiple of the 8 steps of a run, and down to one step; a second backward of the same graph finds what the
+    forward left unchanged, so it gives the gradients of the first (those of the grid up to the order of the
+    FP64 sums)."""
+    from crpropa3_amd.adjoint import boris_grid_propagate
+    if budget is not None:
+        monkeypatch.setenv("CRP_ADJOINT_BLOCK_BYTES", budget)
+    s = setup(n=n, N=16, nsteps=nsteps, K=K, seed=31)
+    ref = oracle_grad(s)
+    dev = torch.device("cuda:0")
+    g = torch.tensor(s["grid"], dtype=torch.float32, device=dev, requires_grad=True)
+    x0 = torch.tensor(s["x0"], device=dev, requires_grad=True)
+    u0 = torch.tensor(s["u0"], device=dev, requires_grad=True)
+    sc = torch.tensor(1.0, dtype=torch.float64, device=dev, requires_grad=True)
+    xo, uo = boris_grid_propagate(g, x0, u0, torch.tensor(s["E"], device=dev), O.eplus, [0, 0, 0], [s["sp"]] * 3,
+                                  s["h"], s["nsteps"], s["K"], scale=sc)
+    loss = ((uo - torch.tensor(s["target"], device=dev)) ** 2).sum() + (torch.tensor(s["wx"], device=dev) * xo).sum()
+    one = [t.double().cpu().numpy() for t in torch.autograd.grad(loss, (g, x0, u0, sc), retain_graph=True)]
+    two = [t.double().cpu().numpy() for t in torch.autograd.grad(loss, (g, x0, u0, sc))]
+    assert np.allclose(one[0], ref[3], rtol=0, atol=1e-6 * np.abs(ref[3]).max())
+    for a, b in ((one[1], ref[4]), (one[2], ref[5])):
+        assert np.allclose(a, b, rtol=1e-7, atol=1e-8 * np.abs(b).max())
+    assert float(one[3]) == pytest.approx(ref[6], rel=1e-8)
+    assert np.array_equal(one[1], two[1]) and np.array_equal(one[2], two[2])
+    # the grid gradient is rounded to float32 after the FP64 sums: at most an ulp apart
+    assert np.allclose(one[0], two[0], rtol=2.0 ** -23, atol=1e-12 * np.abs(one[0]).max())

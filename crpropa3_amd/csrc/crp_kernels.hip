@@ -2820,6 +2820,14 @@ struct AdjPlan {
 	size_t subPerBlock, countStride, startStride, oKeptCounts, keptBytes;
 };
 
+// A workgroup of the reverse sweep needs a compute unit's whole register file but for 104 registers a lane, so
+// it waited until the accumulating workgroups of the block before had left the unit: sweep and accumulation
+// took turns (1.3 + 1.1 ms a block of 65536 particles).  With this much more LDS asked for, one accumulating
+// workgroup (56 registers) fits a unit and not two, and leaves the sweep its place whichever comes first
+// (17.5 + 64.5 KB beside the sweep's 64 at most, of 160): loss and gradient 24.7 -> 20.2 ms.  The accumulation of
+// the last block has nothing beside it and takes all the room.
+constexpr size_t kDepPad = 66000;
+
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 static AdjPlan adj_plan(const crp_adjoint_config *cfg, size_t n) {
@@ -3129,7 +3137,7 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 		const AdjBlock Bk = block(b);
 		const size_t groups = T + (Bk.m + kDepPerGroup - 1) / kDepPerGroup;
 		if (P.tileShift == 3)
-			hipLaunchKernelGGL(k_dep_tiles<3>, dim3((unsigned)groups), dim3(Tile<3>::threads), 0, st, A, Bk);
+			hipLaunchKernelGGL(k_dep_tiles<3>, dim3((unsigned)groups), dim3(Tile<3>::threads), b > 0 ? kDepPad : 0, st, A, Bk);
 		else
 			hipLaunchKernelGGL(k_dep_tiles<4>, dim3((unsigned)groups), dim3(Tile<4>::threads), 0, st, A, Bk);
 	};

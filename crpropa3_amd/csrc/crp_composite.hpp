@@ -105,16 +105,17 @@ struct FieldComposite {
 	// JF12 and the grids read tricubic or nearest neighbour share one out-of-line call site
 	__device__ static __attribute__((noinline)) V3 leaf_eval_call(const CompLeaf *Lp, const V3 &x) {
 		if (ld_const(&Lp->kind) == CL_JF12) {
-			const FieldJF12 j = ld_const(&Lp->jf12);
-			return j.turbulent.interp == kInterpTrilinear ? j.eval(x) : j.eval_any(x);
+			return ld_const(&Lp->jf12.turbulent.interp) == kInterpTrilinear ? jf12_eval<false>(&Lp->jf12, x)
+			                                                                 : jf12_eval<true>(&Lp->jf12, x);
 		}
 		const GridDesc mod = ld_const(&Lp->mod);
 		return FieldGridAny{ld_const(&Lp->grid), mod, mod.values != nullptr}.eval(x);
 	}
 	__device__ static __attribute__((noinline)) float3 leaf_evalf_call(const CompLeaf *Lp, const V3 &x) {
 		if (ld_const(&Lp->kind) == CL_JF12) {
-			const FieldJF12 j = ld_const(&Lp->jf12);
-			return j.turbulent.interp == kInterpTrilinear ? j.evalf(x) : FieldJF12Any{j}.evalf(x);
+			const V3 b = ld_const(&Lp->jf12.turbulent.interp) == kInterpTrilinear ? jf12_eval<false>(&Lp->jf12, x)
+			                                                                      : jf12_eval<true>(&Lp->jf12, x);
+			return make_float3((float)b.x, (float)b.y, (float)b.z);
 		}
 		const GridDesc mod = ld_const(&Lp->mod);
 		return FieldGridAny{ld_const(&Lp->grid), mod, mod.values != nullptr}.evalf(x);

@@ -239,11 +239,20 @@ __device__ __forceinline__ void sde_drift(const Params &P, const V3 &pos, double
 
 enum SdePhase { SDE_BEGIN = 0, SDE_TRIAL = 1, SDE_SUB = 2 };
 
+// The kernel of a uniform field would miss two waves to a SIMD by 17 registers (70000 particles: 15 us a step with
+// one wave, 11 with two); on a tricubic grid two cost more in spills than they bring (416 us against 260).
+template <class F> struct SdeWaves {
+	static constexpr int value = 1;
+};
+template <> struct SdeWaves<FieldUniform> {
+	static constexpr int value = 2;
+};
+
 // MODS: the periodic box, spherical boundary and observer are compiled in (the length limit always is);
 // without them the kernel keeps fewer registers
 template <class F, bool MODS>
-__global__ void __launch_bounds__(256) k_sde(F field0, Params P, Soa S, unsigned long long n,
-                                             unsigned long long *__restrict__ ctr) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SdeWaves<F>::value, 8))) k_sde(F field0, Params P, Soa S,
+                                             unsigned long long n, unsigned long long *__restrict__ ctr) {
 	const int lane = __lane_id();
 	F field = field0; // the lane's copy: a field that reads the candidate's redshift binds it at refill
 	const double cosHalfPi = crp_cos_cr(3.14159265358979323846 / 2.);

@@ -338,10 +338,10 @@ __global__ void __launch_bounds__(256) k_adjoint_backward(AdjArgs A) {
 //      record (with the adjoint aT of T: the gradient of grid value G_c is w_c aT) into its tile's range;
 //   4. accumulates each tile's records into its 9^3 grid points in LDS (FP64), one workgroup per
 //      kDepPerGroup records of a tile, and adds the points into the gradient.
-// Per step the backward thus reads the cell line twice (recompute, reverse) and moves one record
+// Per step the backward thus reads the cell line once (twice with the recompute) and moves one record
 // through memory; the stored values of a step never leave the registers.  The host runs the reverse
-// sweeps on the caller's stream and the recompute of the next block and the accumulation of the
-// previous one on two more streams beside it.  The arithmetic of a step is that of adj_step /
+// sweeps on the caller's stream and, on more streams beside it, the accumulation of the previous block and,
+// where there is one, the recompute of the next.  The arithmetic of a step is that of adj_step /
 // adj_step_reverse, except that the position gradient is taken as aT . dT/df; the deposits are
 // summed in another order.
 // deposit tiles of 2^S cells per axis: 8^3 (S = 3, 9^3 points = 17.5 KB of FP64 LDS per accumulating

@@ -1,10 +1,12 @@
 """Differentiable fixed-step Boris propagation through a periodic Grid3f.
 
 `BorisGridFunction` is a torch.autograd.Function whose forward and backward
-are the HIP kernels behind crp_adjoint_forward / crp_adjoint_backward
-(include/crpropa3_amd.h): the forward stores the state every K steps, the
-backward recomputes each K-step segment and runs the hand-written reverse
-step, scatter-adding into the grid gradient with FP64 atomics.
+are the HIP kernels behind crp_adjoint_forward_planned / crp_adjoint_backward_planned
+(include/crpropa3_amd.h): the forward keeps the states every 8 steps (the state
+every K steps where those take too much), the backward recomputes each run of
+steps from the state before it, runs the hand-written reverse step and
+accumulates the grid gradient in FP64.  One plan of the buffers, made in the
+forward, serves both.
 
 Model (per step h; PropagationBP::dY, src/module/PropagationBP.cpp:19-39, and
 the two direction normalisations of :121 and src/ParticleState.cpp:30-32):
@@ -27,6 +29,12 @@ class AdjointConfig(C.Structure):
                 ("step", C.c_double), ("nsteps", C.c_int), ("checkpoint_every", C.c_int)]
 
 
+class AdjointPlan(C.Structure):
+    """crp_adjoint_plan: the buffers' layout, fixed once for a forward and its backward"""
+    _fields_ = [("block_bytes", C.c_uint64), ("checkpoint_bytes", C.c_uint64), ("scratch_bytes", C.c_uint64),
+                ("tile_shift", C.c_int32), ("keep_states", C.c_int32)]
+
+
 def _bind():
     L = capi.lib()
     if getattr(L, "_adjoint_bound", False):
@@ -36,6 +44,10 @@ def _bind():
     L.crp_adjoint_workspace.argtypes = [P, C.c_size_t, C.POINTER(C.c_size_t), C.POINTER(C.c_size_t)]
     L.crp_adjoint_forward.argtypes = [P, C.c_size_t, vp, vp, vp, vp, vp, vp, vp]
     L.crp_adjoint_backward.argtypes = [P, C.c_size_t, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+    Q = C.POINTER(AdjointPlan)
+    L.crp_adjoint_plan_make.argtypes = [P, C.c_size_t, C.c_int, Q]
+    L.crp_adjoint_forward_planned.argtypes = [P, C.c_size_t, Q, vp, vp, vp, vp, vp, vp, vp]
+    L.crp_adjoint_backward_planned.argtypes = [P, C.c_size_t, Q, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp]
     L._adjoint_bound = True
     return L
 
@@ -74,37 +86,38 @@ class BorisGridFunction(torch.autograd.Function):
         n = x0c.shape[0]
         L = _bind()
         cfg = _config(grid, origin, spacing, float(scale), step, nsteps, K)
-        cb, sb = C.c_size_t(0), C.c_size_t(0)
-        capi.check(L.crp_adjoint_workspace(C.byref(cfg), n, C.byref(cb), C.byref(sb)))
-        ckpt = torch.empty(max(cb.value // 8, 1), dtype=torch.float64, device=grid.device)
+        plan = AdjointPlan()
+        capi.check(L.crp_adjoint_plan_make(C.byref(cfg), n, 1, C.byref(plan)))
+        ckpt = torch.empty(max(plan.checkpoint_bytes // 8, 1), dtype=torch.float64, device=grid.device)
         xo = torch.empty_like(x0c)
         uo = torch.empty_like(u0c)
         stream = C.c_void_p(torch.cuda.current_stream(grid.device).cuda_stream)
-        capi.check(L.crp_adjoint_forward(C.byref(cfg), n, _ptr(x0c), _ptr(u0c), _ptr(kqc), _ptr(ckpt), _ptr(xo),
-                                         _ptr(uo), stream))
+        capi.check(L.crp_adjoint_forward_planned(C.byref(cfg), n, C.byref(plan), _ptr(x0c), _ptr(u0c), _ptr(kqc),
+                                                 _ptr(ckpt), _ptr(xo), _ptr(uo), stream))
         ctx.save_for_backward(grid, kqc, ckpt)
-        ctx.meta = (origin, spacing, float(scale), step, nsteps, K, sb.value, grid.dtype)
+        ctx.meta = (origin, spacing, float(scale), step, nsteps, K, plan, grid.dtype)
         ctx.scale_is_tensor = torch.is_tensor(scale)
         return xo, uo
 
     @staticmethod
     def backward(ctx, gx, gu):
         grid, kqc, ckpt = ctx.saved_tensors
-        origin, spacing, scale, step, nsteps, K, sbytes, gdtype = ctx.meta
+        origin, spacing, scale, step, nsteps, K, plan, gdtype = ctx.meta
         n = kqc.shape[0]
         dev = grid.device
         L = _bind()
         cfg = _config(grid, origin, spacing, scale, step, nsteps, K)
         gu = torch.zeros((n, 3), dtype=torch.float64, device=dev) if gu is None else gu.to(torch.float64).contiguous()
         gx = None if gx is None else gx.to(torch.float64).contiguous()
-        scratch = torch.empty(max(sbytes // 8, 1), dtype=torch.float64, device=dev)
+        scratch = torch.empty(max(plan.scratch_bytes // 8, 1), dtype=torch.float64, device=dev)
         ggrid = torch.zeros(grid.numel(), dtype=torch.float64, device=dev)
         gscale = torch.zeros(1, dtype=torch.float64, device=dev)
         gx0 = torch.empty((n, 3), dtype=torch.float64, device=dev)
         gu0 = torch.empty((n, 3), dtype=torch.float64, device=dev)
         stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-        capi.check(L.crp_adjoint_backward(C.byref(cfg), n, _ptr(kqc), _ptr(ckpt), _ptr(gx), _ptr(gu), _ptr(scratch),
-                                          _ptr(ggrid), _ptr(gx0), _ptr(gu0), _ptr(gscale), stream))
+        capi.check(L.crp_adjoint_backward_planned(C.byref(cfg), n, C.byref(plan), _ptr(kqc), _ptr(ckpt), _ptr(gx),
+                                                  _ptr(gu), _ptr(scratch), _ptr(ggrid), _ptr(gx0), _ptr(gu0),
+                                                  _ptr(gscale), stream))
         gs = gscale.view(()) if ctx.scale_is_tensor else None
         return (ggrid.view(grid.shape).to(gdtype), gx0, gu0, gs, None, None, None, None, None, None)
 

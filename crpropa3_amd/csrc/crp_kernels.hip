@@ -2811,7 +2811,7 @@ struct AdjPlan {
 	size_t maxRecords; // records of the largest block
 	// byte offsets into the scratch
 	size_t oCarry, oSub[2], oSRec[2], oCounts[2], oTileStart[2], oWgStart[2], total;
-	// The forward keeps the sub-checkpoints and counts of all blocks where they fit the budget (per step
+	// Where the caller's plan asks for it, the forward keeps the sub-checkpoints and counts of all blocks (per step
 	// and particle 6 bytes, and 4 per tile, group and block): the blocks' offsets and starts are then in the scratch
 	// side by side, countStride and startStride words apart, and the checkpoint buffer holds
 	// [nblocks][subPerBlock][6][n] states, then from oKeptCounts [nblocks][npg][ntiles] counts, in place of the
@@ -2830,16 +2830,31 @@ constexpr size_t kDepPad = 66000;
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-static AdjPlan adj_plan(const crp_adjoint_config *cfg, size_t n) {
+// What the environment asks for at this call: CRP_ADJOINT_TILE_SHIFT=4 16^3-cell tiles on grids where 8^3 would do,
+// CRP_ADJOINT_BLOCK_BYTES another buffer-set budget (0: per-step atomics), so that tests can run the multi-block
+// and the atomic paths on small inputs
+static crp_adjoint_plan adj_choice() {
+	crp_adjoint_plan c;
+	std::memset(&c, 0, sizeof(c));
+	const char *ts = std::getenv("CRP_ADJOINT_TILE_SHIFT");
+	c.tile_shift = (ts && std::atoi(ts) == 4) ? 4 : 3;
+	double budget = (double)kAdjBlockBudget;
+	if (const char *e = std::getenv("CRP_ADJOINT_BLOCK_BYTES"))
+		budget = std::strtod(e, nullptr);
+	c.block_bytes = budget > 0 ? (uint64_t)std::min(std::max(budget, 1.0), 0x1p62) : 0;
+	return c;
+}
+
+// a function of its arguments alone: a forward and its backward that are given the same choice agree on every
+// buffer, whatever the environment says in between
+static AdjPlan adj_plan(const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan &choice) {
 	AdjPlan P;
 	std::memset(&P, 0, sizeof(P));
 	const int K = cfg->checkpoint_every;
 	P.nseg = (cfg->nsteps + K - 1) / K;
 	P.npg = (int)((n + kAdjGroup - 1) / kAdjGroup);
-	// CRP_ADJOINT_TILE_SHIFT=4 asks for 16^3-cell tiles on grids where 8^3 would do (tests)
-	const char *ts = std::getenv("CRP_ADJOINT_TILE_SHIFT");
 	long long tiles = 0;
-	for (int shift = (ts && std::atoi(ts) == 4) ? 4 : 3; shift <= 4; shift++) {
+	for (int shift = choice.tile_shift; shift <= 4; shift++) {
 		const int c = 1 << shift;
 		P.tileShift = shift;
 		P.ntx = (cfg->nx + c - 1) / c;
@@ -2851,11 +2866,7 @@ static AdjPlan adj_plan(const crp_adjoint_config *cfg, size_t n) {
 	}
 	// per segment and buffer set: the sub-checkpoints (48 B per kAdjSub steps) and the records (32 B a step)
 	const double perSeg = (double)K * (double)n * (48.0 / kAdjSub + 32.0);
-	// CRP_ADJOINT_BLOCK_BYTES overrides the buffer-set budget (0: per-step atomics), so that tests
-	// can run the multi-block and the atomic paths on small inputs
-	double budget = (double)kAdjBlockBudget;
-	if (const char *e = std::getenv("CRP_ADJOINT_BLOCK_BYTES"))
-		budget = std::strtod(e, nullptr);
+	const double budget = (double)choice.block_bytes;
 	P.blocked = budget > 0 && cfg->nsteps > 0 && n > 0 && tiles <= kAdjMaxTiles && (double)K * n < 2e9;
 	if (!P.blocked) {
 		P.total = (size_t)K * 6 * n * sizeof(double);
@@ -2876,7 +2887,7 @@ static AdjPlan adj_plan(const crp_adjoint_config *cfg, size_t n) {
 	P.startStride = align256(((size_t)P.ntiles + 1) * sizeof(uint32_t)) / sizeof(uint32_t);
 	P.oKeptCounts = align256((size_t)P.nblocks * P.subPerBlock * 6 * n * sizeof(double));
 	P.keptBytes = P.oKeptCounts + align256((size_t)P.nblocks * P.countStride * sizeof(uint32_t));
-	P.keep = (double)P.keptBytes <= budget && P.nblocks <= 65535;
+	P.keep = choice.keep_states && (double)P.keptBytes <= budget && P.nblocks <= 65535;
 	size_t o = 0;
 	P.oCarry = o;      o += align256(6 * n * sizeof(double));
 	for (int k = 0; k < 2; k++) {
@@ -2943,7 +2954,7 @@ int crp_adjoint_workspace(const crp_adjoint_config *cfg, size_t n, size_t *check
 	int rc = adj_args(cfg, n, A);
 	if (rc != CRP_OK)
 		return rc;
-	const AdjPlan P = adj_plan(cfg, n);
+	const AdjPlan P = adj_plan(cfg, n, adj_choice());
 	if (checkpoint_bytes)
 		*checkpoint_bytes = adj_checkpoint_bytes(cfg, n, P) + adj_cells_bytes(cfg);
 	if (scratch_bytes)
@@ -2951,10 +2962,46 @@ int crp_adjoint_workspace(const crp_adjoint_config *cfg, size_t n, size_t *check
 	return CRP_OK;
 }
 
-int crp_adjoint_forward(const crp_adjoint_config *cfg, size_t n, const double *x0, const double *u0,
-                        const double *kq, double *checkpoints, double *x_out, double *u_out, void *stream) {
+int crp_adjoint_plan_make(const crp_adjoint_config *cfg, size_t n, int keep_states, crp_adjoint_plan *plan) {
 	AdjArgs A;
 	int rc = adj_args(cfg, n, A);
+	if (rc != CRP_OK)
+		return rc;
+	if (!plan)
+		return fail(CRP_E_INVALID, "crp_adjoint_plan_make: NULL plan");
+	crp_adjoint_plan c = adj_choice();
+	c.keep_states = keep_states ? 1 : 0;
+	const AdjPlan P = adj_plan(cfg, n, c);
+	c.keep_states = P.keep ? 1 : 0;
+	c.checkpoint_bytes = adj_checkpoint_bytes(cfg, n, P) + adj_cells_bytes(cfg);
+	c.scratch_bytes = std::max<size_t>(P.total, 8);
+	*plan = c;
+	return CRP_OK;
+}
+
+// the layout that `plan` stands for, or an error if it was made for another config or n
+static int adj_planned(const char *fn, const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan *plan, AdjPlan &P) {
+	if (!plan || (plan->tile_shift != 3 && plan->tile_shift != 4))
+		return fail(CRP_E_INVALID, std::string(fn) + ": not a plan of crp_adjoint_plan_make");
+	P = adj_plan(cfg, n, *plan);
+	if (P.keep != (plan->keep_states != 0) || plan->scratch_bytes != std::max<size_t>(P.total, 8) ||
+	    plan->checkpoint_bytes != adj_checkpoint_bytes(cfg, n, P) + adj_cells_bytes(cfg))
+		return fail(CRP_E_INVALID, std::string(fn) + ": the plan was made for another configuration");
+	return CRP_OK;
+}
+
+// plan NULL: the K-step states, which no choice of the environment changes
+static int adj_forward(const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan *plan, const double *x0,
+                       const double *u0, const double *kq, double *checkpoints, double *x_out, double *u_out, void *stream) {
+	AdjArgs A;
+	int rc = adj_args(cfg, n, A);
+	if (rc != CRP_OK)
+		return rc;
+	AdjPlan P;
+	if (plan)
+		rc = adj_planned("crp_adjoint_forward_planned", cfg, n, plan, P);
+	else
+		P = adj_plan(cfg, n, adj_choice());
 	if (rc != CRP_OK)
 		return rc;
 	if (n == 0)
@@ -2967,7 +3014,6 @@ int crp_adjoint_forward(const crp_adjoint_config *cfg, size_t n, const double *x
 	A.ckpt = checkpoints;
 	A.xout = x_out;
 	A.uout = u_out;
-	const AdjPlan P = adj_plan(cfg, n);
 	if (adj_cells_bytes(cfg)) {
 		float *cells = reinterpret_cast<float *>(reinterpret_cast<char *>(checkpoints) + adj_checkpoint_bytes(cfg, n, P));
 		const size_t ncell = (size_t)cfg->nx * cfg->ny * cfg->nz;
@@ -2998,6 +3044,19 @@ int crp_adjoint_forward(const crp_adjoint_config *cfg, size_t n, const double *x
 	return CRP_OK;
 }
 
+int crp_adjoint_forward(const crp_adjoint_config *cfg, size_t n, const double *x0, const double *u0,
+                        const double *kq, double *checkpoints, double *x_out, double *u_out, void *stream) {
+	return adj_forward(cfg, n, nullptr, x0, u0, kq, checkpoints, x_out, u_out, stream);
+}
+
+int crp_adjoint_forward_planned(const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan *plan, const double *x0,
+                                const double *u0, const double *kq, double *checkpoints, double *x_out, double *u_out,
+                                void *stream) {
+	if (!plan)
+		return fail(CRP_E_INVALID, "crp_adjoint_forward_planned: NULL plan");
+	return adj_forward(cfg, n, plan, x0, u0, kq, checkpoints, x_out, u_out, stream);
+}
+
 // events of one blocked backward: released (after the work they mark has completed) when it returns
 struct AdjEvents {
 	std::vector<hipEvent_t> ev;
@@ -3013,11 +3072,19 @@ struct AdjEvents {
 	}
 };
 
-int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *kq, const double *checkpoints,
-                         const double *grad_x_out, const double *grad_u_out, double *segment_scratch, double *grad_grid,
-                         double *grad_x0, double *grad_u0, double *grad_scale, void *stream) {
+static int adj_backward(const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan *plan, const double *kq,
+                        const double *checkpoints, const double *grad_x_out, const double *grad_u_out,
+                        double *segment_scratch, double *grad_grid, double *grad_x0, double *grad_u0, double *grad_scale,
+                        void *stream) {
 	AdjArgs A;
 	int rc = adj_args(cfg, n, A);
+	if (rc != CRP_OK)
+		return rc;
+	AdjPlan P;
+	if (plan)
+		rc = adj_planned("crp_adjoint_backward_planned", cfg, n, plan, P);
+	else
+		P = adj_plan(cfg, n, adj_choice());
 	if (rc != CRP_OK)
 		return rc;
 	if (n == 0)
@@ -3033,7 +3100,6 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 	A.gradX0 = grad_x0;
 	A.gradU0 = grad_u0;
 	A.gradScale = grad_scale;
-	const AdjPlan P = adj_plan(cfg, n);
 	if (adj_cells_bytes(cfg))
 		A.G.cells = reinterpret_cast<const float *>(reinterpret_cast<const char *>(checkpoints) + adj_checkpoint_bytes(cfg, n, P));
 	hipStream_t sa = (hipStream_t)stream;
@@ -3183,6 +3249,23 @@ int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *
 	CRP_HIP_TRY(hipEventRecord(done, sc));
 	CRP_HIP_TRY(hipStreamWaitEvent(sa, done, 0));
 	return CRP_OK;
+}
+
+int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *kq, const double *checkpoints,
+                         const double *grad_x_out, const double *grad_u_out, double *segment_scratch, double *grad_grid,
+                         double *grad_x0, double *grad_u0, double *grad_scale, void *stream) {
+	return adj_backward(cfg, n, nullptr, kq, checkpoints, grad_x_out, grad_u_out, segment_scratch, grad_grid, grad_x0,
+	                    grad_u0, grad_scale, stream);
+}
+
+int crp_adjoint_backward_planned(const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan *plan, const double *kq,
+                                 const double *checkpoints, const double *grad_x_out, const double *grad_u_out,
+                                 double *scratch, double *grad_grid, double *grad_x0, double *grad_u0,
+                                 double *grad_scale, void *stream) {
+	if (!plan)
+		return fail(CRP_E_INVALID, "crp_adjoint_backward_planned: NULL plan");
+	return adj_backward(cfg, n, plan, kq, checkpoints, grad_x_out, grad_u_out, scratch, grad_grid, grad_x0, grad_u0,
+	                    grad_scale, stream);
 }
 
 // ------------------------------------------------------------------ turbulent grids

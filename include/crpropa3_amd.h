@@ -412,9 +412,9 @@ typedef struct {
 	int checkpoint_every; /* K */
 } crp_adjoint_config;
 
-/* Device workspace sizes: checkpoints ((ceil(nsteps/K)) * 6 * n doubles, then, for grids of at most
- * 8 GiB of cells, a table of the 8 corner values of every cell in one 128-byte line that the forward
- * builds and the backward reads) and the backward's scratch.
+/* Device workspace sizes of crp_adjoint_forward and crp_adjoint_backward: checkpoints ((ceil(nsteps/K)) * 6 * n
+ * doubles rounded up to 256 bytes, then, for grids of at most 8 GiB of cells, a table of the 8 corner values of
+ * every cell in one 128-byte line that the forward builds and the backward reads) and the backward's scratch.
  * For grids of at most 8192 tiles of 8^3 cells (or of 16^3 cells, up to about 320^3 points) the
  * backward recomputes several segments of every
  * particle at once, keeping the state every 8 steps, and sorts one deposit record per step by tile
@@ -422,7 +422,8 @@ typedef struct {
  * 4 GiB each, less for small batches) holds those states and records.  Larger grids use per-step atomics and K * 6 * n doubles of scratch.  The
  * environment variable CRP_ADJOINT_TILE_SHIFT=4 selects 16^3-cell tiles where 8^3 would do (tests).  The
  * environment variable CRP_ADJOINT_BLOCK_BYTES, read at each call, overrides the per-block budget
- * in bytes (0 selects the per-step atomics). */
+ * in bytes (0 selects the per-step atomics).  Neither changes the checkpoints; the scratch has to be as large as
+ * crp_adjoint_workspace says under the backward's environment. */
 int crp_adjoint_workspace(const crp_adjoint_config *cfg, size_t n, size_t *checkpoint_bytes, size_t *scratch_bytes);
 /* Forward: final positions/directions and checkpoints every K steps. */
 int crp_adjoint_forward(const crp_adjoint_config *cfg, size_t n, const double *x0, const double *u0,
@@ -432,6 +433,28 @@ int crp_adjoint_forward(const crp_adjoint_config *cfg, size_t n, const double *x
 int crp_adjoint_backward(const crp_adjoint_config *cfg, size_t n, const double *kq, const double *checkpoints,
                          const double *grad_x_out, const double *grad_u_out, double *scratch, double *grad_grid,
                          double *grad_x0, double *grad_u0, double *grad_scale, void *stream);
+
+/* The same two calls with their buffers' layout fixed once by crp_adjoint_plan_make, the only call here that reads
+ * the environment: the plan goes unchanged to the forward and to its backward, which fail with CRP_E_INVALID when
+ * its sizes are not those of their config and n.  keep_states asks the forward to keep what the backward would
+ * otherwise recompute, the states every 8 steps and the numbers of records per tile, in the checkpoint buffer: 6
+ * bytes a step and particle (K-step states: 48/K) and 4 bytes a tile, 256 particles and block, for a shorter
+ * backward.  Where that exceeds the per-block budget the plan comes back with keep_states 0.  The buffers are
+ * checkpoint_bytes and scratch_bytes long. */
+typedef struct {
+	uint64_t block_bytes;
+	uint64_t checkpoint_bytes, scratch_bytes;
+	int32_t tile_shift;
+	int32_t keep_states;
+} crp_adjoint_plan;
+int crp_adjoint_plan_make(const crp_adjoint_config *cfg, size_t n, int keep_states, crp_adjoint_plan *plan);
+int crp_adjoint_forward_planned(const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan *plan, const double *x0,
+                                const double *u0, const double *kq, double *checkpoints, double *x_out, double *u_out,
+                                void *stream);
+int crp_adjoint_backward_planned(const crp_adjoint_config *cfg, size_t n, const crp_adjoint_plan *plan, const double *kq,
+                                 const double *checkpoints, const double *grad_x_out, const double *grad_u_out,
+                                 double *scratch, double *grad_grid, double *grad_x0, double *grad_u0,
+                                 double *grad_scale, void *stream);
 
 /* ---------------------------------------------------------------- turbulent grids
  * SimpleGridTurbulence::initTurbulence (src/magneticField/turbulentField/SimpleGridTurbulence.cpp:18-113)

@@ -249,3 +249,32 @@ def test_adjoint_kept_and_recomputed_sub_checkpoints(n, nsteps, K, budget, monke
     assert np.array_equal(one[1], two[1]) and np.array_equal(one[2], two[2])
     # the grid gradient is rounded to float32 after the FP64 sums: at most an ulp apart
     assert np.allclose(one[0], two[0], rtol=2.0 ** -23, atol=1e-12 * np.abs(one[0]).max())
+
+
+@pytest.mark.parametrize("before,after", [({}, dict(CRP_ADJOINT_BLOCK_BYTES="0")),
+                                          ({}, dict(CRP_ADJOINT_BLOCK_BYTES="3e4")),
+                                          ({}, dict(CRP_ADJOINT_TILE_SHIFT="4")),
+                                          (dict(CRP_ADJOINT_BLOCK_BYTES="4e5"), {}),
+                                          (dict(CRP_ADJOINT_TILE_SHIFT="4"), {})])
+def test_adjoint_environment_changes_between_forward_and_backward(before, after, monkeypatch):
+    """The buffers' layout is fixed by the forward: another environment at the backward changes nothing."""
+    from crpropa3_amd.adjoint import boris_grid_propagate
+    s = setup(n=600, N=20, nsteps=111, K=13, seed=41)
+    ref = oracle_grad(s)
+    dev = torch.device("cuda:0")
+    g = torch.tensor(s["grid"], dtype=torch.float32, device=dev, requires_grad=True)
+    x0 = torch.tensor(s["x0"], device=dev, requires_grad=True)
+    u0 = torch.tensor(s["u0"], device=dev, requires_grad=True)
+    for k, v in before.items():
+        monkeypatch.setenv(k, v)
+    xo, uo = boris_grid_propagate(g, x0, u0, torch.tensor(s["E"], device=dev), O.eplus, [0, 0, 0], [s["sp"]] * 3,
+                                  s["h"], s["nsteps"], s["K"])
+    for k in before:
+        monkeypatch.delenv(k)
+    for k, v in after.items():
+        monkeypatch.setenv(k, v)
+    loss = ((uo - torch.tensor(s["target"], device=dev)) ** 2).sum() + (torch.tensor(s["wx"], device=dev) * xo).sum()
+    loss.backward()
+    assert np.allclose(g.grad.double().cpu().numpy(), ref[3], rtol=0, atol=1e-6 * np.abs(ref[3]).max())
+    for a, b in ((x0.grad, ref[4]), (u0.grad, ref[5])):
+        assert np.allclose(a.cpu().numpy(), b, rtol=1e-7, atol=1e-8 * np.abs(b).max())

@@ -681,6 +681,9 @@ __global__ void __launch_bounds__(kAdjGroup) __attribute__((amdgpu_waves_per_eu(
 		}
 		const double kq = A.kq[i];
 		const int m = Bk.s1 - Bk.s0;
+		// the block's records (below 2e9): kept counts that another kq, scale or grid than the forward's does not
+		// meet would lead past them
+		const uint32_t m32 = (uint32_t)Bk.m;
 		for (int sb = (m - 1) / L; sb >= 0; sb--) {
 			// steps [sb L, sb L + len) of the block, recomputed from their sub-checkpoint (the step
 			// guards, uniform branches, also keep every step in a basic block of its own: one block of
@@ -712,10 +715,13 @@ __global__ void __launch_bounds__(kAdjGroup) __attribute__((amdgpu_waves_per_eu(
 				if (k < len) {
 					const V3 aT = adj_reverse_stored(A.G, A.h, kq, d[k], ax, au, gs);
 					const uint32_t t = d[k].rec[0] >> (3 * S);
-					uint4 *pr = reinterpret_cast<uint4 *>(Bk.srec + base[t] + atomicAdd(&rank[t], 1u));
-					pr[0] = make_uint4(d[k].rec[0], d[k].rec[1], d[k].rec[2], d[k].rec[3]);
-					pr[1] = make_uint4(__float_as_uint((float)aT.x), __float_as_uint((float)aT.y),
-					                   __float_as_uint((float)aT.z), 0u);
+					const uint32_t p = base[t] + atomicAdd(&rank[t], 1u);
+					if (p < m32) {
+						uint4 *pr = reinterpret_cast<uint4 *>(Bk.srec + p);
+						pr[0] = make_uint4(d[k].rec[0], d[k].rec[1], d[k].rec[2], d[k].rec[3]);
+						pr[1] = make_uint4(__float_as_uint((float)aT.x), __float_as_uint((float)aT.y),
+						                   __float_as_uint((float)aT.z), 0u);
+					}
 				}
 			}
 		}

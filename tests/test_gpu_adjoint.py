@@ -278,3 +278,42 @@ def test_adjoint_environment_changes_between_forward_and_backward(before, after,
     assert np.allclose(g.grad.double().cpu().numpy(), ref[3], rtol=0, atol=1e-6 * np.abs(ref[3]).max())
     for a, b in ((x0.grad, ref[4]), (u0.grad, ref[5])):
         assert np.allclose(a.cpu().numpy(), b, rtol=1e-7, atol=1e-8 * np.abs(b).max())
+
+
+@pytest.mark.parametrize("factor", [-3.0, 1e6, float("nan")])
+def test_adjoint_backward_with_other_charges_stays_in_its_scratch(factor):
+    """A backward whose kq is not the forward's finds other tiles than the forward counted: its gradients mean
+    nothing, but nothing outside the plan's scratch is written, and the next correct backward is unharmed."""
+    import ctypes as C
+    from crpropa3_amd import adjoint, capi
+    s = setup(n=300, N=32, nsteps=100, K=10, seed=5)
+    dev = torch.device("cuda:0")
+    L = adjoint._bind()
+    g = torch.tensor(s["grid"], device=dev)
+    x0, u0, kq, gu = (torch.tensor(s[k], device=dev) for k in ("x0", "u0", "kq", "target"))
+    cfg = adjoint._config(g, [0, 0, 0], [s["sp"]] * 3, 1.0, s["h"], s["nsteps"], s["K"])
+    plan = adjoint.AdjointPlan()
+    capi.check(L.crp_adjoint_plan_make(C.byref(cfg), 300, 1, C.byref(plan)))
+    assert plan.keep_states == 1
+    ckpt = torch.empty(plan.checkpoint_bytes // 8, dtype=torch.float64, device=dev)
+    xo, uo, gx0, gu0 = (torch.empty_like(x0) for _ in range(4))
+    size = -(-plan.scratch_bytes // 8)
+    guard = 1 << 20
+    scratch = torch.full((size + guard,), 7.0, dtype=torch.float64, device=dev)
+    gg = torch.zeros(g.numel() + 4096, dtype=torch.float64, device=dev)
+    gs = torch.zeros(1, dtype=torch.float64, device=dev)
+    p = adjoint._ptr
+    capi.check(L.crp_adjoint_forward_planned(C.byref(cfg), 300, C.byref(plan), p(x0), p(u0), p(kq), p(ckpt), p(xo), p(uo),
+                                             None))
+    kept = ckpt.clone()
+    res = []
+    for k in (kq, kq * factor, kq):
+        gg.zero_()
+        capi.check(L.crp_adjoint_backward_planned(C.byref(cfg), 300, C.byref(plan), p(k), p(ckpt), None, p(gu), p(scratch),
+                                                  p(gg), p(gx0), p(gu0), p(gs), None))
+        torch.cuda.synchronize()
+        assert (scratch[size:] == 7.0).all() and (gg[g.numel():] == 0).all()
+        assert torch.equal(ckpt.view(torch.int64), kept.view(torch.int64))
+        res.append((gx0.clone(), gu0.clone(), gg.clone()))
+    assert torch.equal(res[0][0], res[2][0]) and torch.equal(res[0][1], res[2][1])
+    assert torch.allclose(res[0][2], res[2][2], rtol=0, atol=1e-12 * float(res[0][2].abs().max()))

@@ -70,11 +70,22 @@ def _config(grid, origin, spacing, scale, step, nsteps, K):
     return cfg
 
 
+def _roomy(nbytes, device):
+    """Whether a buffer that lives until the backward leaves the card room: an eighth of what is free at most (small
+    ones always), so that many of them alive at once do not fill it and the rest of a program finds its memory."""
+    if nbytes <= 1 << 28 or torch.cuda.is_current_stream_capturing():
+        return True
+    free = torch.cuda.mem_get_info(device)[0]
+    if 8 * nbytes <= free:
+        return True
+    return 8 * nbytes <= free + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+
+
 class BorisGridFunction(torch.autograd.Function):
     """(grid, x0, u0, scale) -> (x_final, u_final); see the module docstring."""
 
     @staticmethod
-    def forward(ctx, grid, x0, u0, scale, kq, origin, spacing, step, nsteps, K):
+    def forward(ctx, grid, x0, u0, scale, kq, origin, spacing, step, nsteps, K, keep_states=None):
         if not (grid.is_cuda and x0.is_cuda and u0.is_cuda and kq.is_cuda):
             raise ValueError("BorisGridFunction: tensors must be on the GPU")
         grid = grid.detach().contiguous()
@@ -87,7 +98,10 @@ class BorisGridFunction(torch.autograd.Function):
         L = _bind()
         cfg = _config(grid, origin, spacing, float(scale), step, nsteps, K)
         plan = AdjointPlan()
-        capi.check(L.crp_adjoint_plan_make(C.byref(cfg), n, 1, C.byref(plan)))
+        keep = any(ctx.needs_input_grad) if keep_states is None else bool(keep_states)
+        capi.check(L.crp_adjoint_plan_make(C.byref(cfg), n, int(keep), C.byref(plan)))
+        if keep_states is None and plan.keep_states and not _roomy(plan.checkpoint_bytes, grid.device):
+            capi.check(L.crp_adjoint_plan_make(C.byref(cfg), n, 0, C.byref(plan)))
         ckpt = torch.empty(max(plan.checkpoint_bytes // 8, 1), dtype=torch.float64, device=grid.device)
         xo = torch.empty_like(x0c)
         uo = torch.empty_like(u0c)
@@ -119,21 +133,28 @@ class BorisGridFunction(torch.autograd.Function):
                                                   _ptr(gu), _ptr(scratch), _ptr(ggrid), _ptr(gx0), _ptr(gu0),
                                                   _ptr(gscale), stream))
         gs = gscale.view(()) if ctx.scale_is_tensor else None
-        return (ggrid.view(grid.shape).to(gdtype), gx0, gu0, gs, None, None, None, None, None, None)
+        return (ggrid.view(grid.shape).to(gdtype), gx0, gu0, gs, None, None, None, None, None, None, None)
 
 
 def boris_grid_propagate(grid, x0, u0, energy, charge, origin, spacing, step, nsteps, checkpoint_every=64,
-                         scale=1.0):
+                         scale=1.0, keep_states=None):
     """Differentiable fixed-step Boris push of particles through `scale * grid`.
 
     grid: (nx, ny, nz, 3) float32 CUDA tensor (periodic Grid3f values); x0, u0: (n, 3)
     float64 CUDA tensors (positions [m], unit directions); energy [J], charge [C]: (n,)
     tensors or floats.  `scale` may be a float or a 0-d tensor requiring grad.
-    Returns (x_final, u_final)."""
+    Between forward and backward the graph holds the state every `checkpoint_every` (K) steps, 48/K bytes a step
+    and particle, and the grid's cell table; or, with `keep_states`, the states every 8 steps, 6 bytes a step and
+    particle whatever K is, for a shorter backward (the same values).  keep_states None keeps them where a
+    backward can follow, they take at most 4 GiB and the card has eight times that free; False leaves K to bound
+    the memory.  Returns (x_final, u_final)."""
     dev = grid.device
     E = torch.as_tensor(energy, dtype=torch.float64, device=dev).expand(x0.shape[0])
     q = torch.as_tensor(charge, dtype=torch.float64, device=dev).expand(x0.shape[0])
     kq = (q * C_LIGHT * step / (2 * E)).contiguous()
     if not torch.is_tensor(scale):
         scale = torch.tensor(float(scale), dtype=torch.float64, device=dev)
-    return BorisGridFunction.apply(grid, x0, u0, scale, kq, origin, spacing, step, nsteps, checkpoint_every)
+    if keep_states is None and not torch.is_grad_enabled():
+        keep_states = False
+    return BorisGridFunction.apply(grid, x0, u0, scale, kq, origin, spacing, step, nsteps, checkpoint_every,
+                                   keep_states)

@@ -317,3 +317,56 @@ def test_adjoint_backward_with_other_charges_stays_in_its_scratch(factor):
         res.append((gx0.clone(), gu0.clone(), gg.clone()))
     assert torch.equal(res[0][0], res[2][0]) and torch.equal(res[0][1], res[2][1])
     assert torch.allclose(res[0][2], res[2][2], rtol=0, atol=1e-12 * float(res[0][2].abs().max()))
+
+
+def test_adjoint_checkpoint_interval_bounds_memory():
+    """What a graph holds until its backward: with keep_states False the states every K steps and the cell table;
+    without a backward to come nothing more is written either, and the default keeps 6 bytes a step.  The values
+    are the same bits (the grid gradient's FP64 sums in another order, then rounded to float32)."""
+    from crpropa3_amd import adjoint
+    n, nsteps, K, N = 4096, 256, 64, 16
+    s = setup(n=n, N=N, nsteps=nsteps, K=K, seed=51)
+    dev = torch.device("cuda:0")
+    E, target = torch.tensor(s["E"], device=dev), torch.tensor(s["target"], device=dev)
+    g = torch.tensor(s["grid"], dtype=torch.float32, device=dev, requires_grad=True)
+    x0 = torch.tensor(s["x0"], device=dev, requires_grad=True)
+    u0 = torch.tensor(s["u0"], device=dev, requires_grad=True)
+    few, many = 48 * n * (nsteps // K) + 128 * N ** 3, 6 * n * nsteps + 128 * N ** 3
+    slack = 48 * n * 3  # x, u, kq and the like
+
+    def run(**kw):
+        return adjoint.boris_grid_propagate(g, x0, u0, E, O.eplus, [0, 0, 0], [s["sp"]] * 3, s["h"], nsteps, K, **kw)
+
+    res = {}
+    for keep in (None, False, True):
+        before = torch.cuda.memory_allocated()
+        x, u = run(keep_states=keep)
+        held = torch.cuda.memory_allocated() - before
+        want = few if keep is False else many
+        assert want <= held <= want + slack + 4 * 8 * (n // 256) * 8, (keep, held)
+        res[keep] = (x.detach(), u.detach()) + torch.autograd.grad(((u - target) ** 2).sum(), (g, x0, u0))
+        del x, u
+    for keep in (False, True):
+        for a, b in zip(res[None], res[keep]):
+            if a.dtype == torch.float64:
+                assert torch.equal(a, b)
+            else:
+                assert torch.allclose(a, b, rtol=2.0 ** -23, atol=1e-12 * float(a.abs().max()))
+    with torch.no_grad():
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        x, u = run()
+        assert torch.cuda.max_memory_allocated() - before <= few + slack
+        assert torch.equal(x, res[None][0]) and torch.equal(u, res[None][1])
+
+
+def test_adjoint_keeps_no_states_on_a_full_card(monkeypatch):
+    """The default keeps the states only where the card has eight times their size free."""
+    from crpropa3_amd import adjoint
+    dev = torch.device("cuda:0")
+    assert adjoint._roomy(1 << 20, dev)
+    assert adjoint._roomy(1 << 30, dev)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (3 << 30, 288 << 30))
+    unused = torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
+    assert not adjoint._roomy((3 << 30) + unused, dev)
+    assert adjoint._roomy(1 << 28, dev)

@@ -157,7 +157,11 @@ static struct PinnedPool {
 	void *idle[kSlotsMax];
 	int nidle = 0, objects = 0;
 
-	void *take() { // nullptr: no pinned memory to be had
+	// nullptr: no pinned memory to be had (CRP_PINNED_SLOTS=0, read at each call, says so, for tests of what follows)
+	void *take() {
+		const char *e = std::getenv("CRP_PINNED_SLOTS");
+		if (e && std::atoi(e) == 0)
+			return nullptr;
 		{
 			std::lock_guard<std::mutex> g(lock);
 			if (nidle > 0)
@@ -2341,6 +2345,25 @@ int crp_batch_upload(crp_batch_t *b, size_t n, const crp_host_state *s) {
 	return CRP_OK;
 }
 
+// crp_batch_download without pinned memory: array by array
+static int download_pageable(const crp_batch *b, const PackArgs &A, double *const *dst3, double *const *dst1,
+                             char *const *dstw) {
+	const size_t n = b->n;
+	CRP_HIP_TRY(hipStreamSynchronize(b->stream));
+	std::vector<double> col(n);
+	for (int k = 0; k < A.n3; k++)
+		for (int c = 0; c < 3; c++) {
+			CRP_HIP_TRY(hipMemcpy(col.data(), A.v3[k][c], n * sizeof(double), hipMemcpyDeviceToHost));
+			for (size_t i = 0; i < n; i++)
+				dst3[k][3 * i + c] = col[i];
+		}
+	for (int k = 0; k < A.n1; k++)
+		CRP_HIP_TRY(hipMemcpy(dst1[k], A.d1[k], n * sizeof(double), hipMemcpyDeviceToHost));
+	for (int k = 0; k < A.nw; k++)
+		CRP_HIP_TRY(hipMemcpy(dstw[k], A.w1[k], n * sizeof(uint32_t), hipMemcpyDeviceToHost));
+	return CRP_OK;
+}
+
 int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 	if (!b || !s)
 		return fail(CRP_E_INVALID, "crp_batch_download: NULL argument");
@@ -2389,8 +2412,10 @@ int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 	std::atomic<int> err{(int)hipSuccess};
 	auto worker = [&](int w) {
 		double *const slot = (double *)gPinned.take();
+		if (!slot) // the chunks are left to the others
+			return;
 		hipEvent_t ev = nullptr;
-		hipError_t e = slot ? hipSetDevice(b->device) : hipErrorOutOfMemory;
+		hipError_t e = hipSetDevice(b->device);
 		if (e == hipSuccess)
 			e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
 		const bool ready = e == hipSuccess;
@@ -2418,8 +2443,7 @@ int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 			(void)hipEventDestroy(ev);
 		if (e != hipSuccess && ready)
 			(void)hipStreamSynchronize(b->stream); // nothing writes to the slot any more
-		if (slot)
-			gPinned.give(slot);
+		gPinned.give(slot);
 		if (e != hipSuccess && (ready || w == 0)) // a helper that could not start leaves its chunks to the others
 			err = (int)e;
 	};
@@ -2437,6 +2461,8 @@ int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 	CRP_HIP_TRY(hipSetDevice(caller));
 	if (err != (int)hipSuccess)
 		return fail(CRP_E_HIP, std::string("crp_batch_download: ") + hipGetErrorString((hipError_t)err.load()));
+	if (nextChunk < nchunk) // nobody had a slot
+		return download_pageable(b, A, dst3, dst1, dstw);
 	return CRP_OK;
 }
 
@@ -2463,9 +2489,24 @@ int crp_batch_detections(const crp_batch_t *b, int ntimes, double *out) {
 		return CRP_OK;
 	const int kk = std::min(ntimes, b->snap ? b->snapK : 0);
 	const size_t rec = kSnapDoubles * sizeof(double), chunk = std::min(n, kSlotBytes / rec);
+	std::fill(out + (size_t)kk * n * kSnapDoubles, out + (size_t)ntimes * n * kSnapDoubles, NAN);
+	if (kk == 0)
+		return CRP_OK;
 	double *const slot = (double *)gPinned.take();
-	if (!slot)
-		return fail(CRP_E_NOMEM, "crp_batch_detections: no pinned memory");
+	if (!slot) { // column by column
+		CRP_HIP_TRY(hipStreamSynchronize(b->stream));
+		std::vector<int32_t> det(n);
+		std::vector<double> col(n);
+		CRP_HIP_TRY(hipMemcpy(det.data(), b->det, n * sizeof(int32_t), hipMemcpyDeviceToHost));
+		for (int k = 0; k < kk; k++)
+			for (int c = 0; c < kSnapDoubles; c++) {
+				CRP_HIP_TRY(hipMemcpy(col.data(), b->snap + ((size_t)k * kSnapDoubles + c) * b->cap, n * sizeof(double),
+				                      hipMemcpyDeviceToHost));
+				for (size_t i = 0; i < n; i++)
+					out[((size_t)k * n + i) * kSnapDoubles + c] = k < det[i] ? col[i] : NAN;
+			}
+		return CRP_OK;
+	}
 	hipError_t e = hipSuccess;
 	for (int k = 0; k < kk && e == hipSuccess; k++)
 		for (size_t i0 = 0; i0 < n && e == hipSuccess; i0 += chunk) {
@@ -2482,7 +2523,6 @@ int crp_batch_detections(const crp_batch_t *b, int ntimes, double *out) {
 	gPinned.give(slot);
 	if (e != hipSuccess)
 		return fail(CRP_E_HIP, std::string("crp_batch_detections: ") + hipGetErrorString(e));
-	std::fill(out + (size_t)kk * n * kSnapDoubles, out + (size_t)ntimes * n * kSnapDoubles, NAN);
 	return CRP_OK;
 }
 

@@ -204,3 +204,26 @@ def test_tricubic_row_table(kind, fixed, shape, clip):
         out = b.download()
         for k in ("pos", "dir", "next_step", "trajectory_length"):
             assert same(out[k], getattr(ref, k)[idx]), k
+
+
+def test_transfers_without_pinned_memory(monkeypatch):
+    """With no pinned memory to be had, downloads, detections and field samples return the same bytes; a batch
+    without detections needs none."""
+    rng = np.random.default_rng(41)
+    n = 25001
+    f = capi.Field.grid3f(noise((8, 9, 7)), [0, 0, 0], [20 * KPC] * 3)
+    pos = rng.uniform(0, 150 * KPC, (n, 3))
+    p = capi.Propagator("BP", f, 1e-3, 5 * KPC, 5 * KPC, max_length=60 * KPC)
+    p.set_observer([12 * KPC, 31 * KPC, 49 * KPC, 200 * KPC])
+    b, empty = capi.Batch(n), capi.Batch(n)
+    for x in (b, empty):
+        x.upload(pos, O.normalise(rng.normal(size=(n, 3))), 10 ** rng.uniform(0, 2, n) * EEV, np.full(n, EPLUS))
+    p.propagate(b, max_steps=8)
+    got = [b.download(), b.detections(4), empty.detections(2), f.eval(pos)]
+    monkeypatch.setenv("CRP_PINNED_SLOTS", "0")
+    ref = [b.download(), b.detections(4), empty.detections(2), f.eval(pos)]
+    assert np.isnan(got[2]).all() and np.isfinite(got[1][0]).all() and np.isnan(got[1][3]).all()
+    for k in got[0]:
+        assert np.array_equal(got[0][k].view(np.uint8), ref[0][k].view(np.uint8)), k
+    for a, c in zip(got[1:], ref[1:]):
+        assert np.array_equal(a.view(np.uint64), c.view(np.uint64))

@@ -196,6 +196,23 @@ static struct PinnedPool {
 	}
 } gPinned;
 
+// makes `device` current for a scope: a batch's kernels are launched on its own device from whichever one is
+// current, and pinned memory and events are made there
+struct OnDevice {
+	int before = -1;
+	hipError_t e;
+	explicit OnDevice(int device) {
+		e = hipGetDevice(&before);
+		if (e == hipSuccess && before != device)
+			e = hipSetDevice(device);
+	}
+	~OnDevice() {
+		if (before >= 0)
+			(void)hipSetDevice(before);
+	}
+	OnDevice(const OnDevice &) = delete;
+};
+
 static Soa soa_of(const crp_batch *b) {
 	Soa s;
 	s.px = b->px; s.py = b->py; s.pz = b->pz;
@@ -2411,13 +2428,12 @@ int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 	std::atomic<size_t> nextChunk{0};
 	std::atomic<int> err{(int)hipSuccess};
 	auto worker = [&](int w) {
-		double *const slot = (double *)gPinned.take();
+		const OnDevice on(b->device); // before the slot: a thread's first call would open device 0
+		double *const slot = on.e == hipSuccess ? (double *)gPinned.take() : nullptr;
 		if (!slot) // the chunks are left to the others
 			return;
 		hipEvent_t ev = nullptr;
-		hipError_t e = hipSetDevice(b->device);
-		if (e == hipSuccess)
-			e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+		hipError_t e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
 		const bool ready = e == hipSuccess;
 		for (size_t c; e == hipSuccess && (c = nextChunk++) < nchunk;) {
 			const size_t i0 = c * chunk, m = std::min(chunk, n - i0);
@@ -2447,8 +2463,6 @@ int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 		if (e != hipSuccess && (ready || w == 0)) // a helper that could not start leaves its chunks to the others
 			err = (int)e;
 	};
-	int caller = 0;
-	CRP_HIP_TRY(hipGetDevice(&caller));
 	std::vector<std::thread> team;
 	try {
 		for (int w = 1; w < nthread; w++)
@@ -2458,7 +2472,6 @@ int crp_batch_download(const crp_batch_t *b, crp_host_state *s) {
 	worker(0);
 	for (std::thread &t : team)
 		t.join();
-	CRP_HIP_TRY(hipSetDevice(caller));
 	if (err != (int)hipSuccess)
 		return fail(CRP_E_HIP, std::string("crp_batch_download: ") + hipGetErrorString((hipError_t)err.load()));
 	if (nextChunk < nchunk) // nobody had a slot
@@ -2492,6 +2505,8 @@ int crp_batch_detections(const crp_batch_t *b, int ntimes, double *out) {
 	std::fill(out + (size_t)kk * n * kSnapDoubles, out + (size_t)ntimes * n * kSnapDoubles, NAN);
 	if (kk == 0)
 		return CRP_OK;
+	const OnDevice on(b->device);
+	CRP_HIP_TRY(on.e);
 	double *const slot = (double *)gPinned.take();
 	if (!slot) { // column by column
 		CRP_HIP_TRY(hipStreamSynchronize(b->stream));

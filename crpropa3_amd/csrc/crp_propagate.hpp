@@ -249,8 +249,9 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 			else
 				yOut.x = v3(pos.x + dir.x * step, pos.y + dir.y * step, pos.z + dir.z * step);
 		};
-		// the trial of a fixed step, and of an adaptive one (returns the error over the tolerance)
-		auto fixed_trial = [&]() {
+		// the trial of a fixed step, and of an adaptive one (returns the error over the tolerance); `own`: the lane has
+		// one, where the straight line's range tests decide (they fail for lanes without a charged particle)
+		auto fixed_trial = [&](bool own) {
 			if (MIX) {
 				if (kCK) {
 					double eU;
@@ -272,7 +273,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 						bool bad = !bp_in_range(q, m_, step);
 						yOut = bp_dy_fast(field, pos, dir, step, q, m_, im_, bad);
 						nDir = unit_twice_fast<true>(yOut.u, bad);
-						if (bad) {
+						if (bad && own) {
 							yOut = bp_dy(field.lane_field(), pos, dir, step, q, m_, im_);
 							nDir = unit_twice_tested(yOut.u);
 						}
@@ -282,7 +283,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 				}
 			}
 		};
-		auto adaptive_trial = [&]() -> double {
+		auto adaptive_trial = [&](bool own) -> double {
 			if (MIX) {
 				if (kCK) {
 					double eU;
@@ -319,7 +320,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 				cmp = bp_dy_fast(field, half.x, half.u, step / 2, q, m_, im_, bad);
 				nDir = unit_twice_fast<true>(yOut.u, bad);
 			}
-			if (!kFast || bad) {
+			if (!kFast || (bad && own)) {
 				auto &&f = lane_field(field);
 				yOut = bp_dy(f, pos, dir, step, q, m_, im_);
 				const Y half = bp_dy(f, pos, dir, step / 2, q, m_, im_);
@@ -373,7 +374,7 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 				step = P.maxStep;
 				newStep = step;
 				if (!kWave)
-					fixed_trial();
+					fixed_trial(true);
 				nEval += kEvalsPerTrial;
 				commit = true;
 			} else {
@@ -388,9 +389,9 @@ k_propagate(F field0, Params P, Soa S, unsigned long long n,
 		if (kWave && !go)
 			b0.have = b0f.have = true; // asks for no evaluation of its own
 		if (kWave && !kAdaptive)
-			fixed_trial();
+			fixed_trial(have && !neutral);
 		if (kAdaptive && (kWave || go)) {
-			const double r = adaptive_trial();
+			const double r = adaptive_trial(!kWave || go);
 			if (go)
 				step_control(r);
 		}

@@ -725,12 +725,21 @@ static int dispatch_kind(const F &f, const crp_propagator *p, const Params &P, c
 // (FieldGridCellsWave).  The rate of a lane's own loads falls from 5.3e10 lines/s at 2 GiB and 4.9e10 at
 // 3.0 GB to 1.7e10 at 3.2 GB and 1.3e10 at 17 GB; the waves' loads reach 4.9e10 at 3.2 GB and 4.6e10 at
 // 17 GB.  Line numbers are 32 bits.
+// A wave's gather takes as long however many of its lanes have a particle, and a batch of fewer than 64 to a SIMD
+// leaves lanes without one.  Up to about 44 to a SIMD the lanes' own loads are faster for every kind of step and both
+// precisions (4 GB, adaptive Cash-Karp: 40000 particles 23.5 us a step against 27.9, 4096 19.6 against 23.2), beyond
+// it the waves' (49152 28.9 against 29.7, 65536 28.3 against 38.8).
 constexpr size_t kWaveGatherBytes = 3000000000ull;
+constexpr size_t kWaveGatherPerCU = 4 * 44;
 
 static int dispatch_cells(const FieldGridCells &f, const crp_propagator *p, const Params &P, crp_batch *b,
                           int *launches) {
 	const size_t ncell = (size_t)f.g.nx * f.g.ny * f.g.nz;
-	if (p->type == 2 || ncell * kCellFloats * sizeof(float) <= kWaveGatherBytes || ncell > 0xffffffffull)
+	const int ncu = num_cus();
+	if (ncu < 0)
+		return CRP_E_HIP;
+	if (p->type == 2 || ncell * kCellFloats * sizeof(float) <= kWaveGatherBytes || ncell > 0xffffffffull ||
+	    b->n < kWaveGatherPerCU * (size_t)ncu)
 		return dispatch_kind(f, p, P, b, launches);
 	const FieldGridCellsBig big{f};
 	return p->precision == CRP_PRECISION_MIXED ? dispatch_kind_p<FieldGridCellsBig, true>(big, p, P, b, launches)

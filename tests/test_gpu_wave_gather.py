@@ -71,3 +71,31 @@ def test_wave_gather_mixed(fields, kind, fixed):
     b, _ = _run(fields[False, "cells"], kind, fixed, 1000, steps, capi.PRECISION_FP64)
     err = np.abs(a["pos"] - b["pos"]).max(axis=1) / np.abs(b["pos"]).max()
     assert err.max() < 1e-8
+
+
+@pytest.mark.parametrize("n", [45055, 45056, 45057, 66001])
+@pytest.mark.parametrize("clip", [False, True])
+@pytest.mark.parametrize("fixed", [True, False])
+@pytest.mark.parametrize("kind", ["BP", "CK"])
+def test_batches_around_the_switch_to_wave_gathers(fields, kind, fixed, clip, n):
+    """Waves gather from 176 particles to a compute unit on (45056 on 256 units), the lanes' own loads serve smaller
+    batches: either side of the line, a ragged last wave, and enough particles that lanes take a second one."""
+    print(kind, fixed, clip, n, flush=True)
+    a, sa = _run(fields[clip, "cells"], kind, fixed, n, 6, capi.PRECISION_FP64)
+    b, sb = _run(fields[clip, "points"], kind, fixed, n, 6, capi.PRECISION_FP64)
+    assert sa.accepted_steps == sb.accepted_steps and sa.rejected_trials == sb.rejected_trials
+    for k in a:
+        assert np.array_equal(a[k].view(np.uint8), b[k].view(np.uint8)), k
+
+
+@pytest.mark.parametrize("n", [45055, 45056, 66001])
+@pytest.mark.parametrize("fixed", [True, False])
+@pytest.mark.parametrize("kind", ["BP", "CK"])
+def test_wave_gather_mixed_large_batches(fields, kind, fixed, n):
+    """test_wave_gather_mixed's bound where the waves gather."""
+    print(kind, fixed, n, flush=True)
+    steps = 3 if fixed else 1
+    a, _ = _run(fields[False, "cells"], kind, fixed, n, steps, capi.PRECISION_MIXED)
+    b, _ = _run(fields[False, "points"], kind, fixed, n, steps, capi.PRECISION_FP64)
+    err = np.abs(a["pos"] - b["pos"]).max(axis=1) / np.abs(b["pos"]).max()
+    assert err.max() < 1e-8

@@ -280,10 +280,12 @@ __device__ __forceinline__ double mirror_fold(double x, int n, double invn) {
 }
 
 __device__ __forceinline__ void reflective_clamp(double x, int n, double invn, int &lo, int &hi, double &frac) {
-	if (__builtin_fabs(x) < 0x1p50)
-		x = mirror_fold(x, n, invn);
-	while ((x < -0.5) || (x > (n - 0.5)))
-		x = 2 * n * (x > (n - 0.5)) - x - 1;
+	if ((x < -0.5) || (x > (n - 0.5))) { // most positions are inside, and a wave of them takes none of this
+		if (__builtin_fabs(x) < 0x1p50)
+			x = mirror_fold(x, n, invn);
+		while ((x < -0.5) || (x > (n - 0.5)))
+			x = 2 * n * (x > (n - 0.5)) - x - 1;
+	}
 	double fl = __builtin_floor(x);
 	lo = (int)fl;
 	hi = lo + (lo < n - 1);

@@ -25,6 +25,7 @@
 #include <mutex>
 #include <string>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "crp_device.hpp"
@@ -563,6 +564,53 @@ static auto propagate_kernel() {
 		return k_propagate<F, KIND, MIX>;
 }
 
+// steps of a particle in a run, at least
+static double run_steps(const Params &P) {
+	double steps = P.maxSteps >= 0 ? (double)P.maxSteps : HUGE_VAL;
+	if (P.maxLen > 0 && P.maxStep > 0)
+		steps = std::min(steps, P.maxLen / P.maxStep);
+	return steps;
+}
+
+// a grid whose cell table outgrows the first-level address translation (dispatch_cells)
+constexpr size_t kWaveGatherBytes = 3000000000ull;
+template <class F> static bool beyond_translation(const F &) { return false; }
+static bool beyond_translation(const FieldGridCells &f) {
+	return (size_t)f.g.nx * f.g.ny * f.g.nz * kCellFloats * sizeof(float) > kWaveGatherBytes;
+}
+
+// Particles that a wave of a small batch takes at least, 0 for the general rule of launch_propagate: where all
+// lanes go the same way, a uniform field or fixed steps through anything but the branches of JF12 and of
+// composites.  In a short run the start of a launch over more units takes longer than fuller waves lose.  Us a step, one wave to a unit (below 4096) or waves of 16 / 32 / 64:
+//   uniform, 1000, 100 fixed Boris steps 1.97 / 1.58 / 1.58; 32768 2.81 / 2.78 / 2.16; SDE 1000 9.3 / 7.4 / 7.4
+//   grid, fixed Cash-Karp, 1000 7.72 / 6.85 / 6.98; 8192 7.27 / 7.37 / 7.88, over 2000 steps 6.72 / 7.06 / 7.72
+//   grid, fixed Boris, 1000 2.14 / 1.79 / 1.69; 16384 2.93 / 2.30 / 2.10, over 2000 steps 1.65 / 1.65 / 1.69
+//   the same, mixed, 16384 2.50 / 1.85 / 1.71, over 2000 steps 1.23 / 1.25 / 1.31; 1000 over 2000 1.16 / 1.23 / 1.30
+//   plane waves, fixed Boris, 1000 63.5 / 57.0 / 62.3; 8192 55.4 / 57.2 / 62.6
+//   table of 4.2 GB, fixed Boris, 1000 2.12 / 1.72 / 2.47, 16384 2.98 / 2.37 / 2.85, over 2000 steps 1.83 / 1.89 / 2.64;
+//     fixed Cash-Karp, 1000 over 2000 steps 7.38 / 7.50 / 13.4
+template <class F, int KIND, bool MIX>
+static size_t least_lanes(const F &f, const Params &P, size_t n, int ncu) {
+	constexpr bool grid = std::is_same<F, FieldGridCells>::value || std::is_same<F, FieldGrid>::value ||
+	                      std::is_same<F, FieldGridCells16>::value;
+	constexpr bool waves = std::is_same<F, FieldPlaneWave>::value;
+	constexpr bool apart = std::is_same<F, FieldJF12Ref<false>>::value || std::is_same<F, FieldJF12Ref<true>>::value ||
+	                       std::is_same<F, FieldComposite>::value;
+	if (std::is_same<F, FieldUniform>::value || std::is_same<F, FieldNone>::value)
+		return 64;
+	if (apart || (KIND != PK_BP_FIXED && KIND != PK_CK_FIXED))
+		return 0;
+	const bool many = n >= (size_t)ncu * 64;
+	const double steps = run_steps(P);
+	if (KIND == PK_BP_FIXED && !waves && steps <= (many ? 512 : 200))
+		return grid && !beyond_translation(f) ? 64 : 32;
+	if (MIX || (KIND == PK_CK_FIXED && beyond_translation(f)))
+		return 0;
+	if (KIND == PK_CK_FIXED && !waves && many && steps <= 200)
+		return 32;
+	return n < (size_t)ncu * 16 ? 32 : 16;
+}
+
 template <class F, int KIND, bool MIX>
 static int launch_propagate(const F &f, const crp_propagator *p, const Params &Pin, crp_batch *b, int *launches) {
 	auto kern = propagate_kernel<F, KIND, MIX>();
@@ -584,14 +632,18 @@ static int launch_propagate(const F &f, const crp_propagator *p, const Params &P
 	// unit (8192 particles in waves of 8, four to a unit: a Cash-Karp step takes 76 us in JF12 and 32 in a grid,
 	// in waves of 16 41 and 22; 64 particles one to a wave: 104 us in JF12, 46 with one wave to a unit): below 16
 	// particles to a unit, each has one wave, and from there on waves of 16 or more (2048 particles: the grid's
-	// step 49 us with one wave to a unit, 53 in waves of 16; plane waves 11 and 14; at 4096 10.8 and 9.1).
+	// step 49 us with one wave to a unit, 53 in waves of 16; at 4096 10.8 and 9.1).
+	// That pays where the particles of a wave run apart.  A launch also takes longer while more units fetch the code,
+	// whatever its length (100 and 400 mixed Boris steps in waves of 16 rather than 64: 8192 particles 23 us, 16384 60
+	// to 80), and where nothing runs apart a fuller wave loses little or nothing (least_lanes).
 	// Groups of lanes on a particle always fill their waves (1000 particles, a tricubic Boris step: 3.1 us, 3.6
 	// with fewer).
 	constexpr size_t group = KIND == PK_SDE ? 1 : LaneGroup<typename KernelField<F, MIX>::type>::value;
-	const bool lone = group == 1 && b->n < (size_t)ncu * 16;
+	const size_t fill = least_lanes<F, KIND, MIX>(f, Pin, b->n, ncu);
+	const bool lone = group == 1 && fill == 0 && b->n < (size_t)ncu * 16;
 	const int active = lone ? 1 : block / 64; // waves of a workgroup that take particles
 	const size_t waves = std::min<size_t>((size_t)ncu * bpc * active, (size_t)ncu * (lone ? 1 : 4));
-	const size_t least = lone ? 1 : 16;
+	const size_t least = lone ? 1 : std::max<size_t>(16, fill);
 	const int lanes = (int)std::min<size_t>(64, group * std::max<size_t>(least, (b->n + waves - 1) / waves));
 	const size_t perBlock = (size_t)lanes / group * active;
 	const size_t want = (b->n + perBlock - 1) / perBlock;
@@ -729,7 +781,6 @@ static int dispatch_kind(const F &f, const crp_propagator *p, const Params &P, c
 // leaves lanes without one.  Up to about 44 to a SIMD the lanes' own loads are faster for every kind of step and both
 // precisions (4 GB, adaptive Cash-Karp: 40000 particles 23.5 us a step against 27.9, 4096 19.6 against 23.2), beyond
 // it the waves' (49152 28.9 against 29.7, 65536 28.3 against 38.8).
-constexpr size_t kWaveGatherBytes = 3000000000ull;
 constexpr size_t kWaveGatherPerCU = 4 * 44;
 
 static int dispatch_cells(const FieldGridCells &f, const crp_propagator *p, const Params &P, crp_batch *b,
@@ -738,7 +789,7 @@ static int dispatch_cells(const FieldGridCells &f, const crp_propagator *p, cons
 	const int ncu = num_cus();
 	if (ncu < 0)
 		return CRP_E_HIP;
-	if (p->type == 2 || ncell * kCellFloats * sizeof(float) <= kWaveGatherBytes || ncell > 0xffffffffull ||
+	if (p->type == 2 || !beyond_translation(f) || ncell > 0xffffffffull ||
 	    b->n < kWaveGatherPerCU * (size_t)ncu)
 		return dispatch_kind(f, p, P, b, launches);
 	const FieldGridCellsBig big{f};
@@ -759,10 +810,7 @@ static bool tricubic_rows(const GridDesc &g, const crp_propagator *p, const Para
 	if (g.interp != kInterpTricubic || g.reflective || b->n <= kQuadParticles || bytes > kRowsBytesMax)
 		return false;
 	const double evals = p->type == 1 ? 6 : (P.minStep == P.maxStep ? 1 : 3);
-	double steps = P.maxSteps >= 0 ? (double)P.maxSteps : HUGE_VAL;
-	if (P.maxLen > 0 && P.maxStep > 0)
-		steps = std::min(steps, P.maxLen / P.maxStep); // at least
-	if (steps * evals * (double)b->n < 2.0 * (double)ncell)
+	if (run_steps(P) * evals * (double)b->n < 2.0 * (double)ncell)
 		return false;
 	if (b->rowsBytes < bytes) {
 		if (b->rows)

@@ -227,3 +227,36 @@ def test_transfers_without_pinned_memory(monkeypatch):
         assert np.array_equal(got[0][k].view(np.uint8), ref[0][k].view(np.uint8)), k
     for a, c in zip(got[1:], ref[1:]):
         assert np.array_equal(a.view(np.uint64), c.view(np.uint64))
+
+
+@pytest.mark.parametrize("n", [1, 31, 33, 4095, 4097, 16383, 16385, 33000])
+@pytest.mark.parametrize("name,kind,steps", [("grid", "BP", 20), ("grid", "BP", 520), ("grid", "CK", 20), ("reflective", "CK", 220),
+                                             ("uniform", "BP", 20), ("uniform", "CK", 20)])
+def test_fixed_steps_of_small_batches(name, kind, steps, n):
+    """Fixed steps fill their waves fuller, by batch, field and length of the run: a particle's steps do not depend
+    on it, on either path."""
+    rng = np.random.default_rng(29)
+    m = 97
+    g, sp = noise((16, 16, 16)), [50 * KPC] * 3
+    pos, d, E = rng.uniform(-100 * KPC, 900 * KPC, (m, 3)), rng.normal(size=(m, 3)), 10 ** rng.uniform(0, 2, m) * EEV
+    q = np.where(np.arange(m) % 5 == 0, 0.0, EPLUS)
+    if name == "uniform":
+        B = (1e-13, -2e-13, 3e-14)
+        f, of = capi.Field.uniform(B), O.OracleField.uniform(B)
+    else:
+        r = name == "reflective"
+        f, of = capi.Field.grid3f(g, [0, 0, 0], sp, reflective=r), O.OracleField.grid(g, [0, 0, 0], sp, r)
+    i, h = np.arange(n) % m, 20 * KPC
+    ref = O.OracleState(pos, d, E, q)
+    O.propagate(of, O.PROP_BP if kind == "BP" else O.PROP_CK, ref, steps, min_step=h, max_step=h, libm=O.LIBM_CR)
+    for precision in (capi.PRECISION_FP64, capi.PRECISION_MIXED):
+        b = capi.Batch(n)
+        b.upload(pos[i], O.normalise(d)[i], E[i], q[i])
+        st = capi.Propagator(kind, f, 1e-3, h, h, precision=precision).propagate(b, max_steps=steps)
+        out = b.download()
+        assert st.accepted_steps == steps * n
+        for k in ("pos", "dir", "next_step", "trajectory_length"):
+            if precision == capi.PRECISION_FP64:
+                assert same(out[k], getattr(ref, k)[i]), k
+            else:
+                assert same(out[k], out[k][:m][i]), k

@@ -798,16 +798,23 @@ static int dispatch_cells(const FieldGridCells &f, const crp_propagator *p, cons
 }
 
 // Tricubic grids.  Up to kQuadParticles a batch leaves lanes idle and is bound by each particle's chain: four
-// lanes share a particle (128^3 grid, 300 Boris steps: 1000 to 16384 particles in 1.5 - 2.0 ms against 3.9, 32768
-// in 3.8 against 4.4); above, by the rate of line requests (65536: 7.2 ms with quads, 6.1 a lane each), and a table
-// of row pairs pays where the run evaluates the field more often than the table has entries.
+// lanes share a particle; above, by the rate of line requests, and a table of row pairs pays where the run evaluates
+// the field more often than the table has entries.  Quads and the table, us a step (quads / table):
+//   48^3, points within an XCD's 4 MB of L2: fixed Boris 28000 6.8 / 7.3, 32768 7.3 / 7.5, 33000 9.1 / 7.5; adaptive
+//     Cash-Karp 32768 44 / 57, 40000 55 / 60
+//   128^3, points beyond it: fixed Cash-Karp 16384 23 / 30, 20000 36 / 31, 24000 38 / 32, 32768 56 / 34; adaptive Boris
+//     24000 32 / 34, 28000 36 / 34; adaptive Cash-Karp 20000 53 / 57, 24000 58 / 57, 28000 67 / 60
+// Without the table (reflective, or too few evaluations) the one lane a particle reads from 32768 on.
 constexpr size_t kQuadParticles = 32768;
+constexpr size_t kQuadParticlesFar = 22528; // and a table, points beyond kNearBytes
+constexpr size_t kNearBytes = (size_t)4 << 20;
 constexpr size_t kRowsBytesMax = (size_t)2 << 30;
 
 // whether this run reads a row-pair table; builds it on the batch's stream
 static bool tricubic_rows(const GridDesc &g, const crp_propagator *p, const Params &P, crp_batch *b) {
 	const size_t ncell = (size_t)g.nx * g.ny * g.nz, bytes = ncell * 32 * sizeof(float);
-	if (g.interp != kInterpTricubic || g.reflective || b->n <= kQuadParticles || bytes > kRowsBytesMax)
+	const size_t quads = ncell * 3 * sizeof(float) > kNearBytes ? kQuadParticlesFar : kQuadParticles;
+	if (g.interp != kInterpTricubic || g.reflective || b->n <= quads || bytes > kRowsBytesMax)
 		return false;
 	const double evals = p->type == 1 ? 6 : (P.minStep == P.maxStep ? 1 : 3);
 	if (run_steps(P) * evals * (double)b->n < 2.0 * (double)ncell)

@@ -260,3 +260,30 @@ def test_fixed_steps_of_small_batches(name, kind, steps, n):
                 assert same(out[k], getattr(ref, k)[i]), k
             else:
                 assert same(out[k], out[k][:m][i]), k
+
+
+@pytest.mark.parametrize("n", [22528, 22529, 32768, 32769])
+@pytest.mark.parametrize("shape", [(73, 72, 71), (33, 6, 19)])
+@pytest.mark.parametrize("kind,fixed", [("BP", True), ("CK", False)])
+def test_tricubic_switch_from_quads_to_the_row_table(kind, fixed, shape, n):
+    """Either side of both lines (points beyond and within 4 MB): copies of the same particles against the oracle."""
+    rng = np.random.default_rng(19)
+    m = 257
+    sp, steps = [20 * KPC] * 3, 40 if fixed else 7
+    g = noise(shape)
+    pos, d, E = rng.uniform(-0.6, 1.6, (m, 3)) * np.array(shape) * 20 * KPC, rng.normal(size=(m, 3)), \
+        10 ** rng.uniform(0, 2, m) * EEV
+    q = np.where(np.arange(m) % 6 == 1, 0.0, EPLUS)
+    lo, hi = (20 * KPC, 20 * KPC) if fixed else (KPC, 60 * KPC)
+    f = capi.Field.grid3f(g, [0, 0, 0], sp)
+    f.set_interpolation("TRICUBIC")
+    ref = O.OracleState(pos, d, E, q)
+    O.propagate(O.OracleField.grid(g, [0, 0, 0], sp, interp=O.GRID_TRICUBIC), O.PROP_BP if kind == "BP" else O.PROP_CK,
+                ref, steps, tolerance=1e-3, min_step=lo, max_step=hi, libm=O.LIBM_CR)
+    idx = np.arange(n) % m
+    b = capi.Batch(n)
+    b.upload(pos[idx], O.normalise(d)[idx], E[idx], q[idx])
+    capi.Propagator(kind, f, 1e-3, lo, hi).propagate(b, max_steps=steps)
+    out = b.download()
+    for k in ("pos", "dir", "next_step", "trajectory_length"):
+        assert same(out[k], getattr(ref, k)[idx]), k

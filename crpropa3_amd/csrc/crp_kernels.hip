@@ -1709,9 +1709,15 @@ int crp_field_create_planewave(int nm, const double *k, const double *Ak, const 
 		f->owned[j] = d;
 	}
 	double most = 0; // the largest phase gradient; a phase of 2^18 turns holds the bias too
-	for (int i = 0; i < nm; i++)
-		most = std::max({most, std::fabs(mm[i].ktx), std::fabs(mm[i].kty), std::fabs(mm[i].ktz), std::fabs(mm[i].bt) > 0x1p17 ? HUGE_VAL : 0.0});
-	f->pw.reach = most > 0 && most < HUGE_VAL ? 0x1p17 / most : 0.0;
+	bool plain = true; // a mode that is not finite shows in the FP64 fraction and not in the phase's low word
+	for (int i = 0; i < nm; i++) {
+		for (double k : {mm[i].ktx, mm[i].kty, mm[i].ktz}) {
+			plain &= std::isfinite(k);
+			most = std::max(most, std::fabs(k));
+		}
+		plain &= std::fabs(mm[i].bt) <= 0x1p17;
+	}
+	f->pw.reach = plain && most > 0 ? 0x1p17 / most : 0.0;
 	f->pw.nm = nm;
 	f->pw.m64 = (const PwMode64 *)f->owned[0];
 	f->pw.mm = (const PwModeMixed *)f->owned[1];

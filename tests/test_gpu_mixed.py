@@ -174,3 +174,23 @@ def test_fp16_brick_storage_propagation():
     dr = np.linalg.norm(ref["pos"] - pos, axis=1)
     dm = np.linalg.norm(m["pos"] - pos, axis=1)
     assert _ks_equivalent(dm, dr, "FP16 displacement") > 1e-3
+
+
+@pytest.mark.parametrize("which", ["k", "kappa", "beta"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_mixed_planewave_mode_that_is_not_finite(which, value):
+    """A mode whose phase is NaN makes the field NaN on both paths, as a sum of cosines does."""
+    rng = np.random.default_rng(3)
+    nm, n = 9, 70
+    k = 2 * np.pi / np.linspace(1, 9, nm) / 1e17
+    kappa, xi = O.normalise(rng.normal(size=(nm, 3))), O.normalise(rng.normal(size=(nm, 3)))
+    beta = rng.uniform(0, 6, nm)
+    dict(k=k, kappa=kappa, beta=beta)[which].reshape(-1)[4] = value
+    f = capi.Field.planewave(k, np.full(nm, 1e-10), xi, kappa, beta)
+    pos, d = rng.uniform(-1e18, 1e18, (n, 3)), O.normalise(rng.normal(size=(n, 3)))
+    for precision in (capi.PRECISION_FP64, capi.PRECISION_MIXED):
+        b = capi.Batch(n)
+        b.upload(pos, d, np.full(n, 1e16 * O.eV), np.full(n, O.eplus))
+        capi.Propagator("BP", f, 1e-3, 1e15, 1e15, precision=precision).propagate(b, max_steps=2)
+        assert np.isnan(f.eval(pos, precision)).all()
+        assert np.isnan(b.download()["dir"]).all()

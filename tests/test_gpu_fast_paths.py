@@ -287,3 +287,35 @@ def test_tricubic_switch_from_quads_to_the_row_table(kind, fixed, shape, n):
     out = b.download()
     for k in ("pos", "dir", "next_step", "trajectory_length"):
         assert same(out[k], getattr(ref, k)[idx]), k
+
+
+@pytest.mark.parametrize("kind,fixed", [("BP", True), ("BP", False), ("CK", True), ("CK", False)])
+def test_tricubic_quads_with_boundaries_and_observer(kind, fixed):
+    """Four lanes to a particle in a periodic box that shifts source and created positions, a sphere, a length limit
+    and an observer: the same bits and counts as one lane to a particle (33100 copies, the row table)."""
+    rng = np.random.default_rng(23)
+    m = 331
+    sp, L = [20 * KPC] * 3, np.array([120, 140, 100]) * KPC
+    f = capi.Field.grid3f(noise((6, 7, 5)), [0, 0, 0], sp)
+    f.set_interpolation("TRICUBIC")
+    pos, d, E = rng.uniform(0, 1, (m, 3)) * L, O.normalise(rng.normal(size=(m, 3))), 10 ** rng.uniform(0, 2, m) * EEV
+    q = np.where(np.arange(m) % 6 == 1, 0.0, EPLUS)
+    src, made = rng.normal(size=(m, 3)) * KPC, rng.normal(size=(m, 3)) * KPC
+    lo, hi = (15 * KPC, 15 * KPC) if fixed else (KPC, 60 * KPC)
+    res = []
+    for n in (m, 33100):
+        p = capi.Propagator(kind, f, 1e-3, lo, hi, max_length=700 * KPC)
+        p.set_observer([40 * KPC, 130 * KPC, 390 * KPC])
+        p.set_periodic_box([0, 0, 0], L)
+        p.set_spherical_boundary(L / 2, 95 * KPC, 1 * KPC)
+        b, i = capi.Batch(n), np.arange(n) % m
+        b.upload(pos[i], d[i], E[i], q[i], source_pos=src[i], created_pos=made[i])
+        st = p.propagate(b, max_steps=60)
+        res.append((b.download(), b.detections(3), st))
+    (a, da, sa), (c, dc, sc) = res
+    assert not same(a["source_pos"], src) and (a["detection_index"] > 0).any() and (a["active"] == 0).any()
+    for k in a:
+        assert np.array_equal(a[k].view(np.uint8), c[k][:m].view(np.uint8)), k
+        assert np.array_equal(c[k][:m].view(np.uint8), c[k][m:2 * m].view(np.uint8)), k
+    assert np.array_equal(da.view(np.uint64), dc[:, :m].view(np.uint64))
+    assert sc.accepted_steps == 100 * sa.accepted_steps and sc.finished == 100 * sa.finished

@@ -1,6 +1,8 @@
-"""Cell tables beyond the reach of the first-level address translation (3 GB) are gathered by waves together:
-the same bits as the point layout's eight scattered reads, for every step kind, with ragged batches, neutral
-and inactive particles and positions outside a clipped volume."""
+"""Cell tables beyond the reach of the first-level address translation (3 GB): batches of 44 particles to a SIMD and
+more (45056 on 256 compute units) are gathered by waves together, smaller ones read by each lane.  The same bits as
+the point layout's eight scattered reads, for every step kind, with ragged batches, neutral and inactive particles
+and positions outside a clipped volume; the tests with 45055 particles and more take both sides of the line, those
+with up to 1000 the lanes' loads."""
 import numpy as np
 import pytest
 

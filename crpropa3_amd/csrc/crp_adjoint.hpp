@@ -326,8 +326,8 @@ __global__ void __launch_bounds__(256) k_adjoint_backward(AdjArgs A) {
 // every reverse step adds 24 FP64 atomics into the grid gradient.  The blocked backward instead
 //   1. takes the state (x, u) before every kAdjSub-th step of the block (sub-checkpoints, 6 doubles
 //      per kAdjSub steps) and, per particle group, the number of steps whose half-step position falls in
-//      each tile of 2^S cells per axis.  The forward keeps both where all of them fit the buffer budget
-//      (k_adjoint_forward_keep); else a block of segments of every particle is recomputed at once
+//      each tile of 2^S cells per axis.  The forward keeps both where the caller's plan asks for it and all of
+//      them fit the buffer budget (k_adjoint_forward_keep); else a block of segments of every particle is recomputed at once
 //      (segments x n independent lanes);
 //   2. scans the counts into every tile's start and every particle group's place within each tile;
 //   3. runs the reverse steps of the block per particle (one lane per particle, the only sequential

@@ -370,3 +370,45 @@ def test_adjoint_keeps_no_states_on_a_full_card(monkeypatch):
     unused = torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
     assert not adjoint._roomy((3 << 30) + unused, dev)
     assert adjoint._roomy(1 << 28, dev)
+
+
+@pytest.mark.parametrize("before,after", [({}, {}), ({}, dict(CRP_ADJOINT_BLOCK_BYTES="0")),
+                                          ({}, dict(CRP_ADJOINT_BLOCK_BYTES="3e4")),
+                                          (dict(CRP_ADJOINT_TILE_SHIFT="4"), {})])
+def test_adjoint_calls_without_a_plan(before, after, monkeypatch):
+    """crp_adjoint_forward and crp_adjoint_backward with checkpoints of the documented size and a scratch sized at
+    the backward: the environment may change in between, and nothing past the buffers is written."""
+    import ctypes as C
+    from crpropa3_amd import adjoint, capi
+    n, N, nsteps, K = 300, 20, 111, 13
+    s = setup(n=n, N=N, nsteps=nsteps, K=K, seed=61)
+    ref = oracle_grad(s)
+    dev = torch.device("cuda:0")
+    L, p = adjoint._bind(), adjoint._ptr
+    g = torch.tensor(s["grid"], device=dev)
+    x0, u0, kq, wx = (torch.tensor(s[k], device=dev) for k in ("x0", "u0", "kq", "wx"))
+    cfg = adjoint._config(g, [0, 0, 0], [s["sp"]] * 3, 1.0, s["h"], nsteps, K)
+    states = (-(-nsteps // K) * 48 * n + 255) // 256 * 32
+    size, guard = states + 16 * N ** 3, 4096
+    ckpt = torch.full((size + guard,), 7.0, dtype=torch.float64, device=dev)
+    xo, uo, gx0, gu0 = (torch.empty_like(x0) for _ in range(4))
+    for k, v in before.items():
+        monkeypatch.setenv(k, v)
+    capi.check(L.crp_adjoint_forward(C.byref(cfg), n, p(x0), p(u0), p(kq), p(ckpt), p(xo), p(uo), None))
+    for k in before:
+        monkeypatch.delenv(k)
+    for k, v in after.items():
+        monkeypatch.setenv(k, v)
+    sb = C.c_size_t(0)
+    capi.check(L.crp_adjoint_workspace(C.byref(cfg), n, None, C.byref(sb)))
+    scratch = torch.full((-(-sb.value // 8) + guard,), 7.0, dtype=torch.float64, device=dev)
+    gg, gs = torch.zeros(g.numel(), dtype=torch.float64, device=dev), torch.zeros(1, dtype=torch.float64, device=dev)
+    gu = 2 * (uo - torch.tensor(s["target"], device=dev))
+    capi.check(L.crp_adjoint_backward(C.byref(cfg), n, p(kq), p(ckpt), p(wx), p(gu), p(scratch), p(gg), p(gx0), p(gu0),
+                                      p(gs), None))
+    torch.cuda.synchronize()
+    assert (ckpt[size:] == 7.0).all() and (scratch[-guard:] == 7.0).all()
+    assert np.allclose(gg.cpu().numpy().reshape(ref[3].shape), ref[3], rtol=0, atol=1e-6 * np.abs(ref[3]).max())
+    for a, b in ((gx0, ref[4]), (gu0, ref[5])):
+        assert np.allclose(a.cpu().numpy(), b, rtol=1e-7, atol=1e-8 * np.abs(b).max())
+    assert gs.item() == pytest.approx(ref[6], rel=1e-8)
